@@ -652,11 +652,22 @@ __global__ __launch_bounds__(64) void decode_splitk(DecodeKArgs ka, int n_items,
     }
 }
 
-// One workgroup per (query head, sequence); lanes stride over head_dim.
-template <typename T>
-__global__ __launch_bounds__(64) void decode_combine(DecodeArgs a) {
+// Merges the partials of one (query head, sequence) per workgroup of 1..8 waves. Latency-bound:
+// the partials of a head are few KiB, so what counts is how many loads are in flight and how
+// many dependent round trips follow each other. LPR lanes hold one partial row (four dims each),
+// so a wave takes 64 / LPR partials at once and four of those per round; every lane merges its
+// own partials online (local running max), so O, m and l all arrive in one round trip, and the
+// lanes' and waves' results are merged at the end, in a fixed order.
+// 256 partials a head (B1 Hq16 Hkv4 D64 over 8192 f32 rows): one wave that walked them in turn
+// took 30.0 us of that decode's 40.2.
+template <typename T, int LPR>
+__global__ __launch_bounds__(512) void decode_combine(DecodeArgs a) {
     constexpr int EB = DecodeIO<T>::kBytes;
-    const int hq = blockIdx.x, s = blockIdx.y, lane = threadIdx.x;
+    constexpr int SPW = 64 / LPR, UN = 4;
+    __shared__ __attribute__((aligned(16))) float o_lds[8][LPR * 4];
+    __shared__ float ml_lds[8][2];
+    const int hq = blockIdx.x, s = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int waves = blockDim.x >> 6;
     const int hl = hq % a.group;
     const int u = (hq / a.group) * a.chunks + hl / 16;
     const int units = a.kv_heads * a.chunks;
@@ -664,59 +675,102 @@ __global__ __launch_bounds__(64) void decode_combine(DecodeArgs a) {
     const int ns = p1 - p0;
     if (ns <= 0) return;  // one segment: finalised by the split kernel
     const float c2 = a.scale * kLog2e;
-    const float* ml0 = a.part_ml + ((int64_t)p0 * 16 + hl % 16) * 2;
-    const int64_t step_ml = 16 * 2;
-    // split statistics: split j in lane j % 64 (one pass for up to 64 splits)
-    float M = -INFINITY;
-    for (int j = lane; j < ns; j += 64) M = fmaxf(M, ml0[j * step_ml]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, shfl_xor(M, o));
-    float L = 0.0f;
-    for (int j = lane; j < ns; j += 64) L += ml0[j * step_ml + 1] * fast_exp2((ml0[j * step_ml] - M) * c2);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) L += shfl_xor(L, o);
-    const float inv = 1.0f / L;
-    const int d = 2 * lane;
-    const float* po = a.part_o + ((int64_t)p0 * 16 + hl % 16) * a.head_dim + d;
+    const int d = 4 * (lane % LPR);
+    const bool dok = d < a.head_dim;
+    const float2* ml0 = (const float2*)a.part_ml + (int64_t)p0 * 16 + hl % 16;
+    const float* po = a.part_o + ((int64_t)p0 * 16 + hl % 16) * a.head_dim + (dok ? d : 0);
     const int64_t step_o = (int64_t)16 * a.head_dim;
-    float acc0 = 0.0f, acc1 = 0.0f;
-    for (int jb = 0; jb < ns; jb += 64) {
-        // weight of split jb + lane, broadcast by shuffle; O loads unrolled for memory parallelism
-        const int jl = jb + lane;
-        const float wl = jl < ns ? fast_exp2((ml0[jl * step_ml] - M) * c2) : 0.0f;
-        const int cnt = min(64, ns - jb);
-        int j = 0;
-        for (; j + 4 <= cnt; j += 4) {
-            float2 v[4];
+    float M = -INFINITY, L = 0.0f;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const int stride = waves * SPW;
+    for (int j = wave * SPW + lane / LPR; j < ns; j += UN * stride) {
+        float2 ml[UN];
+        f32x4_t v[UN];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                v[u] = d < a.head_dim ? *(const float2*)(po + (jb + j + u) * step_o)
-                                      : make_float2(0.f, 0.f);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float wgt = __shfl(wl, j + u, 64);
-                acc0 = fmaf(v[u].x, wgt, acc0);
-                acc1 = fmaf(v[u].y, wgt, acc1);
-            }
+        for (int i = 0; i < UN; ++i) {  // past the end: the first partial again, not counted
+            const int64_t at = j + i * stride < ns ? j + i * stride : j;
+            ml[i] = ml0[at * 16];
+            v[i] = *(const f32x4_t*)(po + at * step_o);
         }
-        for (; j < cnt; ++j) {
-            const float wgt = __shfl(wl, j, 64);
-            if (d < a.head_dim) {
-                const float2 v = *(const float2*)(po + (jb + j) * step_o);
-                acc0 = fmaf(v.x, wgt, acc0);
-                acc1 = fmaf(v.y, wgt, acc1);
+        float mx = M;
+#pragma unroll
+        for (int i = 0; i < UN; ++i) mx = fmaxf(mx, ml[i].x);
+        const float keep = fast_exp2((M - mx) * c2);  // M = -inf -> 0
+        L *= keep;
+        acc *= keep;
+        M = mx;
+#pragma unroll
+        for (int i = 0; i < UN; ++i) {
+            if (i == 0 || j + i * stride < ns) {
+                const float w = fast_exp2((ml[i].x - M) * c2);
+                L = fmaf(ml[i].y, w, L);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = fmaf(v[i][e], w, acc[e]);
             }
         }
     }
-    if (d < a.head_dim) {
+    // lanes of the other partials (they hold no partial: M = -inf, weight 0)
+#pragma unroll
+    for (int o = LPR; o < 64; o <<= 1) {
+        const float Mo = shfl_xor(M, o), Lo = shfl_xor(L, o);
+        const float mx = fmaxf(M, Mo);
+        const float w0 = M == -INFINITY ? 0.0f : fast_exp2((M - mx) * c2);
+        const float w1 = Mo == -INFINITY ? 0.0f : fast_exp2((Mo - mx) * c2);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = acc[e] * w0 + shfl_xor(acc[e], o) * w1;
+        L = L * w0 + Lo * w1;
+        M = mx;
+    }
+    if (waves > 1) {
+        if (lane < LPR) *(f32x4_t*)(o_lds[wave] + d) = acc;
+        if (lane == 0) {
+            ml_lds[wave][0] = M;
+            ml_lds[wave][1] = L;
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        float mx = M;
+        for (int w = 1; w < waves; ++w) mx = fmaxf(mx, ml_lds[w][0]);
+        float w0 = M == -INFINITY ? 0.0f : fast_exp2((M - mx) * c2);
+        acc *= w0;
+        L *= w0;
+        for (int w = 1; w < waves; ++w) {
+            const float Mw = ml_lds[w][0];
+            w0 = Mw == -INFINITY ? 0.0f : fast_exp2((Mw - mx) * c2);
+            const f32x4_t v = *(const f32x4_t*)(o_lds[w] + d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = fmaf(v[e], w0, acc[e]);
+            L = fmaf(ml_lds[w][1], w0, L);
+        }
+        M = mx;
+    }
+    const float inv = 1.0f / L;
+    if (lane < LPR && dok) {
         uint8_t* dst = (uint8_t*)a.o + (((int64_t)s * a.q_heads + hq) * a.head_dim + d) * EB;
         if constexpr (std::is_same<T, float>::value) {
-            *(float2*)dst = make_float2(acc0 * inv, acc1 * inv);
+            *(f32x4_t*)dst = acc * inv;
         } else {
-            *(uint32_t*)dst = Half<T>::pack(acc0 * inv, acc1 * inv);
+            *(u32x2_t*)dst = u32x2_t{Half<T>::pack(acc[0] * inv, acc[1] * inv),
+                                     Half<T>::pack(acc[2] * inv, acc[3] * inv)};
         }
     }
     if (lane == 0) a.lse[(int64_t)s * a.q_heads + hq] = M * a.scale + logf(L);
+}
+
+// Waves per combine workgroup: enough that the unit with the most partials takes one round of
+// four partials per lane group, at most 8 (two rounds for 256 partials at D 64).
+template <typename T>
+static void launch_combine(const DecodeArgs& a, hipStream_t s) {
+    const int lpr = a.head_dim <= 32 ? 8 : a.head_dim <= 64 ? 16 : 32;
+    const int per_wave = 4 * (64 / lpr);
+    int waves = 1;
+    while (waves < 8 && waves * per_wave < a.max_parts) waves *= 2;
+    const dim3 g((unsigned)a.q_heads, (unsigned)a.n_seqs), b(64 * waves);
+    switch (lpr) {
+        case 8: decode_combine<T, 8><<<g, b, 0, s>>>(a); break;
+        case 16: decode_combine<T, 16><<<g, b, 0, s>>>(a); break;
+        default: decode_combine<T, 32><<<g, b, 0, s>>>(a); break;
+    }
 }
 
 template <typename K>
@@ -848,11 +902,10 @@ void launch_decode(Dtype dt, const DecodeArgs& a, hipStream_t s, unsigned grid[3
     unsigned gx = 0;
     split_kernel(dt, ka, s, &gx, mfma, false);
     if (between) between(user);
-    const dim3 cg((unsigned)a.q_heads, (unsigned)a.n_seqs);
     switch (dt) {
-        case Dtype::BF16: decode_combine<bf16_t><<<cg, 64, 0, s>>>(a); break;
-        case Dtype::F16: decode_combine<f16_t><<<cg, 64, 0, s>>>(a); break;
-        default: decode_combine<float><<<cg, 64, 0, s>>>(a); break;
+        case Dtype::BF16: launch_combine<bf16_t>(a, s); break;
+        case Dtype::F16: launch_combine<f16_t>(a, s); break;
+        default: launch_combine<float>(a, s); break;
     }
     grid[0] = gx;
     grid[1] = 1;

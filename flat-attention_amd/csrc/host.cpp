@@ -1924,6 +1924,7 @@ struct fa_decode_plan {
     uint64_t split_tokens = 0;  // longest segment of the current work list
     uint64_t n_work = 0;        // segments
     uint64_t n_waves = 0, n_slots = 0, units = 0;
+    uint64_t max_parts = 0;  // most partial slots of any (sequence, unit)
     int grouped = 0;  // > 0: head-grouped workgroups of this many waves (one per unit)
     uint64_t max_pos = 0;
     // device
@@ -2079,6 +2080,9 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
         }
     }
     p->n_work = segs.size();
+    p->max_parts = 0;
+    for (size_t i = 0; i + 1 < unit_part.size(); ++i)
+        p->max_parts = std::max<uint64_t>(p->max_parts, (uint64_t)(unit_part[i + 1] - unit_part[i]));
     p->n_waves = n_waves;
     p->units = units;
     p->split_tokens = longest;
@@ -2342,6 +2346,7 @@ int enqueue_decode(fa_ctx* ctx, const fa_decode_plan* p, const float2* table, co
     a.page_size = (int)p->page_size;
     a.bt_stride = (int)p->max_pages;
     a.scale = p->scale;
+    a.max_parts = (int)p->max_parts;
     a.grouped = p->grouped;
     unsigned grid[3], block;
     int dispatches = 0;

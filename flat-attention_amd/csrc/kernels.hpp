@@ -96,6 +96,7 @@ struct DecodeArgs {
     const float2* rope_table;
     int n_seqs, n_waves, q_heads, kv_heads, group, head_dim, chunks;
     int page_size, bt_stride;
+    int max_parts;  // most partial slots of any (sequence, unit)
     float scale;
     // > 0: head-grouped MFMA split kernel, workgroups of `grouped` waves (one per unit) sharing
     // one segment list; seg[1] is then the partial-slot stride between units.

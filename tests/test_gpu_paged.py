@@ -172,6 +172,25 @@ def test_split_count_invariance(hip):
             assert_close(f"LSE split {split}", l, ref[1], 1e-4, 1e-5)
 
 
+@pytest.mark.parametrize("D,dtype", [(32, fa.DTYPE_F32), (64, fa.DTYPE_BF16), (80, fa.DTYPE_F32),
+                                     (128, fa.DTYPE_F32), (128, fa.DTYPE_F16)])
+@pytest.mark.parametrize("most", [2, 8, 9, 33, 130])
+def test_combine_merges_any_number_of_partials(hip, D, dtype, most):
+    """decode_combine: 2 .. `most` 16-key partials a unit (one lane group's round, several waves,
+    several rounds, a last round that is only partly filled) beside a unit without partials."""
+    rnd = {fa.DTYPE_F32: lambda x: x, fa.DTYPE_BF16: bf16_round, fa.DTYPE_F16: f16_round}[dtype]
+    atol, rtol = (F32_ATOL, F32_RTOL) if dtype == fa.DTYPE_F32 else (H16_ATOL, 0.0)
+    ps, hq, hkv = 16, 6, 2
+    ctx_lens = [16 * most - 3, 16, 16 * (most // 2) + 1]
+    bt, kp, vp, total = _make_pool(np.random.default_rng(most), ctx_lens, ps, hkv, D, rnd)
+    q = rnd(normal(len(ctx_lens) * hq * D, most))
+    o, l, plan = _decode(hip, bt, ctx_lens, kp, vp, total, ps, hq, hkv, D, q, dtype, split=16)
+    assert plan.info()["work_items"] == hkv * sum((c + 15) // 16 for c in ctx_lens)
+    eo, el = oracle.paged_decode(q, kp, vp, total, ps, bt, ctx_lens, hq, hkv, D, True, 1e4)
+    assert_close("O", o, eo, atol, rtol)
+    assert_close("LSE", l, el, atol, rtol)
+
+
 def test_cfg4_full_size_bf16_decode(hip):
     """64 sequences, ctx ~ U[512, 8192], page 16, Hq32 Hkv8 D128, bf16 KV,
     randomly permuted physical pages. Full oracle comparison."""
