@@ -904,16 +904,29 @@ struct PrefillChoice {
                           // from the pre-pass (prerot), Q split in the kernel
 };
 
+int prefill_a64_mode(const fa_ctx* ctx) {
+    return ctx->prefill_kernel_policy == 0  ? fa::kA64Never
+           : ctx->prefill_kernel_policy > 0 ? fa::kA64Always
+                                            : fa::kA64Auto;
+}
+
 PrefillChoice choose_prefill(const fa_ctx* ctx, const PrefillJob& j) {
     PrefillChoice c;
     if (j.rope) {
         c.prerot = j.a.rope_k && !j.paged && want_prerotate(ctx, (uint64_t)j.a.head_dim);
+        // Few keys of narrow rows in the key-group kernel: rotating them in every workgroup costs
+        // less than the pre-pass's launch (D 64, Hq8 Hkv2: 10.1 against 11.2 us at 512 keys, level
+        // at 1024; D 128: 14.1 against 12.9 at 256).
+        if (c.prerot && ctx->prerotate_policy < 0 && ctx->prefill_precision == 0 &&
+            j.a.head_dim <= 64 && j.a.kv_len <= 512 &&
+            fa::prefill_key_groups(j.dt, false, j.a) == 4)
+            c.prerot = false;
         if (ctx->prefill_precision == 1 && j.a.rope_k && !j.paged && j.dtype != FA_DTYPE_F32) {
             // the assembly kernel where it takes the launch (the arguments it would receive:
             // K rotated by the pre-pass, the residual beside it), else the HIP split kernel
             fa::PrefillArgs t = j.a;
             t.rope_k = 0;
-            t.a64 = ctx->prefill_kernel_policy != 0;
+            t.a64 = prefill_a64_mode(ctx);
             t.rope_rows = (int)j.max_pos;
             t.rope_table = (const float2*)(uintptr_t)16;
             t.k_lo = (const void*)(uintptr_t)16;
@@ -989,7 +1002,7 @@ int resolve_prefill(fa_ctx* ctx, PrefillJob& j, bool own, PrefillRun* r) {
         if (c.split_qk) r->j.a.split_qk = 1;
         r->j.a.rope_rows = (int)j.max_pos;
     }
-    r->j.a.a64 = ctx->prefill_kernel_policy != 0;
+    r->j.a.a64 = prefill_a64_mode(ctx);
     r->prerot = prerot;
     if (prerot) {
         const uint64_t wsb = r->prec64 ? 2 * j.kv_bytes : j.kv_bytes;
@@ -1016,7 +1029,7 @@ void describe_prefill(const fa_ctx* ctx, const PrefillJob& j, const fa::PrefillA
     if (j.rope && a.rope_k && !prerot && !j.paged && a.head_dim % 8 != 0)
         fb = "K pre-rotation pass needs head_dim % 8 == 0; K rotated on load";
     const char* dt = j.dtype == FA_DTYPE_BF16 ? "bf16" : j.dtype == FA_DTYPE_F16 ? "f16" : "f32";
-    const bool a64 = fa::prefill_a64_eligible(j.dt, j.paged, a);
+    const bool a64 = fa::prefill_uses_a64(j.dt, j.paged, a);
     const char* base =
         j.dtype == FA_DTYPE_F32 ? "prefill_mfma_f32" : (a64 ? "prefill_a64" : "prefill_mfma16");
     char name[64];
@@ -1063,7 +1076,7 @@ int enqueue_prefill(fa_ctx* ctx, const PrefillRun& r) {
     const int kid = prefill_kernel_id(j.dtype, r.prerot || (j.paged && j.rope));
     // the assembly and the f32 kernel (one dispatch each) record their span's events as part of
     // their dispatch
-    const bool own = (j.dtype == FA_DTYPE_F32 || fa::prefill_a64_eligible(j.dt, j.paged, a)) &&
+    const bool own = (j.dtype == FA_DTYPE_F32 || fa::prefill_uses_a64(j.dt, j.paged, a)) &&
                      dispatch_events(ctx, &a.ev_start, &a.ev_stop);
     if (!own) begin_span(ctx);
     fa::launch_prefill(j.dt, j.paged, a, ctx->stream, grid, &block);
@@ -1214,7 +1227,7 @@ int fa_forward_gqa_rope_telemetry(fa_ctx* ctx, const fa_grouped_shape* sh, const
     if (c.prerot) a.rope_k = 0;
     if (c.split_qk) a.split_qk = 1;
     if (c.prec64) a.k_lo = (const void*)(uintptr_t)16;  // stands for the residual the call writes
-    a.a64 = ctx->prefill_kernel_policy != 0;
+    a.a64 = prefill_a64_mode(ctx);
     a.rope_rows = (int)j.max_pos;
     if (j.rope) a.rope_table = (const float2*)(uintptr_t)16;  // stands for the table the call builds
     describe_prefill(ctx, j, a, c.prerot, 1u + c.prerot, allocs, bytes, out);

@@ -10,6 +10,11 @@ namespace fa {
 
 enum class Dtype : int { F32 = 0, F16 = 1, BF16 = 2 };
 
+enum : int { kA64Never = 0, kA64Auto = 1, kA64Always = 2 };
+
+// Compute units of the current device.
+int device_cus();
+
 // Prefill / rectangular attention over contiguous or paged K/V.
 // Query row (b, h, t) lives at q + b*q_sb + h*q_sh + t*q_ss (head_dim contiguous); the same
 // scheme addresses O with o_* strides and LSE with lse_sb/lse_sh (t contiguous).
@@ -44,8 +49,9 @@ struct PrefillArgs {
     // 16-bit contiguous K rotated on load only: carry the rotated Q and K as 16-bit high part +
     // 16-bit residual and take three MFMAs per score block (f32-level scores).
     int split_qk;
-    // Allow the assembly main loop (fa_prefill_a64_bf16) where it applies (prefill_a64_eligible).
-    int a64;
+    // The assembly main loop (fa_prefill_a64_bf16) where it applies (prefill_a64_eligible): never,
+    // where it is the faster one, or always.
+    int a64;  // kA64Never, kA64Auto, kA64Always
     // Rows of rope_table (positions it covers); bounds the assembly kernel's table reads.
     int rope_rows;
     // Precise scores in the assembly kernel (contiguous K/V, K rotated by the pre-pass): the
@@ -69,6 +75,11 @@ void launch_prefill_a64(Dtype dt, const PrefillArgs& a, bool paged, hipStream_t 
 // Workgroups of its persistent grid: min(query blocks, CUs of the current device).
 unsigned prefill_a64_workgroups(const PrefillArgs& a);
 
+// Key groups of the 16-bit launch of `a`: 2 or 4 where the row blocks alone would leave most of
+// the chip idle (prefill_mfma16's KW), 0 otherwise.
+int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a);
+// Whether launch_prefill runs the assembly kernel on `a`.
+bool prefill_uses_a64(Dtype dt, bool paged, const PrefillArgs& a);
 void launch_prefill(Dtype dt, bool paged, const PrefillArgs& a, hipStream_t s,
                     unsigned grid[3], unsigned* block);
 // The grid, workgroup size and query rows per workgroup launch_prefill uses for `a` (host only).

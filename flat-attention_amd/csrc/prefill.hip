@@ -8,7 +8,8 @@
 // Workgroup = 8 waves = 256 query rows in two groups of four on a ping-pong schedule (one
 // group's MFMAs against the other group's softmax) for contiguous K/V and for paged K/V with a
 // page size that is a multiple of 16; 4 waves = 128 rows otherwise (other page sizes, K rotated
-// in the kernel). Rows of one (batch, kv-head) are flattened as row = t * group +
+// in the kernel); launches of few blocks split the eight waves over key groups instead (KW below:
+// 128 or 64 rows). Rows of one (batch, kv-head) are flattened as row = t * group +
 // head_in_group, so one workgroup holds every query head of a GQA group for consecutive
 // positions: each K/V tile staged in LDS feeds all of them.
 // Per 64-key tile and wave (32 rows):
@@ -20,6 +21,7 @@
 // K rows are fed to the MFMA in a permuted order (bits 2 and 3 of the row swapped) so that the
 // eight scores a lane holds per 16-key step are contiguous keys, which is the order the P^T
 // operand of the second MFMA needs.
+#include <algorithm>
 #include <type_traits>
 
 #include <hip/hip_ext.h>
@@ -43,9 +45,26 @@ struct FastDiv {
     }
 };
 
+// The divisors of the block map are known on the host: an integer division by a kernel argument
+// is some thirty instructions, and a lone wave issues one in about six cycles.
 struct PrefillKArgs {
     PrefillArgs a;
-    FastDiv ps;
+    FastDiv ps, grp;   // page size, query heads per kv head
+    FastDiv nqb;       // query blocks of a (batch, kv head) unit
+    FastDiv per_xcd;   // blocks of an XCD's chunk
+    FastDiv units;     // units in it (d = 0: not a whole number)
+    FastDiv inner;     // units per step of the outer unit index (kv heads, or batch: var_meta)
+    void set_grid(unsigned nb, unsigned rows) {
+        const uint32_t n = (uint32_t)(((int64_t)a.q_len * a.group + rows - 1) / rows);
+        nqb = FastDiv(n);
+        grp = FastDiv((uint32_t)a.group);
+        inner = FastDiv((uint32_t)(a.var_meta ? a.batch : a.kv_heads));
+        units.d = 0;
+        if (nb % 8 == 0 && nb / 8 % n == 0) {
+            per_xcd = FastDiv(nb / 8);
+            units = FastDiv(nb / 8 / n);
+        }
+    }
 };
 
 template <bool PAGED>
@@ -62,36 +81,63 @@ __device__ __forceinline__ int64_t kv_row_offset(const PrefillKArgs& ka, int b, 
 }
 
 
-// Padded query row `row` (t = row / group) of a variable-length batch: O = 0 in every dim,
-// LSE = -inf. Lane group g writes the dims of 4-element groups of its parity, as the epilogue.
+// Padded query rows [from, to) (row = t * group + head) of a variable-length batch: O = 0 in every
+// dim, LSE = -inf. The whole workgroup writes them, consecutive threads consecutive 16-byte (f32:
+// 4-byte) pieces of a row; a lane per row with 2-byte stores took longer than the rows that had
+// work (one query beside 700 padded ones).
 template <typename E>
-__device__ __forceinline__ void write_padded_row(const PrefillArgs& a, int b, int kvh, int row,
-                                                 int g, int D) {
-    const int t = row / a.group, hq = kvh * a.group + row % a.group;
-    E* orow = (E*)a.o + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)t * a.o_ss;
-    for (int d0 = 4 * g; d0 < D; d0 += 8)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (d0 + j < D) orow[d0 + j] = E(0);
-    if (g == 0) a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = -INFINITY;
+__device__ __forceinline__ void write_padded_rows(const PrefillKArgs& ka, int b, int kvh, int from,
+                                                  int to, int D) {
+    const PrefillArgs& a = ka.a;
+    constexpr int W = sizeof(E) == 2 ? 8 : 1;  // (16-bit storage: head_dim % 8 == 0)
+    const int per = D / W;
+    for (int i = threadIdx.x; i < (to - from) * per; i += blockDim.x) {
+        const int r = from + i / per, d = i % per * W;
+        const int t = (int)ka.grp.div((uint32_t)r), hq = kvh * a.group + r - t * a.group;
+        E* o = (E*)a.o + (int64_t)b * a.o_sb + (int64_t)hq * a.o_sh + (int64_t)t * a.o_ss + d;
+        if constexpr (W == 8) *(u32x4_t*)o = u32x4_t{0u, 0u, 0u, 0u};
+        else *o = E(0);
+    }
+    for (int r = from + threadIdx.x; r < to; r += blockDim.x) {
+        const int t = (int)ka.grp.div((uint32_t)r), hq = kvh * a.group + r - t * a.group;
+        a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = -INFINITY;
+    }
 }
 
-// Query block of this workgroup: (batch * kv_heads + kv head, query block index). The blocks
-// an XCD runs form a contiguous chunk of xcd_remap's order; when that chunk is a whole number of
-// (batch, kv head) units it is dispatched heaviest first across its units (query blocks in
-// decreasing causal length, units interleaved), otherwise unit by unit, heaviest first.
-__device__ __forceinline__ void block_coords(int bid, int nb, int nqb, int& bh, int& qb) {
-    const int logical = xcd_remap(bid, nb);
-    const int per_xcd = nb / 8;
-    if (nb % 8 == 0 && per_xcd % nqb == 0) {
-        const int units = per_xcd / nqb;
-        const int x = logical / per_xcd, l = logical % per_xcd;
-        bh = x * units + l % units;
-        qb = nqb - 1 - l / units;
+// Query block of this workgroup: batch element, kv head and query block index. The blocks an XCD
+// runs form a contiguous chunk of xcd_remap's order; when that chunk is a whole number of (batch,
+// kv head) units it is dispatched heaviest first across its units (query blocks in decreasing
+// causal length, units interleaved), otherwise unit by unit, heaviest first.
+// Units are numbered batch element first, except in a variable-length batch, whose sequences
+// differ in work: there kv head first, so that every XCD gets its share of each sequence, and the
+// units of a round are rotated from round to round. A chunk's workgroups go to the XCD's four
+// shader engines in turn and each waits for a place on its own: with four sequences in a fixed
+// order one engine held every block of the longest, and the blocks behind its ninth waited 32 us
+// for it while the others had finished (Hq32 Hkv8 D128, 700 queries over 1500 keys and three
+// shorter sequences).
+__device__ __forceinline__ void block_coords(const PrefillKArgs& ka, int bid, int& b, int& kvh,
+                                             int& qb) {
+    const int nqb = (int)ka.nqb.d;
+    const int logical = xcd_remap(bid, (int)gridDim.x);
+    int bh;
+    if (ka.units.d > 0) {
+        const int x = (int)ka.per_xcd.div((uint32_t)logical);
+        const int l = logical - x * (int)ka.per_xcd.d;
+        const int lu = (int)ka.units.div((uint32_t)l);
+        int u = l - lu * (int)ka.units.d;
+        if (ka.a.var_meta) {  // the sequence of a place in the round differs from round to round
+            const int v = u + lu;
+            u = v - (int)ka.units.div((uint32_t)v) * (int)ka.units.d;
+        }
+        bh = x * (int)ka.units.d + u;
+        qb = nqb - 1 - lu;
     } else {
-        bh = logical / nqb;
-        qb = nqb - 1 - logical % nqb;
+        bh = (int)ka.nqb.div((uint32_t)logical);
+        qb = nqb - 1 - (logical - bh * nqb);
     }
+    const int hi = (int)ka.inner.div((uint32_t)bh), lo = bh - hi * (int)ka.inner.d;
+    b = ka.a.var_meta ? lo : hi;
+    kvh = ka.a.var_meta ? hi : lo;
 }
 
 // Running-max slack (log2 units) tolerated before O is rescaled: probabilities stay <= 2^8.
@@ -150,17 +196,25 @@ __host__ __device__ constexpr bool prefill_pingpong(int pmode, bool ropek) {
 // plus the 16-bit rounding of their residual, and S = Khi.Qhi + Khi.Qlo + Klo.Qhi (the lo.lo
 // term is below f32 rounding of the sum), so scores keep f32-level accuracy where a once-rounded
 // rotation would move a score of magnitude s by up to s * 2^-8.
-template <typename T, int DPAD, int PMODE, bool ROPEK, bool FULLD, int NW, bool SPLIT = false>
+// KW > 1 (key groups, for launches whose row blocks alone would leave most of the chip idle):
+// the workgroup's waves form KW groups of RW = NW / KW waves on the same 32 RW rows; group k runs
+// the tiles k, k + KW, ... with an LDS region and a running (m, l, O) of its own, and the groups'
+// results are merged in LDS at the end.
+template <typename T, int DPAD, int PMODE, bool ROPEK, bool FULLD, int NW, bool SPLIT = false,
+          int KW = 1>
 __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(PrefillKArgs ka) {
     static_assert(!SPLIT || (ROPEK && NW == 4), "split scores need the in-kernel K rotation");
     using H = Half<T>;
     const PrefillArgs& a = ka.a;
-    constexpr int BM = 32 * NW, BN = 64;
-    constexpr bool PP = NW == 8;
+    constexpr int RW = NW / KW;             // waves (of 32 rows) side by side
+    constexpr int BM = 32 * RW, BN = 64;
+    constexpr bool PP = NW == 8 && KW == 1;
+    constexpr int NST = KW > 2 ? 1 : 2;     // K/V stages (of each group)
     constexpr int KS = DPAD / 16;           // QK^T k-steps (16 dims each)
     constexpr int MB = DPAD / 32;           // 32-dim blocks of O^T
     constexpr int CPR = DPAD / 8;           // 16-byte chunks per row
-    constexpr int KRPP = 256 / CPR;         // rows staged per pass
+    constexpr int GT = PP ? 256 : 64 * RW;  // threads that stage one tile
+    constexpr int KRPP = GT / CPR;          // rows staged per pass
     constexpr int KPASS = BN / KRPP;
     constexpr int KROWB = DPAD * 2 + 16;    // padded K row (bytes)
     constexpr int VROWB = DPAD * 2 + 64;    // padded V row (bytes)
@@ -174,31 +228,36 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
     // registers and no LDS store instructions. One instruction fills 64 consecutive 16-byte
     // slots; padded rows are kept by giving pad slots an out-of-range (zero-filling, no
     // memory traffic) offset. Instructions beyond a tile's slot count target a dummy KiB.
-    constexpr bool DMA = CONTIG && !ROPEK;
+    constexpr bool DMA = CONTIG && !ROPEK && KW <= 2;
     // 16-byte slots per padded row: K, V, V^T (64 keys of one dim)
     constexpr int KSL = KROWB / 16, VSL = VROWB / 16;
     // transfer instructions per tile (64 slots each)
     constexpr int KINS = KSL, VINS = VSL;
     // Waves sharing the transfers: all of them, or group 1 alone under the ping-pong schedule.
-    constexpr int NWD = PP ? 4 : NW;
+    constexpr int NWD = PP ? 4 : RW;
     constexpr int KI = (KINS + NWD - 1) / NWD, VI = (VINS + NWD - 1) / NWD;  // per wave
-    constexpr int DUMMY = 2 * STAGE;
+    constexpr int DUMMY = KW * NST * STAGE;
     // LDS: the K/V stages (+ the dummy KiB of the transfers), reused at the end to stage the
     // output rows (NW waves x 32 rows of DPAD * 2 + 16 bytes)
-    constexpr int SMEM_KV = 2 * STAGE + (DMA ? 1024 : 0);
-    constexpr int SMEM_O = NW * 32 * (DPAD * 2 + 16);
-    __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM_KV > SMEM_O ? SMEM_KV : SMEM_O];
+    // (KW > 1: the f32 O of every group, rows of MROW bytes)
+    constexpr int SMEM_KV = KW * NST * STAGE + (DMA ? 1024 : 0);
+    constexpr int SMEM_O = RW * 32 * (DPAD * 2 + 16);
+    constexpr int MROW = DPAD * 4 + 16;
+    constexpr int SMEM_M = KW > 1 ? KW * BM * MROW : 0;
+    constexpr int SMEM_E = SMEM_M > SMEM_O ? SMEM_M : SMEM_O;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM_KV > SMEM_E ? SMEM_KV : SMEM_E];
     int st_r = 0, st_w = 0;  // byte offsets of the stage being read / written
     int st_k = 0, st_v = 0;  // stage offsets the K (S^T) and V (P.V) operand reads use
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar registers
+    // uniform: scalar registers
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KW > 1 ? wave_id % RW : wave_id;  // this wave's 32 rows of the block
+    const int kg = KW > 1 ? wave_id / RW : 0;          // its key group
     const int D = a.head_dim, half = D >> 1;
     const int rows_pad = a.q_len * a.group;  // padded extent of the grid
-    const int nqb = (rows_pad + BM - 1) / BM;
-    int bh, qb;  // heavy (late, causal) blocks dispatch first
-    block_coords(blockIdx.x, gridDim.x, nqb, bh, qb);
-    const int b = bh / a.kv_heads, kvh = bh % a.kv_heads;
+    int b, kvh, qb;  // heavy (late, causal) blocks dispatch first
+    block_coords(ka, blockIdx.x, b, kvh, qb);
     const int r0 = qb * BM;
     // Per-sequence extents of a variable-length batch (PrefillArgs::var_meta); the grid covers
     // the padded extents. A block of padded query rows only writes O = 0, LSE = -inf.
@@ -212,31 +271,31 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         q_rope_off_ = m[3];
     }
     const int rows_total = q_len_ * a.group;
-    if (a.var_meta && r0 >= rows_total) {
-        const int prow = r0 + wave * 32 + (lane & 31);
-        if (prow < rows_pad) write_padded_row<uint16_t>(a, b, kvh, prow, g, D);
-        return;
+    if (a.var_meta && r0 + BM > rows_total) {
+        write_padded_rows<uint16_t>(ka, b, kvh, max(r0, rows_total), min(r0 + BM, rows_pad), D);
+        if (r0 >= rows_total) return;
     }
 
     // This lane's query row.
     const int row = r0 + wave * 32 + (lane & 31);
     const bool row_ok = row < rows_total;
-    const int t = row_ok ? row / a.group : q_len_ - 1;
-    const int hq = kvh * a.group + (row_ok ? row % a.group : 0);
+    const int row_t = (int)ka.grp.div((uint32_t)row);
+    const int t = row_ok ? row_t : q_len_ - 1;
+    const int hq = kvh * a.group + (row_ok ? row - row_t * a.group : 0);
     const int cpos = causal_off_ + t;
 
     // Key tiles this wave's rows need (its group's 128 rows under the ping-pong schedule) and,
     // for the ping-pong barrier count, the whole block's.
     const int r0w = PP ? r0 + 128 * (wave >> 2) : r0;
-    const int t_max = min(q_len_ - 1, (r0w + 127) / a.group);
-    const int t_min = r0w / a.group;
+    const int t_max = min(q_len_ - 1, (int)ka.grp.div((uint32_t)(r0w + (PP ? 127 : BM - 1))));
+    const int t_min = (int)ka.grp.div((uint32_t)r0w);
     int n_keys = kv_len_;
     if (a.causal) n_keys = min(n_keys, causal_off_ + t_max + 1);
     const int n_tiles = __builtin_amdgcn_readfirstlane((n_keys + BN - 1) / BN);
     const int cpos_min = causal_off_ + t_min;
     int n_keys_blk = kv_len_;
     if (a.causal)
-        n_keys_blk = min(n_keys_blk, causal_off_ + min(q_len_ - 1, (r0 + BM - 1) / a.group) + 1);
+        n_keys_blk = min(n_keys_blk, causal_off_ + min(q_len_ - 1, (int)ka.grp.div((uint32_t)(r0 + BM - 1))) + 1);
     const int n_blk = __builtin_amdgcn_readfirstlane((n_keys_blk + BN - 1) / BN);
     (void)n_blk;
 
@@ -301,8 +360,9 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         (int64_t)kvh * a.k_sh * 2 + (CONTIG ? (int64_t)b * a.k_sb * 2 : 0);
     const uint8_t* const kb8 = (const uint8_t*)a.k + head_off;
     const uint8_t* const vb8 = (const uint8_t*)a.v + head_off;
-    // (ping-pong: the 256 threads of the transferring group 1 stage the tiles)
-    const int tst = PP ? (tid & 255) : tid;
+    // (ping-pong: the 256 threads of the transferring group 1 stage the tiles; key groups: each
+    // its own)
+    const int tst = PP ? (tid & 255) : KW > 1 ? tid % GT : tid;
     const int k_dc = tst % CPR, k_r = tst / CPR;
     const uint32_t kd2 = (uint32_t)(FULLD ? k_dc * 8 : min(k_dc * 8, D - 8)) * 2u;
     const uint32_t lane_off = (uint32_t)k_r * row_bytes + kd2;  // this thread's row/chunk
@@ -509,7 +569,8 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
 
     // ---- probabilities, row sum and the P^T operands (16 keys each)
     auto softmax_exp = [&](f32x16_t (&sacc)[2], u32x4_t (&pop)[4]) {
-        const float neg = -m_run * c2;
+        // (a later key group's first tiles may hold no key that this row sees: m_run = -inf)
+        const float neg = KW > 1 && m_run == -INFINITY ? 0.0f : -m_run * c2;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -782,29 +843,67 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
                 }
             }
         } else {
-        // Stage j & 1 holds tile j. Iteration j first starts tile j+1's transfer into the other
-        // stage (free: every wave passed the barrier that ended iteration j-1), computes tile j,
-        // then waits for its own transfers and meets the other waves: one barrier per tile.
-        if (n_tiles > 0) dma_tile(0, 0);
+        // Step i of key group kg is tile kg + KW i, in the group's stage i & 1. It first starts
+        // the next step's transfer into the other stage (free: every wave passed the barrier
+        // that ended step i-1), computes its tile, then waits for its own transfers and meets the
+        // other waves: one barrier per step, a group without a tile in the last step included.
+        const int gbase = kg * NST * STAGE;
+        const int n_steps = KW > 1 ? (n_tiles + KW - 1) / KW : n_tiles;
+        if (kg < n_tiles) dma_tile(kg, gbase);
         wait_dma();
         __syncthreads();
-        auto tile_step = [&](int tile, auto masked) {
-            st_r = (tile & 1) * STAGE;
+        auto tile_step = [&](int i, auto masked) {
+            const int tile = kg + KW * i;
+            st_r = gbase + (i & 1) * STAGE;
             st_k = st_v = st_r;
-            if (tile + 1 < n_tiles) dma_tile(tile + 1, STAGE - st_r);
-            f32x16_t sacc[2];
-            u32x4_t pop[4];
-            compute_s(sacc, std::true_type{}, no_hook);
-            softmax_max(sacc, tile, masked);
-            rescale_o();
-            softmax_exp(sacc, pop);
-            compute_pv(pop, no_hook);
+            if (tile + KW < n_tiles) dma_tile(tile + KW, gbase + STAGE - (i & 1) * STAGE);
+            if (KW == 1 || tile < n_tiles) {
+                f32x16_t sacc[2];
+                u32x4_t pop[4];
+                compute_s(sacc, std::true_type{}, no_hook);
+                softmax_max(sacc, tile, masked);
+                rescale_o();
+                softmax_exp(sacc, pop);
+                compute_pv(pop, no_hook);
+            }
             wait_dma();
             __syncthreads();
         };
-        int tile = 0;
-        for (; tile < n_full; ++tile) tile_step(tile, NoMask{});
-        for (; tile < n_tiles; ++tile) tile_step(tile, Mask{});
+        int i = 0;
+        for (; i < (n_full - kg + KW - 1) / KW; ++i) tile_step(i, NoMask{});
+        for (; i < n_steps; ++i) tile_step(i, Mask{});
+        }
+    } else if constexpr (KW > 1) {
+        // Step i of group kg is tile kg + KW i. The tile waits in registers until the group's
+        // stage is free; every wave of the workgroup meets the same barriers, a group without a
+        // tile left in the last step included. One stage: free after the barrier that ends the
+        // step before; two: stage i & 1 was last read in step i - 2.
+        const int gbase = kg * NST * STAGE;
+        const int n_steps = (n_tiles + KW - 1) / KW;
+        if (n_steps > 0) {
+            load_one(min(kg, n_tiles - 1), kb8, kreg);
+            load_v(min(kg, n_tiles - 1));
+        }
+        for (int i = 0; i < n_steps; ++i) {
+            const int tile = kg + KW * i;
+            st_w = st_r = gbase + (NST == 2 ? (i & 1) * STAGE : 0);
+            st_k = st_v = st_r;
+            if (NST == 1 && i > 0) __syncthreads();
+            store_k(tile);
+            store_v();
+            __syncthreads();
+            if (tile < n_tiles) {
+                load_one(min(tile + KW, n_tiles - 1), kb8, kreg);
+                load_v(min(tile + KW, n_tiles - 1));
+                f32x16_t sacc[2];
+                u32x4_t pop[4];
+                compute_s(sacc, std::true_type{}, no_hook);
+                if (tile < n_full) softmax_max(sacc, tile, NoMask{});
+                else softmax_max(sacc, tile, Mask{});
+                rescale_o();
+                softmax_exp(sacc, pop);
+                compute_pv(pop, no_hook);
+            }
         }
     } else {
         // Double-buffered: stage j & 1 holds tile j. Tile j+1 (loaded into registers one tile
@@ -847,6 +946,65 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         for (; tile < n_tiles; ++tile) tile_step(tile, Mask{});
     }
 
+    // ---- key groups: every wave scales its O by its weight in the row's result (the groups' m
+    // and l go through LDS) and leaves it in LDS as f32; all waves then add up and write rows.
+    if constexpr (KW > 1) {
+        float2* const ml_lds = (float2*)smem;  // [KW][RW][32]
+        const float l_own = l_run + xor32(l_run);
+        __syncthreads();
+        if (g == 0) ml_lds[(kg * RW + wave) * 32 + lane] = make_float2(m_run, l_own);
+        __syncthreads();
+        float mx = -INFINITY, l_all = 0.0f;
+        float2 ml[KW];
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            ml[k] = ml_lds[(k * RW + wave) * 32 + (lane & 31)];
+            mx = fmaxf(mx, ml[k].x);
+        }
+        // a group whose keys this row does not see: m = -inf, l = 0, O = 0
+#pragma unroll
+        for (int k = 0; k < KW; ++k)
+            l_all = fmaf(ml[k].y, ml[k].x == -INFINITY ? 0.0f : fast_exp2((ml[k].x - mx) * c2),
+                         l_all);
+        const float w =
+            (m_run == -INFINITY ? 0.0f : fast_exp2((m_run - mx) * c2)) * (1.0f / l_all);
+        if (kg == 0 && g == 0 && row_ok)
+            a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = mx * a.scale + logf(l_all);
+        __syncthreads();
+        uint8_t* const dst = smem + (kg * BM + wave * 32 + (lane & 31)) * MROW + 16 * g;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4)
+                *(f32x4_t*)(dst + mb * 128 + q4 * 32) =
+                    f32x4_t{oacc[mb][4 * q4] * w, oacc[mb][4 * q4 + 1] * w,
+                            oacc[mb][4 * q4 + 2] * w, oacc[mb][4 * q4 + 3] * w};
+        __syncthreads();
+        constexpr int RPP = 64 * NW / CPR;  // rows per pass, eight dims a thread
+        const int ch = tid % CPR;
+#pragma unroll
+        for (int r = tid / CPR; r < BM; r += RPP) {
+            f32x4_t s0 = (f32x4_t)0.0f, s1 = (f32x4_t)0.0f;
+#pragma unroll
+            for (int k = 0; k < KW; ++k) {
+                const uint8_t* src = smem + (k * BM + r) * MROW + ch * 32;
+                s0 += *(const f32x4_t*)src;
+                s1 += *(const f32x4_t*)(src + 16);
+            }
+            const int rr = r0 + r, t_r = (int)ka.grp.div((uint32_t)rr);
+            if (rr < rows_total && (FULLD || ch * 8 < D)) {
+                const int hq_r = kvh * a.group + rr - t_r * a.group;
+                uint16_t* o = (uint16_t*)a.o + (int64_t)b * a.o_sb + (int64_t)hq_r * a.o_sh +
+                              (int64_t)t_r * a.o_ss + ch * 8;
+                __builtin_nontemporal_store(
+                    u32x4_t{H::pack(s0[0], s0[1]), H::pack(s0[2], s0[3]), H::pack(s1[0], s1[1]),
+                            H::pack(s1[2], s1[3])},
+                    (u32x4_t*)o);
+            }
+        }
+        return;
+    }
+
     // ---- epilogue: the wave's 32 normalised O rows are staged in its own LDS region (free once
     // every wave has passed its last K/V read) and written back as whole rows with streaming
     // 16-byte stores, so they leave the caches while this compute-bound kernel still runs
@@ -882,8 +1040,6 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
     if (row_ok) {
         if (g == 0)
             a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = m_run * a.scale + logf(l_tot);
-    } else if (a.var_meta && row < rows_pad) {
-        write_padded_row<uint16_t>(a, b, kvh, row, g, D);
     }
 }
 
@@ -922,10 +1078,8 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5;
     const int D = a.head_dim, half = D >> 1;
     const int rows_pad = a.q_len * a.group;  // padded extent of the grid
-    const int nqb = (rows_pad + BM - 1) / BM;
-    int bh, qb;
-    block_coords(blockIdx.x, gridDim.x, nqb, bh, qb);
-    const int b = bh / a.kv_heads, kvh = bh % a.kv_heads;
+    int b, kvh, qb;
+    block_coords(ka, blockIdx.x, b, kvh, qb);
     const int r0 = qb * BM;
     // Per-sequence extents of a variable-length batch (PrefillArgs::var_meta); the grid covers
     // the padded extents. A block of padded query rows only writes O = 0, LSE = -inf.
@@ -939,18 +1093,18 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
         q_rope_off_ = m[3];
     }
     const int rows_total = q_len_ * a.group;
-    if (a.var_meta && r0 >= rows_total) {
-        const int prow = r0 + wave * 32 + (lane & 31);
-        if (prow < rows_pad) write_padded_row<float>(a, b, kvh, prow, g, D);
-        return;
+    if (a.var_meta && r0 + BM > rows_total) {
+        write_padded_rows<float>(ka, b, kvh, max(r0, rows_total), min(r0 + BM, rows_pad), D);
+        if (r0 >= rows_total) return;
     }
     const int row = r0 + wave * 32 + (lane & 31);
     const bool row_ok = row < rows_total;
-    const int t = row_ok ? row / a.group : q_len_ - 1;
-    const int hq = kvh * a.group + (row_ok ? row % a.group : 0);
+    const int row_t = (int)ka.grp.div((uint32_t)row);
+    const int t = row_ok ? row_t : q_len_ - 1;
+    const int hq = kvh * a.group + (row_ok ? row - row_t * a.group : 0);
     const int cpos = causal_off_ + t;
-    const int t_max = min(q_len_ - 1, (r0 + BM - 1) / a.group);
-    const int t_min = r0 / a.group;
+    const int t_max = min(q_len_ - 1, (int)ka.grp.div((uint32_t)(r0 + BM - 1)));
+    const int t_min = (int)ka.grp.div((uint32_t)r0);
     int n_keys = kv_len_;
     if (a.causal) n_keys = min(n_keys, causal_off_ + t_max + 1);
     const int n_tiles = (n_keys + BN - 1) / BN;
@@ -1192,8 +1346,6 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
             }
         if (g == 0)
             a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = m_run * a.scale + logf(l_tot);
-    } else if (a.var_meta && row < rows_pad) {
-        write_padded_row<float>(a, b, kvh, row, g, D);
     }
 }
 
@@ -1220,8 +1372,45 @@ static void launch16r(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s
     }
 }
 
+// The key-group variants: eight waves, KW groups.
+template <typename T, int PMODE, bool ROPEK, int KW>
+static void launch16k(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s) {
+    const bool full = ka.a.head_dim == dpad;
+    switch (dpad) {
+        case 32:
+            full ? prefill_mfma16<T, 32, PMODE, ROPEK, true, 8, false, KW><<<grid, 512, 0, s>>>(ka)
+                 : prefill_mfma16<T, 32, PMODE, ROPEK, false, 8, false, KW><<<grid, 512, 0, s>>>(ka);
+            break;
+        case 64:
+            full ? prefill_mfma16<T, 64, PMODE, ROPEK, true, 8, false, KW><<<grid, 512, 0, s>>>(ka)
+                 : prefill_mfma16<T, 64, PMODE, ROPEK, false, 8, false, KW><<<grid, 512, 0, s>>>(ka);
+            break;
+        default:
+            full ? prefill_mfma16<T, 128, PMODE, ROPEK, true, 8, false, KW><<<grid, 512, 0, s>>>(ka)
+                 : prefill_mfma16<T, 128, PMODE, ROPEK, false, 8, false, KW><<<grid, 512, 0, s>>>(ka);
+            break;
+    }
+}
+
+template <typename T, int KW>
+static void launch16k_mode(const PrefillKArgs& ka, bool paged, int dpad, dim3 grid,
+                           hipStream_t s) {
+    if (!paged) {
+        if (ka.a.rope_k) launch16k<T, kContig, true, KW>(ka, dpad, grid, s);
+        else launch16k<T, kContig, false, KW>(ka, dpad, grid, s);
+    } else {
+        launch16k<T, kPaged16, false, KW>(ka, dpad, grid, s);
+    }
+}
+
 template <typename T>
 static void launch16(const PrefillKArgs& ka, bool paged, int dpad, dim3 grid, hipStream_t s) {
+    if (const int kw = prefill_key_groups(
+            std::is_same<T, bf16_t>::value ? Dtype::BF16 : Dtype::F16, paged, ka.a)) {
+        if (kw == 4) launch16k_mode<T, 4>(ka, paged, dpad, grid, s);
+        else launch16k_mode<T, 2>(ka, paged, dpad, grid, s);
+        return;
+    }
     if (!paged) {
         if (ka.a.rope_k && ka.a.split_qk) {
             launch16r<T, kContig, true, true>(ka, dpad, grid, s);
@@ -1256,8 +1445,52 @@ static void launch32(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s)
     }
 }
 
+// Which launches take key groups (times in us per call, bf16, the whole call; other loop / two
+// groups / four groups; one workgroup of them fills a CU's LDS at D 128):
+//   four, while 64-row blocks do not outnumber the CUs:
+//     causal RoPE Hq8 Hkv2 S1024 D64 24.3 / 17.5 / 14.6, D128 28.2 (assembly) / 23.3 / 20.8;
+//     Hq32 Hkv8 S512 D128, 256 blocks, 19.6 / 17.4 / 16.0; S1024, 512 blocks, 28.8 / 24.5 / 29.9;
+//     H16 S2048 D128, 512 blocks, 48.3 / 32.6 / 34.2;
+//   two, while 128-row blocks do not outnumber the CUs (the assembly loop: H32/8 S1024, 256
+//     blocks, 28.8 / 24.5; twice that 31.8 / 35.7), or two rounds of them where the other loop is
+//     the ping-pong one (B2 H16 S2048 D128, 512 blocks, 52.5 / 44.5; B4 H16 S2048, 1024 blocks,
+//     74.9 / 88.9; D64 B4 H16 S1024, 512 blocks, 22.4 / 19.8), or four at D 32 (B4 H16 S2048, 39.7
+//     / 33.9). A padded batch has blocks without work: one round (six sequences up to 300 x 500,
+//     480 blocks, 29.9 / 31.9).
+//   Under six key tiles the assembly kernel stays: its fixed cost is the smaller one (S128 12.8
+//   against 11.9, S300 level). Paged pools that it reads stay with it (one 16-query chunk over
+//   2048 cached tokens 54.6 / 67.5 / 60.7): the key groups wait for each tile's page ids.
+int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a) {
+    if (dt == Dtype::F32 || a.split_qk || a.k_lo || (paged && a.page_size % 16)) return 0;
+    const bool a64 = prefill_a64_eligible(dt, paged, a);
+    if (a64 && (paged || a.a64 == kA64Always)) return 0;
+    const int64_t keys =
+        a.causal ? std::min<int64_t>(a.kv_len, (int64_t)a.causal_offset + a.q_len) : a.kv_len;
+    const int64_t tiles = (keys + 63) / 64;
+    if (tiles < (a64 ? 6 : 2)) return 0;
+    const int64_t cus = device_cus(), rows = (int64_t)a.q_len * a.group;
+    const int64_t units = (int64_t)a.batch * a.kv_heads;
+    const int64_t rounds = a64 || a.var_meta ? 1 : a.head_dim <= 32 ? 4 : 2;
+    if (units * ((rows + 63) / 64) <= cus) return 4;
+    if (units * ((rows + 127) / 128) <= rounds * cus) return 2;
+    return 0;
+}
+
+bool prefill_uses_a64(Dtype dt, bool paged, const PrefillArgs& a) {
+    return !prefill_key_groups(dt, paged, a) && prefill_a64_eligible(dt, paged, a);
+}
+
 void prefill_geometry(Dtype dt, bool paged, const PrefillArgs& a, unsigned grid[3],
                       unsigned* block, unsigned* rows) {
+    if (const int kw = prefill_key_groups(dt, paged, a)) {
+        const int bm = 256 / kw;
+        grid[0] = (unsigned)((int64_t)a.batch * a.kv_heads *
+                             (((int64_t)a.q_len * a.group + bm - 1) / bm));
+        grid[1] = grid[2] = 1;
+        *block = 512;
+        *rows = (unsigned)bm;
+        return;
+    }
     if (prefill_a64_eligible(dt, paged, a)) {  // assembly kernel: 4 waves x 64 rows, persistent
         grid[0] = prefill_a64_workgroups(a);
         grid[1] = grid[2] = 1;
@@ -1282,12 +1515,13 @@ void launch_prefill(Dtype dt, bool paged, const PrefillArgs& a, hipStream_t s, u
     ka.a = a;
     if (paged) ka.ps = FastDiv((uint32_t)a.page_size);
     const int dpad = a.head_dim <= 32 ? 32 : (a.head_dim <= 64 ? 64 : 128);
-    if (prefill_a64_eligible(dt, paged, a)) {
+    if (prefill_uses_a64(dt, paged, a)) {
         launch_prefill_a64(dt, a, paged, s, grid, block);
         return;
     }
     unsigned rows;
     prefill_geometry(dt, paged, a, grid, block, &rows);
+    ka.set_grid(grid[0], rows);
     dim3 g(grid[0]);
     switch (dt) {
         case Dtype::BF16: launch16<bf16_t>(ka, paged, dpad, g, s); break;

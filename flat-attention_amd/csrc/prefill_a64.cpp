@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <atomic>
 #include <mutex>
 
 #include "kernels.hpp"
@@ -81,6 +82,18 @@ hipError_t prefill_a64_load(int device) {
     return hipSuccess;
 }
 
+int device_cus() {
+    static std::atomic<int> known[kMaxDevices];
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+    if ((cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus <= 0)
+        return 256;
+    known[dev].store(cus, std::memory_order_relaxed);
+    return cus;
+}
+
 bool prefill_a64_eligible(Dtype dt, bool paged, const PrefillArgs& a) {
     if (!a.a64 || (dt != Dtype::BF16 && dt != Dtype::F16) || a.head_dim != 128 || a.rope_k ||
         a.split_qk || a.var_meta)
@@ -125,10 +138,7 @@ bool prefill_a64_eligible(Dtype dt, bool paged, const PrefillArgs& a) {
 
 unsigned prefill_a64_workgroups(const PrefillArgs& a) {
     const uint64_t nb = (uint64_t)a.batch * a.kv_heads * (((int64_t)a.q_len * a.group + 255) / 256);
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    return (unsigned)std::min<uint64_t>(nb, (uint64_t)std::max(cus, 1));
+    return (unsigned)std::min<uint64_t>(nb, (uint64_t)device_cus());
 }
 
 void launch_prefill_a64(Dtype dt, const PrefillArgs& a, bool paged, hipStream_t s,

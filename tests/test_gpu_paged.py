@@ -521,6 +521,36 @@ def test_paged_prefill_modes_match_oracle_and_gather_bit_exactly(hip, dtype, ps,
         assert_close(f"LSE seq {s}", l1[s * hq * ql:(s + 1) * hq * ql], el, atol, rtol)
 
 
+@pytest.mark.parametrize("ps,D,cached,ql,groups", [(16, 64, 3, 70, 4), (32, 64, 300, 50, 4),
+                                                   (32, 128, 90, 33, 4), (48, 64, 200, 700, 2)])
+def test_paged_prefill_key_groups_match_oracle_and_gather_bit_exactly(hip, ps, D, cached, ql,
+                                                                      groups):
+    """The key-group prefill over a paged cache: pages of one and several 16-key groups, key
+    tiles and pages that end part-way; identity and shuffled tables bitwise identical."""
+    dtype, n_seqs, hq, hkv, theta = fa.DTYPE_BF16, 2, 16, 8, 1e4
+    kv_len = cached + ql
+    pages_per = -(-kv_len // ps)
+    total = n_seqs * pages_per + 3
+    width = hkv * D
+    raw_k = bf16_round(normal(n_seqs * kv_len * width, 61 + ps))
+    v = bf16_round(normal(n_seqs * kv_len * width, 62 + ps))
+    q = bf16_round(normal(n_seqs * ql * hq * D, 63 + ps))
+    ident = np.arange(n_seqs * pages_per, dtype=np.int32).reshape(n_seqs, pages_per)
+    shuf = np.random.default_rng(ps).permutation(total)[:n_seqs * pages_per].astype(
+        np.int32).reshape(n_seqs, pages_per)
+    o1, l1 = _paged_prefill(hip, ident, ps, total, n_seqs, hq, hkv, D, cached, ql, theta, raw_k,
+                            v, q, dtype, True)
+    assert hip.last_telemetry().query_rows == 256 // groups
+    o2, l2 = _paged_prefill(hip, shuf, ps, total, n_seqs, hq, hkv, D, cached, ql, theta, raw_k,
+                            v, q, dtype, True)
+    assert np.array_equal(o1.view(np.uint32), o2.view(np.uint32))
+    assert np.array_equal(l1.view(np.uint32), l2.view(np.uint32))
+    eo, el = oracle.forward_projection_asymmetric(q, raw_k, v, n_seqs, hq, hkv, ql, kv_len, D,
+                                                  cached, True, theta, cached, 0, True)
+    assert_close("O", o1, eo, H16_ATOL, 0.0)
+    assert_close("LSE", l1, el, H16_ATOL, 0.0)
+
+
 @pytest.mark.parametrize("pattern", ["rising", "falling", "alternating"])
 @pytest.mark.parametrize("dtype", [fa.DTYPE_BF16, fa.DTYPE_F16])
 @pytest.mark.parametrize("layout", ["1", "0"])

@@ -156,6 +156,61 @@ def _gqa_rope_16bit(hip, dtype, rnd, D):
         assert_close("LSE", l, el, H16_ATOL, 0.0)
 
 
+@pytest.mark.parametrize("dtype,rnd", [(fa.DTYPE_BF16, bf16_round), (fa.DTYPE_F16, f16_round)])
+@pytest.mark.parametrize("B,hq,hkv,S,D,rope,groups", [
+    (1, 8, 2, 65, 64, True, 4),      # two key tiles: groups 2 and 3 have none; K rotated on load
+    (1, 6, 1, 127, 40, True, 4),     # head dim below the padded width, group of 6
+    (1, 8, 2, 515, 64, True, 4),     # nine tiles, the last of three keys; K rotated by the pre-pass
+    (1, 8, 2, 400, 128, True, 4),    # where the assembly kernel would apply
+    (2, 4, 4, 333, 128, False, 4),   # MHA, no RoPE, the last block of 13 rows
+    (1, 32, 8, 900, 128, True, 2),   # 15 tiles: the second group has none in the last step
+    (2, 24, 24, 130, 80, False, 4),  # 80 dims, the last block of 2 rows
+    (4, 16, 16, 300, 64, False, 2),  # five tiles
+    (4, 64, 64, 200, 32, False, 2),  # two rounds of workgroups
+])
+@pytest.mark.parametrize("causal", [True, False])
+def test_key_group_prefill_matches_oracle(hip, dtype, rnd, B, hq, hkv, S, D, rope, groups, causal):
+    """prefill_mfma16 with its waves split over key groups: row blocks and key tiles that end
+    part-way, groups without a tile, rows that see no key of a group's first tile (causal)."""
+    q = rnd(normal(B * hq * S * D, 700 + S))
+    k, v = rnd(normal(B * hkv * S * D, 701 + S)), rnd(normal(B * hkv * S * D, 702 + S))
+    shape = fa.GroupedAttentionShape(B, hq, hkv, S, D)
+    rot = fa.RotaryEmbeddingConfig(1e4, 3) if rope else None
+    o, l = _run_grouped(hip, q, k, v, shape, fa.FlatAttentionConfig(causal), rot, dtype)
+    t = hip.last_telemetry()
+    assert "prefill_mfma16" in t.kernel_name
+    assert (t.query_rows, t.workgroup_size) == (256 // groups, 512)
+    units = (0, min(B * hq, 16))
+    eo, el = _oracle_grouped(q, k, v, shape, causal, rot, units=units)
+    n = (units[1] - units[0]) * S
+    assert_close("O", o[:n * D], eo[:n * D], H16_ATOL, 0.0)
+    assert_close("LSE", l[:n], el[:n], H16_ATOL, 0.0)
+    assert np.isfinite(o).all() and np.isfinite(l).all()
+
+
+@pytest.mark.parametrize("kind", ["rising", "falling", "far_apart"])
+def test_key_group_merge_with_extreme_scores(hip, kind):
+    """The key groups' running maxima far apart: every group's last tile outweighs, or is
+    outweighed by, the others' by more than the f32 exponent range."""
+    S, D, H = 512, 64, 2
+    idx = np.arange(S, dtype=np.float32)
+    scores = {"rising": 0.5 * idx, "falling": -0.5 * idx,
+              "far_apart": np.where((np.arange(S) // 64) % 4 == 2, 200.0, -200.0)}[kind]
+    q = np.zeros((H, S, D), np.float32)
+    k = np.zeros((H, S, D), np.float32)
+    q[:, :, 0] = 8.0
+    k[:, :, 0] = bf16_round(scores.astype(np.float32))
+    v = bf16_round(normal(H * S * D, 9))
+    shape = fa.GroupedAttentionShape(1, H, H, S, D)
+    for causal in (True, False):
+        o, l = _run_grouped(hip, q.ravel(), k.ravel(), v, shape, fa.FlatAttentionConfig(causal),
+                            None, fa.DTYPE_BF16)
+        assert hip.last_telemetry().query_rows == 64
+        eo, el = _oracle_grouped(q.ravel(), k.ravel(), v, shape, causal, None)
+        assert_close("O", o, eo, H16_ATOL, 0.0)
+        assert_close("LSE", l, el, H16_ATOL, 0.0)
+
+
 def test_prerotated_and_fused_k_rotation_are_bit_identical(hip):
     B, hq, hkv, S, D = 1, 8, 2, 150, 128
     q, k, v = (bf16_round(normal(n, s)) for n, s in
