@@ -1349,6 +1349,207 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
     }
 }
 
+// ------------------------------------------------------------------ f32, key groups
+// The f32 kernel for launches whose 128-row blocks would leave most of the chip idle: 32 rows to a
+// workgroup, whose NW waves take the 32-key tiles in turn and are merged in LDS at the end. A
+// tile is 4096 (D 64) or 8192 (D 128) clocks of f32 MFMA to a wave, so operands go straight from
+// memory into registers: K rows of the next tile and V columns of the next 32 dims are loaded
+// under the products. Same mapping as prefill_mfma_f32 (lane group g: k-index g of every step).
+// Contiguous K/V that is not rotated here, 16-byte aligned rows, head_dim % 4 == 0.
+template <int DPAD, int NW, bool FULL>
+__global__ __launch_bounds__(64 * NW, DPAD == 128 ? 1 : 2) void prefill_f32_groups(PrefillKArgs ka) {
+    const PrefillArgs& a = ka.a;
+    constexpr int HALFD = DPAD / 2, MB = DPAD / 32, NV = HALFD / 4;
+    constexpr int OROW = DPAD * 4 + 16;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NW * 32 * OROW];
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, c = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int D = a.head_dim, half = D >> 1;
+    int b, kvh, qb;
+    block_coords(ka, blockIdx.x, b, kvh, qb);
+    const int r0 = qb * 32;
+    int q_len_ = a.q_len, kv_len_ = a.kv_len, causal_off_ = a.causal_offset;
+    int q_rope_off_ = a.q_rope_offset;
+    if (a.var_meta) {
+        const int* m = a.var_meta + 4 * b;
+        q_len_ = m[0];
+        kv_len_ = m[1];
+        causal_off_ = m[2];
+        q_rope_off_ = m[3];
+    }
+    const int rows_total = q_len_ * a.group;
+    if (a.var_meta && r0 + 32 > rows_total) {
+        write_padded_rows<float>(ka, b, kvh, max(r0, rows_total),
+                                 min(r0 + 32, a.q_len * a.group), D);
+        if (r0 >= rows_total) return;
+    }
+    const int row = r0 + c;
+    const bool row_ok = row < rows_total;
+    const int row_t = (int)ka.grp.div((uint32_t)row);
+    const int t = row_ok ? row_t : q_len_ - 1;
+    const int hq = kvh * a.group + (row_ok ? row - row_t * a.group : 0);
+    const int t_max = min(q_len_ - 1, (int)ka.grp.div((uint32_t)(r0 + 31)));
+    const int t_min = (int)ka.grp.div((uint32_t)r0);
+    int n_keys = kv_len_;
+    if (a.causal) n_keys = min(n_keys, causal_off_ + t_max + 1);
+    const int n_tiles = __builtin_amdgcn_readfirstlane((n_keys + 31) / 32);
+    // last key that this lane's row sees, first key that some row of the block does not
+    const int lim = a.causal ? min(kv_len_ - 1, causal_off_ + t) : kv_len_ - 1;
+    const int clear = a.causal ? min(kv_len_, causal_off_ + t_min + 1) : kv_len_;
+
+    const int row_bytes = (int)a.k_ss * 4;
+    const int64_t head = ((int64_t)b * a.k_sb + (int64_t)kvh * a.k_sh) * 4;
+    const int nrec = (kv_len_ - 1) * row_bytes + D * 4;
+    auto tile_of = [&](const void* base, int tile) {
+        const int at = tile * 32 * row_bytes;
+        return __builtin_amdgcn_make_buffer_rsrc((uint8_t*)base + head + at, (short)0, nrec - at,
+                                                 0x00020000);
+    };
+    f32x4_t kr[NV];
+    auto load_k = [&](int tile) {
+        const __amdgpu_buffer_rsrc_t rs = tile_of(a.k, tile);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int d = g * HALFD + 4 * j;
+            const int off = FULL || d < D ? c * row_bytes + d * 4 : 0x7fffff00;
+            kr[j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+        }
+    };
+    // Column 32 mb + c of V rows 8 (i / 4) + 4 g + i % 4 (past D: values of columns never stored)
+    auto load_v = [&](__amdgpu_buffer_rsrc_t rs, int mb, float (&vc)[16]) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            vc[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                rs, 4 * g * row_bytes + c * 4, (8 * (i >> 2) + (i & 3)) * row_bytes + mb * 128, 0));
+    };
+    if (wave < n_tiles) load_k(wave);
+
+    f32x4_t qv[NV];
+    {
+        const float* qrow = (const float*)a.q + (int64_t)b * a.q_sb + (int64_t)hq * a.q_sh +
+                            (int64_t)t * a.q_ss;
+        const float2* cs = a.rope_q ? a.rope_table + (int64_t)(q_rope_off_ + t) * half : nullptr;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int d = g * HALFD + 4 * j;
+            qv[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            if (FULL || d < D) qv[j] = *(const f32x4_t*)(qrow + d);
+        }
+        if (a.rope_q) {
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int d = g * HALFD + 4 * j;
+                if (FULL || d < D) {
+                    const float2 c0 = cs[d / 2], c1 = cs[d / 2 + 1];
+                    float e0 = qv[j][0], o0 = qv[j][1], e1 = qv[j][2], o1 = qv[j][3];
+                    rope_pair(e0, o0, c0.x, c0.y);
+                    rope_pair(e1, o1, c1.x, c1.y);
+                    qv[j] = f32x4_t{e0, o0, e1, o1};
+                }
+            }
+        }
+    }
+
+    f32x16_t oacc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) oacc[mb] = (f32x16_t)0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+    const float c2 = a.scale * kLog2e;
+    for (int tile = wave; tile < n_tiles; tile += NW) {
+        f32x16_t s = (f32x16_t)0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j][e], qv[j][e], s, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        const __amdgpu_buffer_rsrc_t rv = tile_of(a.v, tile);
+        float vc[16];
+        load_v(rv, 0, vc);
+        __builtin_amdgcn_sched_barrier(0);
+        if (tile * 32 + 32 > clear) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (tile * 32 + 8 * (i >> 2) + 4 * g + (i & 3) > lim) s[i] = -INFINITY;
+        }
+        float mt = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mt = fmaxf(mt, s[i]);
+        mt = fmaxf(mt, xor32(mt));
+        const bool need = mt * c2 > m_run * c2 + kRescaleLog2;
+        if (__any(need)) {
+            const float m_use = need ? mt : m_run;
+            // (m_run = -inf: 0, and a row that sees no key of the tile keeps its zeros)
+            const float alpha = need ? fast_exp2((m_run - m_use) * c2) : 1.0f;
+            l_run *= alpha;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) oacc[mb] *= alpha;
+            m_run = m_use;
+        }
+        const float neg = m_run == -INFINITY ? 0.0f : -m_run * c2;
+        float lsum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = fast_exp2(fmaf(s[i], c2, neg));
+            lsum += s[i];
+        }
+        l_run += lsum;
+        if (tile + NW < n_tiles) load_k(tile + NW);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            float vm[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) vm[i] = vc[i];
+            __builtin_amdgcn_sched_barrier(0);
+            if (mb + 1 < MB) load_v(rv, mb + 1, vc);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                oacc[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(vm[i], s[i], oacc[mb], 0, 0, 0);
+        }
+    }
+
+    // ---- merge: every wave scales its O by its weight in the row's result, all add up rows
+    float2* const ml_lds = (float2*)smem;
+    const float l_own = l_run + xor32(l_run);
+    if (g == 0) ml_lds[wave * 32 + c] = make_float2(m_run, l_own);
+    __syncthreads();
+    float mx = -INFINITY, l_all = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) mx = fmaxf(mx, ml_lds[k * 32 + c].x);
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+        const float2 ml = ml_lds[k * 32 + c];
+        l_all = fmaf(ml.y, ml.x == -INFINITY ? 0.0f : fast_exp2((ml.x - mx) * c2), l_all);
+    }
+    const float w = (m_run == -INFINITY ? 0.0f : fast_exp2((m_run - mx) * c2)) * (1.0f / l_all);
+    if (wave == 0 && g == 0 && row_ok)
+        a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = mx * a.scale + logf(l_all);
+    __syncthreads();
+    uint8_t* const dst = smem + (wave * 32 + c) * OROW + 16 * g;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+            *(f32x4_t*)(dst + mb * 128 + q4 * 32) =
+                f32x4_t{oacc[mb][4 * q4] * w, oacc[mb][4 * q4 + 1] * w, oacc[mb][4 * q4 + 2] * w,
+                        oacc[mb][4 * q4 + 3] * w};
+    __syncthreads();
+    constexpr int CH = DPAD / 4, RPP = 64 * NW / CH;
+    const int ch = tid % CH;
+    for (int r = tid / CH; r < 32; r += RPP) {
+        f32x4_t o = (f32x4_t)0.0f;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) o += *(const f32x4_t*)(smem + (k * 32 + r) * OROW + ch * 16);
+        const int rr = r0 + r, t_r = (int)ka.grp.div((uint32_t)rr);
+        if (rr < rows_total && (FULL || ch * 4 < D)) {
+            const int hq_r = kvh * a.group + rr - t_r * a.group;
+            *(f32x4_t*)((float*)a.o + (int64_t)b * a.o_sb + (int64_t)hq_r * a.o_sh +
+                        (int64_t)t_r * a.o_ss + ch * 4) = o;
+        }
+    }
+}
+
 // ------------------------------------------------------------------ launcher
 template <typename T, int PMODE, bool ROPEK, bool SPLIT = false>
 static void launch16r(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s) {
@@ -1460,6 +1661,24 @@ static void launch32(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s)
 //   Under six key tiles the assembly kernel stays: its fixed cost is the smaller one (S128 12.8
 //   against 11.9, S300 level). Paged pools that it reads stay with it (one 16-query chunk over
 //   2048 cached tokens 54.6 / 67.5 / 60.7): the key groups wait for each tile's page ids.
+static void launch32g(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s) {
+    const bool full = ka.a.head_dim == dpad;
+    switch (dpad) {
+        case 32:
+            full ? launch_timed(prefill_f32_groups<32, 8, true>, grid, dim3(512), s, ka)
+                 : launch_timed(prefill_f32_groups<32, 8, false>, grid, dim3(512), s, ka);
+            break;
+        case 64:
+            full ? launch_timed(prefill_f32_groups<64, 8, true>, grid, dim3(512), s, ka)
+                 : launch_timed(prefill_f32_groups<64, 8, false>, grid, dim3(512), s, ka);
+            break;
+        default:
+            full ? launch_timed(prefill_f32_groups<128, 4, true>, grid, dim3(256), s, ka)
+                 : launch_timed(prefill_f32_groups<128, 4, false>, grid, dim3(256), s, ka);
+            break;
+    }
+}
+
 int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a) {
     if (dt == Dtype::F32 || a.split_qk || a.k_lo || (paged && a.page_size % 16)) return 0;
     const bool a64 = prefill_a64_eligible(dt, paged, a);
@@ -1480,6 +1699,29 @@ bool prefill_uses_a64(Dtype dt, bool paged, const PrefillArgs& a) {
     return !prefill_key_groups(dt, paged, a) && prefill_a64_eligible(dt, paged, a);
 }
 
+// Contiguous f32 rows that buffer loads and transfers take: 16-byte aligned, one (batch, kv head)
+// slice addressable by 32-bit offsets.
+static bool f32_rows_ok(const PrefillArgs& a) {
+    return !a.rope_k && a.head_dim % 4 == 0 && (uintptr_t)a.k % 16 == 0 && (uintptr_t)a.v % 16 == 0 &&
+           a.k_ss % 4 == 0 && a.k_sh % 4 == 0 && a.k_sb % 4 == 0 &&
+           (uint64_t)a.kv_len * (uint64_t)a.k_ss * 4u <= INT32_MAX;
+}
+
+// f32 launches that take prefill_f32_groups: those whose 128-row blocks do not fill the places of
+// prefill_mfma_f32, two to a CU (times in us per call, that kernel / this one): H2 S128 D64 causal
+// 19.4 / 7.4, B4 H2 S655 D128 105.0 / 35.2, H8 S2048 D64 causal 161.6 / 49.2, B4 H16 S512 D128
+// causal, 256 blocks, 91.4 / 66.8; at 512 blocks H16 B2 S2048 D128 397.7 / 340.8, but Hq32 Hkv8
+// B2 S1000 D64 121.8 / 129.6; at 1024 blocks B4 H16 S2048 D128 628.8 / 691.2, where the tiles
+// that four waves share in LDS count for more.
+static bool prefill_f32_grouped(bool paged, const PrefillArgs& a) {
+    if (paged || !f32_rows_ok(a) || (uintptr_t)a.q % 16 || a.q_ss % 4 || a.q_sh % 4 || a.q_sb % 4 ||
+        (uintptr_t)a.o % 16 || a.o_ss % 4 || a.o_sh % 4 || a.o_sb % 4)
+        return false;
+    const int64_t blocks = (int64_t)a.batch * a.kv_heads *
+                           (((int64_t)a.q_len * a.group + 127) / 128);
+    return blocks < 2 * (int64_t)device_cus() + (a.head_dim > 64 ? 1 : 0);
+}
+
 void prefill_geometry(Dtype dt, bool paged, const PrefillArgs& a, unsigned grid[3],
                       unsigned* block, unsigned* rows) {
     if (const int kw = prefill_key_groups(dt, paged, a)) {
@@ -1496,6 +1738,14 @@ void prefill_geometry(Dtype dt, bool paged, const PrefillArgs& a, unsigned grid[
         grid[1] = grid[2] = 1;
         *block = 256;
         *rows = 256;
+        return;
+    }
+    if (dt == Dtype::F32 && prefill_f32_grouped(paged, a)) {
+        grid[0] = (unsigned)((int64_t)a.batch * a.kv_heads *
+                             (((int64_t)a.q_len * a.group + 31) / 32));
+        grid[1] = grid[2] = 1;
+        *block = a.head_dim > 64 ? 256 : 512;
+        *rows = 32;
         return;
     }
     // 16-bit contiguous K/V without in-kernel K rotation runs 256-row ping-pong workgroups
@@ -1528,12 +1778,9 @@ void launch_prefill(Dtype dt, bool paged, const PrefillArgs& a, hipStream_t s, u
         case Dtype::F16: launch16<f16_t>(ka, paged, dpad, g, s); break;
         default:
             if (paged) launch32<true>(ka, dpad, g, s);
-            // transfers: 16-byte aligned rows, and one (batch, kv head) slice addressable by
-            // 32-bit buffer offsets (register staging uses 64-bit addresses)
-            else if (!a.rope_k && a.head_dim % 4 == 0 && (uintptr_t)a.k % 16 == 0 &&
-                     (uintptr_t)a.v % 16 == 0 && a.k_ss % 4 == 0 && a.k_sh % 4 == 0 &&
-                     a.k_sb % 4 == 0 && (uint64_t)a.kv_len * (uint64_t)a.k_ss * 4u <= INT32_MAX)
-                launch32<false, true>(ka, dpad, g, s);
+            else if (prefill_f32_grouped(paged, a)) launch32g(ka, dpad, g, s);
+            // transfers (register staging uses 64-bit addresses)
+            else if (f32_rows_ok(a)) launch32<false, true>(ka, dpad, g, s);
             else launch32<false>(ka, dpad, g, s);
             break;
     }

@@ -156,6 +156,27 @@ def _gqa_rope_16bit(hip, dtype, rnd, D):
         assert_close("LSE", l, el, H16_ATOL, 0.0)
 
 
+@pytest.mark.parametrize("B,hq,hkv,S,D,rope,rows", [
+    (1, 2, 2, 1, 32, False, 32), (1, 4, 2, 33, 64, True, 32), (1, 3, 1, 257, 128, True, 32),
+    (2, 2, 2, 300, 20, False, 32), (1, 6, 3, 65, 100, True, 32),
+    (1, 8, 8, 70, 42, False, 128),     # head dim off the 16-byte chunk: the staged kernel
+    (8, 64, 64, 20, 64, False, 128),   # 512 blocks of 128 rows: the LDS kernel's two per CU
+    (8, 64, 64, 20, 80, False, 32), (8, 66, 66, 20, 80, False, 128)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_f32_key_group_prefill_matches_oracle(hip, B, hq, hkv, S, D, rope, rows, causal):
+    """f32 rows whose 32-key tiles are dealt to the waves of a 32-row workgroup: fewer tiles than
+    waves, row blocks and tiles that end part-way, columns past the head dim; and which kernel."""
+    q = normal(B * hq * S * D, 750 + S)
+    k, v = normal(B * hkv * S * D, 751 + S), normal(B * hkv * S * D, 752 + S)
+    shape = fa.GroupedAttentionShape(B, hq, hkv, S, D)
+    rot = fa.RotaryEmbeddingConfig(1e4, 3) if rope and D % 8 == 0 else None
+    o, l = _run_grouped(hip, q, k, v, shape, fa.FlatAttentionConfig(causal), rot, fa.DTYPE_F32)
+    assert hip.last_telemetry().query_rows == rows
+    eo, el = _oracle_grouped(q, k, v, shape, causal, rot)
+    assert_close("O", o, eo, F32_ATOL, F32_RTOL)
+    assert_close("LSE", l, el, F32_ATOL, F32_RTOL)
+
+
 @pytest.mark.parametrize("dtype,rnd", [(fa.DTYPE_BF16, bf16_round), (fa.DTYPE_F16, f16_round)])
 @pytest.mark.parametrize("B,hq,hkv,S,D,rope,groups", [
     (1, 8, 2, 65, 64, True, 4),      # two key tiles: groups 2 and 3 have none; K rotated on load
