@@ -999,7 +999,7 @@ void launch_dma(const BackwardArgs& a, hipStream_t s) {
 }
 
 template <typename T>
-void launch_dims(const BackwardArgs& a, hipStream_t s, bool* a64_out) {
+void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, bool* a64_out) {
     const int64_t rows = (int64_t)a.batch * a.q_heads * a.seq;
     if constexpr (std::is_same_v<T, bf16_t> || std::is_same_v<T, f16_t>) {
         constexpr Dtype dt = std::is_same_v<T, bf16_t> ? Dtype::BF16 : Dtype::F16;
@@ -1017,6 +1017,12 @@ void launch_dims(const BackwardArgs& a, hipStream_t s, bool* a64_out) {
     if (a64_out) *a64_out = false;
     hipLaunchKernelGGL((bwd_delta<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, s, a,
                        rows);
+    if constexpr (std::is_same_v<T, float>) {
+        // (no split: head dims above 64 only)
+        if (sp.parts > 0) launch_backward_f32(a, sp, s);
+        else launch_dma<float, 128>(a, s);
+        return;
+    }
     if (a.head_dim <= 32) launch_dma<T, 32>(a, s);
     else if (a.head_dim <= 64) launch_dma<T, 64>(a, s);
     else launch_dma<T, 128>(a, s);
@@ -1024,11 +1030,12 @@ void launch_dims(const BackwardArgs& a, hipStream_t s, bool* a64_out) {
 
 }  // namespace
 
-void launch_backward(Dtype dt, const BackwardArgs& a, hipStream_t s, bool* a64_out) {
+void launch_backward(Dtype dt, const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s,
+                     bool* a64_out) {
     switch (dt) {
-        case Dtype::F32: launch_dims<float>(a, s, a64_out); break;
-        case Dtype::F16: launch_dims<f16_t>(a, s, a64_out); break;
-        case Dtype::BF16: launch_dims<bf16_t>(a, s, a64_out); break;
+        case Dtype::F32: launch_dims<float>(a, sp, s, a64_out); break;
+        case Dtype::F16: launch_dims<f16_t>(a, sp, s, a64_out); break;
+        case Dtype::BF16: launch_dims<bf16_t>(a, sp, s, a64_out); break;
     }
 }
 

@@ -179,6 +179,9 @@ struct fa_ctx {
     // growable scratch for the backward's stored dS (16-bit storage; fa_ctx_set_backward_policy)
     void* ws_ds = nullptr;
     size_t ws_ds_bytes = 0;
+    // growable scratch for the backward's partial dK, dV (fa::BackwardSplit)
+    void* ws_part = nullptr;
+    size_t ws_part_bytes = 0;
     int backward_ds_policy = -1;
     // dK/dV kernel of the backward: -1 / 1 the assembly kernel where it applies, 0 HIP only
     int backward_kernel_policy = -1;
@@ -592,6 +595,7 @@ int fa_ctx_destroy(fa_ctx* ctx) {
     if (ctx->ws) (void)hipFree(ctx->ws);
     if (ctx->ws_delta) (void)hipFree(ctx->ws_delta);
     if (ctx->ws_ds) (void)hipFree(ctx->ws_ds);
+    if (ctx->ws_part) (void)hipFree(ctx->ws_part);
     if (ctx->meta_dev) (void)hipFree(ctx->meta_dev);
     for (const auto& s : ctx->pending) {
         (void)hipEventDestroy(s.begin);
@@ -3125,9 +3129,17 @@ int fa_backward_grouped(fa_ctx* ctx, const void* q, const void* k, const void* v
         }
     }
     a.a64 = ctx->backward_kernel_policy != 0;
+    fa::BackwardSplit sp{};
+    if (dtype == FA_DTYPE_F32) sp = fa::backward_f32_split(a);
+    if (sp.bytes) {
+        void* part = nullptr;
+        if (int rc = grow(ctx, &ctx->ws_part, &ctx->ws_part_bytes, (size_t)sp.bytes, &part))
+            return rc;
+        sp.part = (float*)part;
+    }
     bool a64 = false;
     begin_span(ctx);
-    fa::launch_backward((Dtype)dtype, a, ctx->stream, &a64);
+    fa::launch_backward((Dtype)dtype, a, sp, ctx->stream, &a64);
     end_span(ctx, FA_KERNEL_BACKWARD_RECOMPUTE);
     HIP_TRY(hipGetLastError());
     const unsigned grid[3] = {(unsigned)(((sh->seq_len + 127) / 128) * sh->batch * sh->kv_heads),

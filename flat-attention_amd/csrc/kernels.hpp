@@ -160,9 +160,20 @@ struct BackwardArgs {
     // It reads `ld` as two f32 arrays of batch*q_heads*seq rows, -LSE / scale then -delta.
     int a64;
 };
+// How a dK/dV launch splits the query blocks that see a key block: `parts` chunks of `chunk` blocks
+// of 32 queries, each chunk's dK and dV in a workspace of `bytes` (`part`) when there are several.
+struct BackwardSplit {
+    float* part;
+    int parts, chunk;
+    uint64_t bytes;
+};
+// The f32 kernels (16-byte aligned rows: BackwardArgs::vec), after bwd_delta; two launches.
+BackwardSplit backward_f32_split(const BackwardArgs& a);
+void launch_backward_f32(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s);
 // Three launches: delta, dK/dV (which also writes dS when `ds` is set), dQ. *a64_out (if set)
 // tells whether the assembly dK/dV kernel ran.
-void launch_backward(Dtype dt, const BackwardArgs& a, hipStream_t s, bool* a64_out = nullptr);
+void launch_backward(Dtype dt, const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s,
+                     bool* a64_out = nullptr);
 
 // The assembly dK/dV kernel (gen_bwd_a64.py): bf16 or f16, head_dim 128, seq a multiple of 128, dS
 // stored, 16-byte aligned tensors, 32-bit offsets; its module loaded on the current device.

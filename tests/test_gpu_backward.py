@@ -121,6 +121,34 @@ def test_f32_tile_edges(hip, dims, causal):
                  (0, 1, 2, 3), 1, 5e-4, 2.5e-3)
 
 
+@pytest.mark.parametrize("dims", [
+    (1, 2, 1, 31, 20),     # one block of 31 rows; columns past the head dim
+    (1, 6, 2, 97, 33),     # head dim off the 16-byte chunk, groups of 3, chunks that end part-way
+    (2, 8, 2, 260, 64),    # nine key blocks, the last of 4 rows; partials added up
+    (1, 8, 8, 129, 100),   # MHA
+    (1, 4, 1, 200, 128),
+    (1, 2, 2, 1056, 32),   # 33 blocks of one wave's chunk
+    (8, 32, 32, 40, 128),  # 256 key blocks: the LDS-staged kernels without a mask
+    (16, 32, 32, 33, 96),  # 512: and with one
+])
+@pytest.mark.parametrize("causal", [True, False])
+def test_f32_backward_splits_match_oracle(hip, dims, causal):
+    """f32 dK/dV split into chunks of query blocks (partials in a workspace, added up in order) and
+    dQ over waves that take the key blocks in turn; bitwise repeatable."""
+    shape = fa.GroupedAttentionShape(*dims)
+    B, Hq, Hkv, S, D = dims
+    q, k, v, do = (normal(n, 171 + i) for i, n in enumerate(
+        (B * Hq * S * D, B * Hkv * S * D, B * Hkv * S * D, B * Hq * S * D)))
+    fwd, want = _expected(q, k, v, do, shape, causal, None)
+    pipe = fa.HipGroupedBackwardRecomputePipeline(hip, fa.DTYPE_F32)
+    got = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
+    again = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
+    for name, a, b_, e in zip(("dQ", "dK", "dV"), (got.dq, got.dk, got.dv),
+                              (again.dq, again.dk, again.dv), want):
+        assert_close(name, a, e, 2e-5 * max(1.0, float(np.abs(e).max())), 1e-4)
+        np.testing.assert_array_equal(a, b_, err_msg=name)
+
+
 @pytest.mark.parametrize("dtype", [fa.DTYPE_BF16, fa.DTYPE_F16])
 @pytest.mark.parametrize("dims,causal", [((1, 8, 2, 256, 128), True),
                                          ((2, 4, 4, 130, 64), False),
