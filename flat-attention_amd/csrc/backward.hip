@@ -18,6 +18,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -336,8 +337,11 @@ __global__ __launch_bounds__(256) void bwd_delta(BackwardArgs a, int64_t rows) {
 // One wave per SIMD (the K/V fragments and both accumulators take ~330 registers), so the
 // overlap has to come from this single instruction stream; scheduling group barriers keep the
 // compiler from separating the phases again.
+// Few key blocks (sp.parts > 1): the tiles of a key block are dealt to several workgroups in chunks
+// of sp.chunk; each writes its dK and dV, unscaled, to its slot of sp.part, and the dQ launch adds
+// them up in chunk order (add_partials).
 template <typename T, int DPAD, bool DMA, bool DSO = false>
-__global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a) {
+__global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit sp) {
     using B = Blk<T>;
     using F = typename B::Frag;
     constexpr int ES = B::ES, MB = DPAD / 32;
@@ -363,12 +367,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a) {
     const int nbk = a.batch * a.kv_heads;
     // key blocks in ascending order: under a causal mask the early blocks see the most queries,
     // so the heaviest workgroups dispatch first
-    const int kb = blockIdx.x / nbk, bkv = blockIdx.x % nbk;
+    const int bkv = blockIdx.x % nbk;
+    int kb, part;
+    sp.coords(blockIdx.x / nbk, (S + kBwdKeys - 1) / kBwdKeys, G, a.causal, kb, part);
     const int b = bkv / a.kv_heads, kvh = bkv - b * a.kv_heads;
     const int k0 = kb * kBwdKeys + wave * 32;
     const int64_t krow0 = (int64_t)bkv * S;
     const int qstart = a.causal ? kb * kBwdKeys : 0;  // a multiple of QT
-    const int nqt = (S - qstart + QT - 1) / QT, ntiles = G * nqt;
+    const int nqt = (S - qstart + QT - 1) / QT, all_tiles = G * nqt;
+    const int tile0 = part * sp.chunk, ntiles = min(all_tiles - tile0, sp.chunk) + tile0;
     const int64_t qhead0 = ((int64_t)b * a.q_heads + (int64_t)kvh * G) * S;  // first row of the group
     auto tile_hq = [&](int j) {  // head of the group and query offset qt of tile j
         const int hh = j / nqt;
@@ -486,11 +493,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a) {
     };
 
     if constexpr (DMA) {
-        dma_tile(0, 0);
+        dma_tile(tile0, (tile0 & 1) * STAGE);
         wait_dma();
         __syncthreads();
     }
-    for (int j = 0; j < ntiles; ++j) {
+    for (int j = tile0; j < ntiles; ++j) {
         int st = 0;
         if constexpr (DMA) {
             st = (j & 1) * STAGE;
@@ -641,6 +648,23 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a) {
         }
     }
     // register r: key k0 + 8 (r / 4) + 4 g + r % 4, dim 32 m + c
+    if (all_tiles > sp.chunk) {  // dK then dV, kBwdKeys rows of D each
+        const int nkb = (S + kBwdKeys - 1) / kBwdKeys;
+        float* const pp = sp.part + (((int64_t)bkv * nkb + kb) * sp.parts + part) * 2 * kBwdKeys * D;
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            const int d = 32 * m + c;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int at = (wave * 32 + 8 * (r >> 2) + 4 * g + (r & 3)) * D + d;
+                if (d < D) {
+                    pp[at] = dk[m][r];
+                    pp[kBwdKeys * D + at] = dv[m][r];
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
         const int d = 32 * m + c;
@@ -655,13 +679,48 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a) {
     }
 }
 
+// ------------------------------------------------------------------ partial dK, dV
+// dK and dV of kAddRows keys of one (batch * kv head, 128 keys): the partials in chunk order. The dQ
+// launches carry these workgroups after their own.
+constexpr int kAddRows = 16;
+template <typename T>
+__device__ __forceinline__ void add_partials(const BackwardArgs& a, const BackwardSplit& sp,
+                                             int block) {
+    using B = Blk<T>;
+    const int S = a.seq, D = a.head_dim, nkb = (S + kBwdKeys - 1) / kBwdKeys;
+    const int r0 = block % (kBwdKeys / kAddRows) * kAddRows, at = block / (kBwdKeys / kAddRows);
+    const int bkv = at / nkb, kb = at - bkv * nkb;
+    const int nqt = nkb - (a.causal ? kb : 0);
+    const int n = (a.group * nqt + sp.chunk - 1) / sp.chunk;
+    if (n <= 1) return;  // written by bwd_dkdv
+    const int64_t step = (int64_t)2 * kBwdKeys * D;
+    const float* pp = sp.part + (int64_t)at * sp.parts * step + r0 * D;
+    const int count = min(kAddRows, S - kb * kBwdKeys - r0) * D;  // (may be negative: no rows)
+    const int64_t out = ((int64_t)bkv * S + kb * kBwdKeys + r0) * D;
+    for (int e = threadIdx.x; e < count; e += blockDim.x) {
+        float k = pp[e], v = pp[kBwdKeys * D + e];
+#pragma unroll 4
+        for (int i = 1; i < n; ++i) {
+            k += pp[i * step + e];
+            v += pp[i * step + kBwdKeys * D + e];
+        }
+        B::store(a.dk, out + e, k * a.scale);
+        B::store(a.dv, out + e, v);
+    }
+}
+
 // ------------------------------------------------------------------ dQ
 // One workgroup: 128 queries of one (batch, query head), 32 per wave, Q and dO of them in
 // registers; tiles of 64 keys (K, V) of the KV head are swept, DMA double-buffered as above.
 // Two waves per SIMD (16-bit), so the phases of the two waves overlap.
 template <typename T, int DPAD, bool DMA>
-__global__ __launch_bounds__(256, Blk<T>::ES == 2 ? 2 : 1) void bwd_dq(BackwardArgs a) {
+__global__ __launch_bounds__(256, Blk<T>::ES == 2 ? 2 : 1) void bwd_dq(BackwardArgs a,
+                                                                      BackwardSplit sp, int n_dq) {
     using B = Blk<T>;
+    if ((int)blockIdx.x >= n_dq) {
+        add_partials<T>(a, sp, blockIdx.x - n_dq);
+        return;
+    }
     using F = typename B::Frag;
     constexpr int ES = B::ES, MB = DPAD / 32, KT = kBwdTile;
     using TG = TileGeom<T, DPAD, KT, ES == 2 && DPAD == 128>;
@@ -820,8 +879,12 @@ __global__ __launch_bounds__(256, Blk<T>::ES == 2 ? 2 : 1) void bwd_dq(BackwardA
 // bounded to it), never used.
 constexpr int kDqDsQueries = 256;
 template <typename T, int DPAD>
-__global__ __launch_bounds__(512, 2) void bwd_dq_ds(BackwardArgs a) {
+__global__ __launch_bounds__(512, 2) void bwd_dq_ds(BackwardArgs a, BackwardSplit sp, int n_dq) {
     using B = Blk<T>;
+    if ((int)blockIdx.x >= n_dq) {
+        add_partials<T>(a, sp, blockIdx.x - n_dq);
+        return;
+    }
     using H = typename B::H;
     static_assert(B::ES == 2, "16-bit storage only");
     constexpr int ES = 2, MB = DPAD / 32, KT = kBwdTile, NW = kDqDsQueries / 32;
@@ -973,29 +1036,31 @@ __global__ __launch_bounds__(512, 2) void bwd_dq_ds(BackwardArgs a) {
 }
 
 template <typename T, int DPAD, bool DMA>
-void launch_typed(const BackwardArgs& a, hipStream_t s) {
+void launch_typed(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
     const int S = a.seq;
     const int nkb = (S + kBwdKeys - 1) / kBwdKeys, nqb = (S + kBwdQueries - 1) / kBwdQueries;
+    const unsigned n_kv =
+        (unsigned)sp.workgroups(nkb, a.group, a.causal) * a.batch * a.kv_heads;
+    const unsigned n_add =
+        sp.parts > 1 ? (unsigned)nkb * a.batch * a.kv_heads * (kBwdKeys / kAddRows) : 0;
     if constexpr (DMA && Blk<T>::ES == 2) {
         if (a.ds) {
-            hipLaunchKernelGGL((bwd_dkdv<T, DPAD, true, true>), dim3(nkb * a.batch * a.kv_heads),
-                               dim3(256), 0, s, a);
-            const int nqd = (S + kDqDsQueries - 1) / kDqDsQueries;
-            hipLaunchKernelGGL((bwd_dq_ds<T, DPAD>), dim3(nqd * a.batch * a.q_heads), dim3(512),
-                               0, s, a);
+            hipLaunchKernelGGL((bwd_dkdv<T, DPAD, true, true>), dim3(n_kv), dim3(256), 0, s, a, sp);
+            const int n_dq = (S + kDqDsQueries - 1) / kDqDsQueries * a.batch * a.q_heads;
+            hipLaunchKernelGGL((bwd_dq_ds<T, DPAD>), dim3(n_dq + n_add), dim3(512), 0, s, a, sp,
+                               n_dq);
             return;
         }
     }
-    hipLaunchKernelGGL((bwd_dkdv<T, DPAD, DMA>), dim3(nkb * a.batch * a.kv_heads), dim3(256), 0,
-                       s, a);
-    hipLaunchKernelGGL((bwd_dq<T, DPAD, DMA>), dim3(nqb * a.batch * a.q_heads), dim3(256), 0, s,
-                       a);
+    hipLaunchKernelGGL((bwd_dkdv<T, DPAD, DMA>), dim3(n_kv), dim3(256), 0, s, a, sp);
+    const int n_dq = nqb * a.batch * a.q_heads;
+    hipLaunchKernelGGL((bwd_dq<T, DPAD, DMA>), dim3(n_dq + n_add), dim3(256), 0, s, a, sp, n_dq);
 }
 
 template <typename T, int DPAD>
-void launch_dma(const BackwardArgs& a, hipStream_t s) {
-    if (a.dma) launch_typed<T, DPAD, true>(a, s);
-    else launch_typed<T, DPAD, false>(a, s);
+void launch_dma(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
+    if (a.dma) launch_typed<T, DPAD, true>(a, sp, s);
+    else launch_typed<T, DPAD, false>(a, sp, s);
 }
 
 template <typename T>
@@ -1003,13 +1068,12 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
     const int64_t rows = (int64_t)a.batch * a.q_heads * a.seq;
     if constexpr (std::is_same_v<T, bf16_t> || std::is_same_v<T, f16_t>) {
         constexpr Dtype dt = std::is_same_v<T, bf16_t> ? Dtype::BF16 : Dtype::F16;
-        if (bwd_a64_eligible(dt, a)) {
+        if (sp.parts == 0) {
             hipLaunchKernelGGL((bwd_delta<T, true>), dim3((unsigned)((rows + 15) / 16)),
                                dim3(256), 0, s, a, rows);
             launch_bwd_a64(dt, a, s);
-            const int nqd = (a.seq + kDqDsQueries - 1) / kDqDsQueries;
-            hipLaunchKernelGGL((bwd_dq_ds<T, 128>), dim3(nqd * a.batch * a.q_heads), dim3(512),
-                               0, s, a);
+            const int n_dq = (a.seq + kDqDsQueries - 1) / kDqDsQueries * a.batch * a.q_heads;
+            hipLaunchKernelGGL((bwd_dq_ds<T, 128>), dim3(n_dq), dim3(512), 0, s, a, sp, n_dq);
             if (a64_out) *a64_out = true;
             return;
         }
@@ -1020,15 +1084,39 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
     if constexpr (std::is_same_v<T, float>) {
         // (no split: head dims above 64 only)
         if (sp.parts > 0) launch_backward_f32(a, sp, s);
-        else launch_dma<float, 128>(a, s);
-        return;
+        else launch_dma<float, 128>(a, BackwardSplit{nullptr, 1, INT32_MAX, 0}, s);
+    } else {
+        if (a.head_dim <= 32) launch_dma<T, 32>(a, sp, s);
+        else if (a.head_dim <= 64) launch_dma<T, 64>(a, sp, s);
+        else launch_dma<T, 128>(a, sp, s);
     }
-    if (a.head_dim <= 32) launch_dma<T, 32>(a, s);
-    else if (a.head_dim <= 64) launch_dma<T, 64>(a, s);
-    else launch_dma<T, 128>(a, s);
 }
 
 }  // namespace
+
+// parts = 0: the assembly kernel. Else tiles (128 queries of one head) per chunk so that the
+// chip's CUs, which hold one workgroup each, get about one round of equal chunks.
+// The assembly kernel takes 3 us a tile against 4.3 but one workgroup per 128 keys: the split wins
+// while those are at most half the CUs and chains are long (bf16 causal D 128, us for the backward,
+// assembly / split: Hq8 Hkv2 S512, 8 workgroups, 62.5 / 33.2; Hq32 Hkv8 B2 S512, 64, 67.1 / 48.7;
+// Hq16 Hkv4 S1024, 32, 111.5 / 51.0; Hq32 Hkv8 S2048, 128, 232.9 / 193.5). Under 512 tokens or
+// eight tiles to a key block it stays. Where the HIP kernel runs anyway (another head dim, a
+// length off 128), one round against one workgroup per 128 keys: Hq8 Hkv2 S512 D64 66.5 / 24.8,
+// Hq6 Hkv1 S1500 D128 332.5 / 57.2, Hq32 Hkv8 S2000 335.5 / 188.3, B2 S3000 618.2 / 550.6.
+BackwardSplit backward_split(Dtype dt, const BackwardArgs& a) {
+    if (dt == Dtype::F32) return backward_f32_split(a);
+    const int64_t nkb = (a.seq + kBwdKeys - 1) / kBwdKeys, nbk = (int64_t)a.batch * a.kv_heads;
+    const int64_t cus = device_cus();
+    BackwardSplit sp{};
+    if (bwd_a64_eligible(dt, a) &&
+        (a.a64 != kA64Auto || a.seq < 512 || a.group * nkb < 8 || nkb * nbk > cus / 2))
+        return sp;
+    const int64_t tiles = nbk * a.group * (a.causal ? nkb * (nkb + 1) / 2 : nkb * nkb);
+    sp.chunk = (int)std::min<int64_t>(std::max<int64_t>(1, (tiles + cus - 1) / cus), a.group * nkb);
+    sp.parts = (int)((a.group * nkb + sp.chunk - 1) / sp.chunk);
+    sp.bytes = sp.parts > 1 ? (uint64_t)nbk * nkb * sp.parts * 2 * kBwdKeys * a.head_dim * 4 : 0;
+    return sp;
+}
 
 void launch_backward(Dtype dt, const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s,
                      bool* a64_out) {

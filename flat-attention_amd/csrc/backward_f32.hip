@@ -103,11 +103,11 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int S = a.seq, D = a.head_dim, nq = (S + 31) / 32, nbk = a.batch * a.kv_heads;
     // early key blocks first: under a causal mask they see the most queries
-    const int bkv = blockIdx.x % nbk, rest = blockIdx.x / nbk;
-    const int part = rest % sp.parts, kb = rest / sp.parts;
+    const int bkv = blockIdx.x % nbk;
+    int kb, part;
+    sp.coords(blockIdx.x / nbk, nq, a.group, a.causal, kb, part);
     const int qb0 = a.causal ? kb : 0, nqv = nq - qb0, items = a.group * nqv;
     const int first = part * sp.chunk, last = min(items, first + sp.chunk);
-    if (first >= items) return;
     const int b = bkv / a.kv_heads, kvh = bkv - b * a.kv_heads;
     const int k0 = kb * 32;
     const int64_t krow0 = (int64_t)bkv * S;
@@ -326,7 +326,8 @@ __global__ __launch_bounds__(64 * NW, DPAD == 128 ? 1 : 2) void bwd_f32_dq(Backw
 template <int DPAD, int NW, bool FULL>
 void launch_v(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
     const int nb = (a.seq + 31) / 32, nbk = a.batch * a.kv_heads;
-    hipLaunchKernelGGL((bwd_f32_dkdv<DPAD, FULL>), dim3((unsigned)(nb * sp.parts * nbk)), dim3(256), 0,
+    hipLaunchKernelGGL((bwd_f32_dkdv<DPAD, FULL>),
+                       dim3((unsigned)(sp.workgroups(nb, a.group, a.causal) * nbk)), dim3(256), 0,
                        s, a, sp);
     const int n_dq = nb * a.batch * a.q_heads;
     const int n_add = sp.parts > 1 ? 2 * nb * nbk : 0;

@@ -3128,9 +3128,10 @@ int fa_backward_grouped(fa_ctx* ctx, const void* q, const void* k, const void* v
             a.ds_bytes = (int)bytes;
         }
     }
-    a.a64 = ctx->backward_kernel_policy != 0;
-    fa::BackwardSplit sp{};
-    if (dtype == FA_DTYPE_F32) sp = fa::backward_f32_split(a);
+    a.a64 = ctx->backward_kernel_policy == 0  ? fa::kA64Never
+            : ctx->backward_kernel_policy > 0 ? fa::kA64Always
+                                              : fa::kA64Auto;
+    fa::BackwardSplit sp = fa::backward_split((Dtype)dtype, a);
     if (sp.bytes) {
         void* part = nullptr;
         if (int rc = grow(ctx, &ctx->ws_part, &ctx->ws_part_bytes, (size_t)sp.bytes, &part))
@@ -3142,7 +3143,11 @@ int fa_backward_grouped(fa_ctx* ctx, const void* q, const void* k, const void* v
     fa::launch_backward((Dtype)dtype, a, sp, ctx->stream, &a64);
     end_span(ctx, FA_KERNEL_BACKWARD_RECOMPUTE);
     HIP_TRY(hipGetLastError());
-    const unsigned grid[3] = {(unsigned)(((sh->seq_len + 127) / 128) * sh->batch * sh->kv_heads),
+    const bool f32_split = dtype == FA_DTYPE_F32 && sp.parts > 0;
+    const int key_blocks = (int)((sh->seq_len + (f32_split ? 31 : 127)) / (f32_split ? 32 : 128));
+    const unsigned grid[3] = {(unsigned)(sp.parts > 0 ? sp.workgroups(key_blocks, a.group, a.causal)
+                                                      : key_blocks) *
+                                  (unsigned)(sh->batch * sh->kv_heads),
                               1, 1};
     char name[64];
     snprintf(name, sizeof name, "bwd_delta + %s + %s<%s>", a64 ? "bwd_dkdv_a64" : "bwd_dkdv",

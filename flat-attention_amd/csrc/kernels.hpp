@@ -156,18 +156,47 @@ struct BackwardArgs {
     int ds_nb, ds_bytes;
     int batch, q_heads, kv_heads, group, seq, head_dim, causal, vec, dma;
     float scale;
-    // Allow the assembly dK/dV kernel (fa_bwd_dkdv_a64_bf16 / _f16) where bwd_a64_eligible() holds.
+    // The assembly dK/dV kernel (fa_bwd_dkdv_a64_bf16 / _f16) where bwd_a64_eligible() holds: never,
+    // where it is the faster one, or always (kA64Never ...).
     // It reads `ld` as two f32 arrays of batch*q_heads*seq rows, -LSE / scale then -delta.
     int a64;
 };
 // How a dK/dV launch splits the query blocks that see a key block: `parts` chunks of `chunk` blocks
 // of 32 queries, each chunk's dK and dV in a workspace of `bytes` (`part`) when there are several.
+// (f32: blocks of 32 queries and 32 keys; 16-bit storage: tiles of 128 and 128.)
 struct BackwardSplit {
     float* part;
     int parts, chunk;
     uint64_t bytes;
+
+    // Key blocks (of nkb) that have a chunk `p`: G (nkb - kb) query blocks see key block kb under a
+    // causal mask.
+    __host__ __device__ int blocks(int p, int nkb, int group, bool causal) const {
+        return causal ? nkb - (int)((int64_t)p * chunk / group) : nkb;
+    }
+    // Workgroups of one (batch, kv head): last chunks first, so that whole chunks lead and the
+    // short ones (causal: the late key blocks, which have only a chunk 0) come last. No workgroup
+    // is without work: one would wait for a free CU like any other, and the dispatcher places them
+    // in order, shader engine by shader engine, so short and long ones in turn left half the
+    // engines idle (Hq32 Hkv8 B2 S3000 D128: 788 us for the backward, 618 unsplit).
+    __host__ __device__ int workgroups(int nkb, int group, bool causal) const {
+        int n = 0;
+        for (int p = 0; p < parts; ++p) n += blocks(p, nkb, group, causal);
+        return n;
+    }
+    __device__ void coords(int idx, int nkb, int group, bool causal, int& kb, int& part) const {
+        for (part = parts - 1; part > 0; --part) {
+            const int n = blocks(part, nkb, group, causal);
+            if (idx < n) break;
+            idx -= n;
+        }
+        kb = idx;
+    }
 };
-// The f32 kernels (16-byte aligned rows: BackwardArgs::vec), after bwd_delta; two launches.
+// The split of a backward under BackwardArgs::a64, `part` still to be set when bytes > 0. parts = 0:
+// the assembly dK/dV kernel (16-bit storage), the LDS-staged f32 kernels.
+BackwardSplit backward_split(Dtype dt, const BackwardArgs& a);
+// The f32 kernels without LDS staging, after bwd_delta; two launches.
 BackwardSplit backward_f32_split(const BackwardArgs& a);
 void launch_backward_f32(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s);
 // Three launches: delta, dK/dV (which also writes dS when `ds` is set), dQ. *a64_out (if set)

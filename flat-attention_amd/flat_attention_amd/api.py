@@ -289,8 +289,9 @@ class HipContext:
         check(lib().fa_ctx_set_backward_policy(self.handle, store_ds))
 
     def set_backward_kernel(self, assembly: int):
-        """-1 (default) and 1: the assembly dK/dV kernel fa_bwd_dkdv_a64_bf16 where it applies
-        (bf16, head_dim 128, seq_len a multiple of 128, dS stored); 0: the HIP kernel only."""
+        """1: the assembly dK/dV kernel fa_bwd_dkdv_a64_bf16 / _f16 where it applies (16-bit,
+        head_dim 128, seq_len a multiple of 128, dS stored); -1 (default): the same, except where
+        few key blocks make the split HIP kernel the faster one; 0: the HIP kernel only."""
         check(lib().fa_ctx_set_backward_kernel(self.handle, assembly))
 
     def set_prefill_precision(self, mode: int):

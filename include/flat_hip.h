@@ -603,9 +603,10 @@ int fa_ctx_set_decode_policy(fa_ctx* ctx, int32_t grouped);
 int fa_ctx_set_backward_policy(fa_ctx* ctx, int32_t store_ds);
 /* dK/dV kernel of the recompute backward (kernel-variant selection, the role of
  * WgpuKernelVariant src/wgpu_backend.rs:31-37 for the backward of src/wgpu_backward_grouped.rs:
- * 181-329): -1 (default) and 1 the assembly kernel fa_bwd_dkdv_a64_bf16 where it applies: bf16,
+ * 181-329): 1 the assembly kernel fa_bwd_dkdv_a64_bf16 / _f16 where it applies: 16-bit storage,
  * head_dim 128, seq_len a multiple of 128, dS stored (fa_ctx_set_backward_policy), 16-byte
- * aligned tensors; 0 the HIP kernel only. Both are within the same tolerance of the oracle (not
+ * aligned tensors; -1 (default) the same, except where few key blocks make the HIP kernel, split
+ * over query tiles, the faster one; 0 the HIP kernel only. Both are within the same tolerance of the oracle (not
  * bitwise equal: the assembly kernel adds -LSE / scale and -delta through the MFMA accumulator
  * inputs, a different f32 summation order); the telemetry's kernel name says which ran
  * (bwd_dkdv_a64). */

@@ -363,6 +363,37 @@ def test_stored_ds_path_matches_recompute_path(hip, request, dtype, dims, causal
         assert_close(name, a, e, 2e-2 * float(np.abs(e).max()), 2e-2)
 
 
+@pytest.mark.parametrize("dtype", [fa.DTYPE_BF16, fa.DTYPE_F16])
+@pytest.mark.parametrize("dims,causal,a64", [
+    ((1, 8, 2, 512, 128), True, False),   # where the assembly kernel would apply: 16 chunks
+    ((1, 8, 2, 512, 128), False, False),
+    ((1, 3, 1, 1000, 64), True, False),   # eight key blocks, the last of 104 rows; group of 3
+    ((2, 16, 8, 400, 40), False, False),  # head dim below the padded width
+    ((1, 48, 12, 1290, 32), True, False),  # chunks of several tiles, the last ones shorter
+    ((1, 2, 2, 512, 128), True, True),    # short chains: the assembly kernel stays
+])
+def test_split_key_blocks_match_oracle(hip, dtype, dims, causal, a64):
+    """dK/dV of few key blocks split over workgroups (partials in a workspace, added up by the dQ
+    launch); bitwise repeatable, also over a workspace that held another call's partials."""
+    rnd = bf16_round if dtype == fa.DTYPE_BF16 else f16_round
+    shape = fa.GroupedAttentionShape(*dims)
+    B, Hq, Hkv, S, D = dims
+    q, k, v, do = (rnd(normal(n, 91 + i)) for i, n in enumerate(
+        (B * Hq * S * D, B * Hkv * S * D, B * Hkv * S * D, B * Hq * S * D)))
+    fwd, _ = _expected(q, k, v, do, shape, causal, None)
+    fwd = fa.FlatAttentionOutput(rnd(fwd.output), fwd.lse)
+    want = oracle.backward_grouped(q, k, v, do, fwd.output, fwd.lse, B, Hq, Hkv, S, D, causal,
+                                   threads=8)
+    pipe = fa.HipGroupedBackwardRecomputePipeline(hip, dtype)
+    got = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
+    assert ("bwd_dkdv_a64" in hip.last_telemetry().kernel_name) == a64
+    again = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
+    for name, a, b_, e in zip(("dQ", "dK", "dV"), (got.dq, got.dk, got.dv),
+                              (again.dq, again.dk, again.dv), want):
+        assert_close(name, a, e, 2e-2 * float(np.abs(e).max()), 2e-2)
+        np.testing.assert_array_equal(a, b_, err_msg=name)
+
+
 def test_stored_ds_falls_back_to_recompute_past_2gib(hip):
     """The dS workspace is used only under 2 GiB: one causal head of 49,152 tokens needs
     2 nt (nt + 1) groups of 8 KiB with nt = 384 (2.42 GB), so the default policy takes the
