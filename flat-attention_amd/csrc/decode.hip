@@ -82,6 +82,14 @@ __device__ __forceinline__ void store8(void* dst, const float* x) {
     }
 }
 
+// Waves per SIMD of decode_splitk. f32 rows of 128 dims: two waves with two steps of K/V in flight
+// each (8 sequences of 100..2000 tokens, Hq16 Hkv4: 29.1 us; 36.7 with one wave and three steps).
+// At 64 dims one wave (8192 tokens, Hq16 Hkv4: 14.6 against 15.1 us; four such sequences 23.4 / 26.1).
+template <typename T, int DPAD, int GT>
+constexpr int splitk_waves() {
+    return std::is_same<T, float>::value && DPAD == 128 && GT <= 4 ? 2 : 1;
+}
+
 // One segment: keys [k0, k1) of sequence s for (kv head, head chunk of <= 16 heads); partial
 // slot `slot` (< 0: write O and LSE). GT: compile-time head-chunk width (>= group size of the
 // chunk, <= 16).
@@ -186,7 +194,7 @@ __device__ __forceinline__ void decode_item(const DecodeKArgs& ka, int s, int kv
     // 16-bit) of loads in flight. Loads never branch: keys past the split end are clamped to its
     // last live key (finite data whose scores are masked to -inf and whose V rows get
     // probability exactly 0).
-    constexpr int NS = 3;
+    constexpr int NS = splitk_waves<T, DPAD, GT>() == 2 ? 2 : 3;
     u32x4_t kbuf[NS][NQ];
     u32x4_t vbuf[NS][4][VCH];
     const int dv_ld = 8 * n < D ? 8 * n : 0;
@@ -639,7 +647,7 @@ __global__ __launch_bounds__(512) void decode_mfma_grouped(DecodeKArgs ka, int c
 // Persistent split kernel: one one-wave workgroup per resident wave, each running the segment
 // list the host built for it (equal key counts per wave), so no wave idles in a partial round.
 template <typename T, int DPAD, int GT>
-__global__ __launch_bounds__(64) void decode_splitk(DecodeKArgs ka, int n_items, int chunks) {
+__global__ __launch_bounds__(64, (splitk_waves<T, DPAD, GT>())) void decode_splitk(DecodeKArgs ka, int n_items, int chunks) {
     __shared__ __attribute__((aligned(16))) float p_lds[16 * 16];
     __shared__ __attribute__((aligned(16))) float misc_lds[3 * 16];
     (void)n_items;
