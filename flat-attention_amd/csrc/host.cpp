@@ -225,12 +225,18 @@ struct fa_ctx {
     std::vector<hipEvent_t> free_events;
     std::vector<Span> pending;
     // allocation-free decode: the device's static scratch (fa::noalloc_scratch, resolved when the
-    // context is created), a host staging area for its metadata and the event that marks the
-    // last copy out of that area
+    // context is created), a host staging area for its metadata in four parts that calls take in
+    // turn, and for each part the event after the kernel that last read it. (With one part a call
+    // waited for the previous call's copy, behind that call's predecessors on the stream.)
     void* na_scratch = nullptr;
     int32_t* na_host = nullptr;  // pinned, kNoAllocMetaBytes
-    hipEvent_t na_copied = nullptr;
-    bool na_pending = false;
+    struct NaSlot {
+        hipEvent_t copied = nullptr;
+        bool pending = false;
+    };
+    static constexpr int kNaSlots = 4;
+    NaSlot na_slot[kNaSlots];
+    int na_next = 0;
     struct Timed {
         double total_ms = 0.0, min_ms = 0.0, max_ms = 0.0;
         uint64_t launches = 0;
@@ -573,8 +579,11 @@ int fa_ctx_create(int device, fa_ctx** out) {
     // the telemetry's kernel name shows)
     (void)fa::prefill_a64_load(device);
     (void)fa::bwd_a64_load(device);
-    if (hipEventCreateWithFlags(&ctx->na_copied, hipEventDisableTiming) != hipSuccess)
-        ctx->na_copied = nullptr;
+    for (fa_ctx::NaSlot& slot : ctx->na_slot)
+        if (hipEventCreateWithFlags(&slot.copied, hipEventDisableTiming) != hipSuccess) {
+            slot.copied = nullptr;
+            break;  // (the last slot's event is there only if all are)
+        }
     if (hipHostMalloc((void**)&ctx->na_host, kNoAllocMetaBytes, hipHostMallocDefault) !=
         hipSuccess)
         ctx->na_host = nullptr;
@@ -602,7 +611,8 @@ int fa_ctx_destroy(fa_ctx* ctx) {
         (void)hipEventDestroy(s.end);
     }
     if (ctx->open_begin) (void)hipEventDestroy(ctx->open_begin);
-    if (ctx->na_copied) (void)hipEventDestroy(ctx->na_copied);
+    for (const fa_ctx::NaSlot& slot : ctx->na_slot)
+        if (slot.copied) (void)hipEventDestroy(slot.copied);
     if (ctx->na_host) (void)hipHostFree(ctx->na_host);
     for (hipEvent_t e : ctx->free_events) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(ctx->stream);
@@ -1962,6 +1972,16 @@ uint64_t max_split_tokens(uint64_t page_size) {
     return std::max<uint64_t>(16, t);
 }
 
+// Tokens per segment: an equal share of `total` for each of G resident workgroups, in whole 16-key
+// steps. Shares of one step are doubled once there are more than 256 of them: by then a head's
+// partials cost the combine more than a second step costs a wave (one sequence of 8192 bf16
+// tokens, Hq16 Hkv4 D64: 13.1 us at 16 tokens, 10.6 at 32; four of 40..600 tokens, Hq32 Hkv8
+// D128: 11.7 at 16, 16.8 at 32).
+uint64_t segment_tokens(uint64_t total, uint64_t G) {
+    const uint64_t L = std::max<uint64_t>(16, ((total + G - 1) / G + 15) / 16 * 16);
+    return L == 16 && total > 256 * 16 ? 32 : L;
+}
+
 // Work list of a decode plan. A unit is (kv head, chunk of <= 16 query heads); the key space
 // of every (sequence, unit) is laid end to end, each unit padded to a multiple of 16 keys, and
 // cut into segments:
@@ -1994,7 +2014,7 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
     if (p->grouped > 0) {
         uint64_t total = 0;
         for (int32_t c : p->ctx_lens) total += ((uint64_t)c + 15) / 16 * 16;
-        const uint64_t L = std::max<uint64_t>(16, ((total + G - 1) / G + 15) / 16 * 16);
+        const uint64_t L = segment_tokens(total, G);
         uint64_t pos = 0;
         int32_t slot = 0;
         for (uint64_t s = 0; s < p->n_seqs; ++s) {
@@ -2029,7 +2049,7 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
     uint64_t total = 0;
     for (int32_t c : p->ctx_lens) total += ((uint64_t)c + 15) / 16 * 16 * units;
     if (p->split_req == 0) {
-        const uint64_t L = std::max<uint64_t>(16, ((total + G - 1) / G + 15) / 16 * 16);
+        const uint64_t L = segment_tokens(total, G);
         uint64_t pos = 0;
         for (uint64_t s = 0; s < p->n_seqs; ++s) {
             const uint64_t c = (uint64_t)p->ctx_lens[s];
@@ -2391,7 +2411,8 @@ int enqueue_decode(fa_ctx* ctx, const fa_decode_plan* p, const float2* table, co
 }
 
 // The enqueue half of fa_paged_decode_noalloc, run while the device's scratch is held.
-int noalloc_enqueue(fa_ctx* ctx, uint8_t* base, const int32_t* h, uint64_t meta_ints,
+int noalloc_enqueue(fa_ctx* ctx, fa_ctx::NaSlot& slot, uint8_t* base, const int32_t* h,
+                    uint64_t meta_ints,
                     uint64_t n_bt, uint64_t n_seqs, uint64_t rope_bytes, uint64_t part_bytes,
                     float theta, uint64_t head_dim, fa_decode_plan* pp, const void* q,
                     const void* k_pool, const void* v_pool, void* out_lse,
@@ -2451,7 +2472,7 @@ int fa_paged_decode_noalloc(fa_ctx* ctx, const int32_t* block_tables, uint64_t m
     // replay would read whatever that area holds by then
     if (int rc = refuse_in_capture(ctx, "host upload")) return rc;
     if (int rc = set_device(ctx)) return rc;
-    if (!ctx->na_scratch || !ctx->na_copied || !ctx->na_host)
+    if (!ctx->na_scratch || !ctx->na_slot[fa_ctx::kNaSlots - 1].copied || !ctx->na_host)
         return fail(FA_ERR_HIP, "the static decode scratch of device %d is not addressable",
                     ctx->device);
 
@@ -2492,12 +2513,20 @@ int fa_paged_decode_noalloc(fa_ctx* ctx, const int32_t* block_tables, uint64_t m
                     "holds %llu",
                     (unsigned long long)(kNoAllocMetaBytes + rope_bytes + part_bytes),
                     (unsigned long long)fa::kNoAllocScratchBytes);
-    // the previous call's copy must have left the host staging area before it is rewritten
-    if (ctx->na_pending) {
-        HIP_TRY(hipEventSynchronize(ctx->na_copied));
-        ctx->na_pending = false;
-    }
-    int32_t* h = ctx->na_host;
+    // A call takes the next quarter of the host area, or all of it when a quarter is too small; the
+    // call that last used a quarter must have read it before it is rewritten.
+    constexpr size_t kSlotBytes = kNoAllocMetaBytes / fa_ctx::kNaSlots;
+    const bool whole = meta_ints * 4 > kSlotBytes;
+    const int at = whole ? 0 : ctx->na_next;
+    for (int i = at; i < (whole ? (int)fa_ctx::kNaSlots : at + 1); ++i)
+        if (ctx->na_slot[i].pending) {
+            HIP_TRY(hipEventSynchronize(ctx->na_slot[i].copied));
+            ctx->na_slot[i].pending = false;
+        }
+    // (after a call that took all of it the next one takes the first quarter, whose event it left)
+    ctx->na_next = whole ? 0 : (at + 1) % fa_ctx::kNaSlots;
+    fa_ctx::NaSlot& slot = ctx->na_slot[at];
+    int32_t* h = ctx->na_host + at * (kSlotBytes / 4);
     memcpy(h, block_tables, n_bt * 4);
     memcpy(h + n_bt, ctx_lens, n_seqs * 4);
     memcpy(h + n_bt + n_seqs, qpos.data(), n_seqs * 4);
@@ -2508,7 +2537,7 @@ int fa_paged_decode_noalloc(fa_ctx* ctx, const int32_t* block_tables, uint64_t m
     // user's kernels before overwriting it, and publish this call's completion afterwards.
     if (hipError_t e = fa::noalloc_order_begin(ctx->device, ctx->stream))
         return fail(FA_ERR_HIP, "ordering the shared decode scratch: %s", hipGetErrorString(e));
-    const int rc = noalloc_enqueue(ctx, base, h, meta_ints, n_bt, n_seqs, rope_bytes, part_bytes,
+    const int rc = noalloc_enqueue(ctx, slot, base, h, meta_ints, n_bt, n_seqs, rope_bytes, part_bytes,
                                    theta, head_dim, &p, q, k_pool, v_pool, out_lse, lay);
     const hipError_t e = fa::noalloc_order_end(ctx->device, ctx->stream, true);
     if (rc) return rc;
@@ -2520,19 +2549,16 @@ int fa_paged_decode_noalloc(fa_ctx* ctx, const int32_t* block_tables, uint64_t m
 }  // extern "C"
 
 namespace {
-int noalloc_enqueue(fa_ctx* ctx, uint8_t* base, const int32_t* h, uint64_t meta_ints,
+int noalloc_enqueue(fa_ctx* ctx, fa_ctx::NaSlot& slot, uint8_t* base, const int32_t* h,
+                    uint64_t meta_ints,
                     uint64_t n_bt, uint64_t n_seqs, uint64_t rope_bytes, uint64_t part_bytes,
                     float theta, uint64_t head_dim, fa_decode_plan* pp, const void* q,
                     const void* k_pool, const void* v_pool, void* out_lse,
                     const fa_packed_layout& lay) {
     fa_decode_plan& p = *pp;
-    HIP_TRY(hipMemcpyAsync(base, h, meta_ints * 4, hipMemcpyHostToDevice, ctx->stream));
-    HIP_TRY(hipEventRecord(ctx->na_copied, ctx->stream));
-    ctx->na_pending = true;
     int32_t* d = (int32_t*)base;
     p.d_bt = d;
     p.d_ctx = d + n_bt;
-    const int32_t* d_positions = p.d_ctx + n_seqs;
     p.d_qpos = p.d_ctx + 2 * n_seqs;
     p.d_work = p.d_ctx + 3 * n_seqs;
     float2* table = (float2*)(base + kNoAllocMetaBytes);
@@ -2541,10 +2567,12 @@ int noalloc_enqueue(fa_ctx* ctx, uint8_t* base, const int32_t* h, uint64_t meta_
     // Nothing in the scratch has to start at zero: every partial slot is written by its segment
     // before the combine reads it.
     begin_span(ctx);
-    fa::launch_rope_rows(table, rope_freqs(theta, head_dim), d_positions, (int)n_seqs,
-                         (int)(head_dim / 2), ctx->stream);
+    fa::launch_decode_setup(base, h, meta_ints * 4, table, rope_freqs(theta, head_dim),
+                            h + n_bt + n_seqs, (int)n_seqs, (int)(head_dim / 2), ctx->stream);
     end_span(ctx, FA_KERNEL_ROPE_TABLE);
     HIP_TRY(hipGetLastError());
+    HIP_TRY(hipEventRecord(slot.copied, ctx->stream));
+    slot.pending = true;
     if (int rc = enqueue_decode(ctx, &p, table, q, k_pool, v_pool, out_lse, lay)) return rc;
     return FA_OK;
 }

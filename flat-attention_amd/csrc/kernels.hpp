@@ -216,10 +216,11 @@ struct RopeFreqs {
     float inv_freq[64];
 };
 void launch_rope_table(float2* table, const RopeFreqs& f, int rows, int half, hipStream_t s);
-// (cos, sin) rows of n listed positions: table[i*half + p] for position positions[i], with the
-// same angle expression as launch_rope_table (bitwise equal rows).
-void launch_rope_rows(float2* table, const RopeFreqs& f, const int* positions, int n, int half,
-                      hipStream_t s);
+// `bytes` of pinned host memory to `dst` (both 16-byte aligned, whole 16-byte pieces are moved) and
+// the (cos, sin) rows of n positions listed in pinned host memory: table[i*half + p], with the same
+// angle expression as launch_rope_table (bitwise equal rows).
+void launch_decode_setup(void* dst, const void* host, size_t bytes, float2* table,
+                         const RopeFreqs& f, const int* positions, int n, int half, hipStream_t s);
 
 // Allocation-free paged decode: size of the per-device static scratch array and its device
 // address (resolved once per device with hipGetSymbolAddress; never the array's host-side name).

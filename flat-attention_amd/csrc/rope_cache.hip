@@ -27,21 +27,34 @@ void launch_rope_table(float2* table, const RopeFreqs& f, int rows, int half, hi
     rope_table_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(table, f, rows, half);
 }
 
-__global__ void rope_rows_kernel(float2* table, RopeFreqs f, const int* positions, int n,
-                                 int half) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)n * half) return;
-    const int r = (int)(i / half), p = (int)(i % half);
-    const float angle = (float)positions[r] * f.inv_freq[p];
-    float s, c;
-    sincosf(angle, &s, &c);
-    table[i] = make_float2(c, s);
+// The device state of an allocation-free decode in one launch: `quads` 16-byte pieces of the host's
+// metadata (pinned memory, read over the bus) to `dst`, and the (cos, sin) rows of the queries,
+// whose positions are read from the host's copy. A copy and the row kernel after it were two
+// dispatches of 4.6 and 2.0 us with a dependency between them.
+__global__ __launch_bounds__(256) void decode_setup_kernel(u32x4_t* dst, const u32x4_t* src,
+                                                           int quads, float2* table, RopeFreqs f,
+                                                           const int* positions, int n, int half,
+                                                           int rope_blocks) {
+    if ((int)blockIdx.x < rope_blocks) {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (i >= n * half) return;
+        const int r = i / half, p = i % half;
+        const float angle = (float)positions[r] * f.inv_freq[p];
+        float s, c;
+        sincosf(angle, &s, &c);
+        table[i] = make_float2(c, s);
+        return;
+    }
+    const int i = (blockIdx.x - rope_blocks) * 256 + threadIdx.x;
+    if (i < quads) dst[i] = src[i];
 }
 
-void launch_rope_rows(float2* table, const RopeFreqs& f, const int* positions, int n, int half,
-                      hipStream_t s) {
-    const int64_t m = (int64_t)n * half;
-    rope_rows_kernel<<<(unsigned)((m + 255) / 256), 256, 0, s>>>(table, f, positions, n, half);
+void launch_decode_setup(void* dst, const void* host, size_t bytes, float2* table,
+                         const RopeFreqs& f, const int* positions, int n, int half,
+                         hipStream_t s) {
+    const int quads = (int)((bytes + 15) / 16), rope_blocks = (n * half + 255) / 256;
+    decode_setup_kernel<<<(unsigned)(rope_blocks + (quads + 255) / 256), 256, 0, s>>>(
+        (u32x4_t*)dst, (const u32x4_t*)host, quads, table, f, positions, n, half, rope_blocks);
 }
 
 // Load / rotate / store 8 consecutive elements (4 pairs) of one head.

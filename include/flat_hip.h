@@ -380,9 +380,9 @@ int fa_paged_decode_plan_set_split(fa_ctx* ctx, fa_decode_plan* plan, uint64_t s
  * positions, work list, the queries' RoPE (cos, sin) rows and the split-K partials live in a
  * static per-device scratch array of 64 MiB (4 MiB of it for tables and work lists), which each
  * GPU holds until the process ends. A call needing more fails with FA_ERR_SCRATCH_EXCEEDED
- * before any device work. The metadata reaches the scratch by a stream-ordered copy from a
- * host area owned by the context; a call waits only until the previous call's copy has left
- * that area. Every call on one GPU shares that GPU's scratch; calls from different contexts
+ * before any device work. A kernel on the stream takes the metadata from a host area owned by
+ * the context, whose four quarters calls use in turn (a call that needs more takes all four); a
+ * call waits only until the call that last used its part has read it. Every call on one GPU shares that GPU's scratch; calls from different contexts
  * (streams) are ordered on the GPU: each call makes its stream wait for the event the previous
  * call on that GPU recorded after its kernels, and records its own (no host wait, no
  * allocation). Refused with FA_ERR_GRAPH_CAPTURE while the context's stream is captured (the

@@ -105,6 +105,37 @@ def test_noalloc_decode_rejects_oversized_metadata_before_device_work(hip):
     _assert_identical(a, b)
 
 
+def test_noalloc_decode_back_to_back_calls_reuse_the_host_area(hip):
+    """Calls issued without a host wait between them: more of them than the host area has parts,
+    and some (a block table of 64 x 4200 entries, over a quarter of it) that take all of it."""
+    cfg, ps, cases = fa.FlatAttentionConfig(True), 16, []
+    for i, (n, hq, hkv, D, wide) in enumerate([(3, 8, 2, 64, 0), (64, 4, 1, 64, 4200),
+                                               (2, 32, 8, 128, 0)]):
+        lens = np.random.default_rng(90 + i).integers(1, 400, n).tolist()
+        bt, kp, vp, total = _pool(np.random.default_rng(95 + i), lens, ps, hkv, D, bf16_round, 90 + i)
+        if wide:
+            bt = np.concatenate([bt, np.zeros((n, wide - bt.shape[1]), np.int32)], 1)
+        cl = np.asarray(lens, np.int32)
+        bufs = [fa.DeviceBuffer.from_array(hip, fa.host_storage(x, fa.DTYPE_BF16))
+                for x in (bf16_round(normal(n * hq * D, 99 + i)), kp, vp)]
+        plan = fa.PagedDecodePlan(hip, bt, cl, ps, total, hq, hkv, D, cfg, 1e4, fa.DTYPE_BF16)
+        lay = plan.layout()
+        ref = fa.DeviceBuffer(hip, lay.combined_bytes)
+        plan.launch(*bufs, ref)
+        cases.append((bt, cl, total, hq, hkv, D, bufs, lay, ref))
+    hip.synchronize()
+    order = [0, 0, 1, 2, 0, 2, 1, 1, 0, 2, 0, 2, 0, 1, 2]
+    outs = [fa.DeviceBuffer(hip, cases[c][7].combined_bytes) for c in order]
+    for c, out in zip(order, outs):
+        bt, cl, total, hq, hkv, D, bufs, lay, ref = cases[c]
+        fa.paged_decode_noalloc(hip, bt, cl, ps, total, hq, hkv, D, cfg, 1e4, fa.DTYPE_BF16,
+                                *bufs, out)
+    for c, out in zip(order, outs):
+        lay, ref = cases[c][7:]
+        _assert_identical(ref.download(np.uint8, lay.combined_bytes),
+                          out.download(np.uint8, lay.combined_bytes))
+
+
 def test_noalloc_decode_two_contexts_interleaved(hip):
     """Two contexts (two streams) on one GPU share the device's scratch. Calls issued back to
     back from both, with no host synchronisation between them, are ordered on the GPU by the
