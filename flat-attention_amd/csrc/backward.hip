@@ -19,6 +19,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -1094,15 +1095,17 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
 
 }  // namespace
 
-// parts = 0: the assembly kernel. Else tiles (128 queries of one head) per chunk so that the
-// chip's CUs, which hold one workgroup each, get about one round of equal chunks.
+// parts = 0: the assembly kernel. Else the number of chunks with the least estimated time, in tiles
+// (128 queries of one head) that a CU, which holds one workgroup, takes one after the other. A
+// workgroup costs about two tiles beside its own, one with partials up to five: its 256 D floats
+// are written and read again, and 256 of them keep the memory busy for 15 us, 3.5 tiles of 4.3 us.
 // The assembly kernel takes 3 us a tile against 4.3 but one workgroup per 128 keys: the split wins
 // while those are at most half the CUs and chains are long (bf16 causal D 128, us for the backward,
-// assembly / split: Hq8 Hkv2 S512, 8 workgroups, 62.5 / 33.2; Hq32 Hkv8 B2 S512, 64, 67.1 / 48.7;
-// Hq16 Hkv4 S1024, 32, 111.5 / 51.0; Hq32 Hkv8 S2048, 128, 232.9 / 193.5). Under 512 tokens or
+// assembly / split: Hq8 Hkv2 S512, 8 workgroups, 62.5 / 33.2; Hq32 Hkv8 B2 S512, 64, 67.1 / 52.2;
+// Hq16 Hkv4 S1024, 32, 111.5 / 51.0; Hq32 Hkv8 S2048, 128, 232.9 / 155.4). Under 512 tokens or
 // eight tiles to a key block it stays. Where the HIP kernel runs anyway (another head dim, a
 // length off 128), one round against one workgroup per 128 keys: Hq8 Hkv2 S512 D64 66.5 / 24.8,
-// Hq6 Hkv1 S1500 D128 332.5 / 57.2, Hq32 Hkv8 S2000 335.5 / 188.3, B2 S3000 618.2 / 550.6.
+// Hq6 Hkv1 S1500 D128 332.5 / 57.2, Hq32 Hkv8 S2000 335.5 / 152.7, B2 S3000 618.2 / 558.0.
 BackwardSplit backward_split(Dtype dt, const BackwardArgs& a) {
     if (dt == Dtype::F32) return backward_f32_split(a);
     const int64_t nkb = (a.seq + kBwdKeys - 1) / kBwdKeys, nbk = (int64_t)a.batch * a.kv_heads;
@@ -1111,9 +1114,29 @@ BackwardSplit backward_split(Dtype dt, const BackwardArgs& a) {
     if (bwd_a64_eligible(dt, a) &&
         (a.a64 != kA64Auto || a.seq < 512 || a.group * nkb < 8 || nkb * nbk > cus / 2))
         return sp;
-    const int64_t tiles = nbk * a.group * (a.causal ? nkb * (nkb + 1) / 2 : nkb * nkb);
-    sp.chunk = (int)std::min<int64_t>(std::max<int64_t>(1, (tiles + cus - 1) / cus), a.group * nkb);
-    sp.parts = (int)((a.group * nkb + sp.chunk - 1) / sp.chunk);
+    const int64_t longest = a.group * nkb;  // tiles of the key block with the most
+    const int64_t tiles = nbk * (a.causal ? longest * (nkb + 1) / 2 : longest * nkb);
+    double best = 0.0;
+    for (int64_t p = 0; p <= std::min<int64_t>(longest, 64); ++p) {
+        BackwardSplit t{};  // (p = 0: the even share of a causal launch)
+        t.chunk = (int)std::min(longest, p ? (longest + p - 1) / p : (tiles + cus - 1) / cus);
+        t.parts = (int)((longest + t.chunk - 1) / t.chunk);
+        const double n = (double)(nbk * t.workgroups((int)nkb, a.group, a.causal));
+        const double whole = t.parts == 1 ? n
+                             : a.causal   ? (double)(nbk * std::min<int64_t>(nkb, t.chunk / a.group))
+                                          : 0.0;
+        const double cost = t.parts == 1 ? 2.0 : 2.0 + 3.0 * std::min(1.0, (n - whole) / cus);
+        double est = t.chunk + cost;                             // one round,
+        if (n > cus && !a.causal) est *= std::ceil(n / cus);     // rounds of equal chunks,
+        else if (n > cus)                                        // or the short ones level the end
+            est = std::max(est, (tiles + 2.0 * whole + cost * (n - whole)) / cus +
+                                    t.chunk / (t.parts > 2 ? 2.0 : 8.0));
+        if (best == 0.0 || est < best) {
+            best = est;
+            sp.chunk = t.chunk;
+        }
+    }
+    sp.parts = (int)((longest + sp.chunk - 1) / sp.chunk);
     sp.bytes = sp.parts > 1 ? (uint64_t)nbk * nkb * sp.parts * 2 * kBwdKeys * a.head_dim * 4 : 0;
     return sp;
 }
