@@ -136,14 +136,24 @@ __device__ __forceinline__ void block_coords(const PrefillKArgs& ka, int bid, in
         qb = nqb - 1 - (logical - bh * nqb);
     }
     const int hi = (int)ka.inner.div((uint32_t)bh), lo = bh - hi * (int)ka.inner.d;
-    b = ka.a.var_meta ? lo : hi;
-    kvh = ka.a.var_meta ? hi : lo;
+    // (the high products ran on the VALU: back to scalar registers)
+    b = __builtin_amdgcn_readfirstlane(ka.a.var_meta ? lo : hi);
+    kvh = __builtin_amdgcn_readfirstlane(ka.a.var_meta ? hi : lo);
+    qb = __builtin_amdgcn_readfirstlane(qb);
 }
 
 // Running-max slack (log2 units) tolerated before O is rescaled: probabilities stay <= 2^8.
 constexpr float kRescaleLog2 = 8.0f;
 
 // ------------------------------------------------------------------ 16-bit MFMA kernel
+// A uniform load from memory that no kernel writes, through the scalar cache. Left to itself the
+// compiler takes a vector load where a store to unrelated memory (the padded rows) may come first,
+// and with it the buffer resource of every page went through vector registers: 8 chunks of 500
+// queries over 2000 cached tokens, Hq32 Hkv8 D128, 32-row pages, 165 us against 239.
+__device__ __forceinline__ int scalar_load(const int* p) {
+    return *(const __attribute__((address_space(4))) int*)(uintptr_t)p;
+}
+
 // K/V source addressing modes.
 enum : int { kContig = 0, kPaged16 = 1, kPagedAny = 2 };
 
@@ -271,9 +281,13 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         q_rope_off_ = m[3];
     }
     const int rows_total = q_len_ * a.group;
-    if (a.var_meta && r0 + BM > rows_total) {
-        write_padded_rows<uint16_t>(ka, b, kvh, max(r0, rows_total), min(r0 + BM, rows_pad), D);
-        if (r0 >= rows_total) return;
+    auto pad_rows = [&]() {
+        if (a.var_meta && r0 + BM > rows_total)
+            write_padded_rows<uint16_t>(ka, b, kvh, max(r0, rows_total), min(r0 + BM, rows_pad), D);
+    };
+    if (a.var_meta && r0 >= rows_total) {
+        pad_rows();
+        return;
     }
 
     // This lane's query row.
@@ -368,6 +382,20 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
     const uint32_t lane_off = (uint32_t)k_r * row_bytes + kd2;  // this thread's row/chunk
     constexpr int kRsrcFlags = 0x00020000;
     u32x4_t kreg[KPASS], vreg[KPASS];
+    // Key groups over pages: 64 entries of the block table, one a lane, reloaded when a tile reaches
+    // past them. (A scalar load of each tile's entries shares its counter with the LDS reads, and
+    // every tile's K and V waited for it.)
+    int bt_reg = 0, bt_first = 0, bt_end = 0;
+    auto ensure_pages = [&](int tile) {
+        const int first = (int)ka.ps.div((uint32_t)(tile * BN));
+        const int last = (int)ka.ps.div((uint32_t)min(tile * BN + BN - 1, kv_len_ - 1));
+        if (first < bt_first || last >= bt_end) {
+            const int pages = (int)ka.ps.div((uint32_t)(kv_len_ - 1)) + 1;
+            bt_reg = a.block_tables[(int64_t)b * a.bt_stride + min(first + lane, pages - 1)];
+            bt_first = first;
+            bt_end = first + 64;
+        }
+    };
     // One tile of K or V (base = kb8 or vb8) into `reg`.
     auto load_one = [&](int tile, const uint8_t* base, u32x4_t (&reg)[KPASS]) {
         const int key_base = tile * BN;
@@ -388,7 +416,11 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
                 const int live = min(16, kv_len_ - g16);
                 const int gq = live > 0 ? g16 : 0;
                 const uint32_t lp = ka.ps.div((uint32_t)gq);
-                const int page = a.block_tables[(int64_t)b * a.bt_stride + lp];
+                int page;  // (a group past kv_len reads nothing: any entry will do)
+                if constexpr (KW > 1)
+                    page = __builtin_amdgcn_readlane(bt_reg, ((int)lp - bt_first) & 63);
+                else
+                    page = scalar_load(a.block_tables + (int64_t)b * a.bt_stride + lp);
                 const int64_t gofs = ((int64_t)page * a.page_size + (gq - (int)lp * a.page_size)) *
                                      (int64_t)row_bytes;
                 const int nrec = live > 0 ? (live - 1) * (int)row_bytes + D * 2 : 0;
@@ -880,10 +912,12 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         // step before; two: stage i & 1 was last read in step i - 2.
         const int gbase = kg * NST * STAGE;
         const int n_steps = (n_tiles + KW - 1) / KW;
-        if (n_steps > 0) {
-            load_one(min(kg, n_tiles - 1), kb8, kreg);
-            load_v(min(kg, n_tiles - 1));
-        }
+        auto load_tile = [&](int tile) {
+            if constexpr (PMODE == kPaged16) ensure_pages(tile);
+            load_one(tile, kb8, kreg);
+            load_v(tile);
+        };
+        if (n_steps > 0) load_tile(min(kg, n_tiles - 1));
         for (int i = 0; i < n_steps; ++i) {
             const int tile = kg + KW * i;
             st_w = st_r = gbase + (NST == 2 ? (i & 1) * STAGE : 0);
@@ -893,8 +927,7 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
             store_v();
             __syncthreads();
             if (tile < n_tiles) {
-                load_one(min(tile + KW, n_tiles - 1), kb8, kreg);
-                load_v(min(tile + KW, n_tiles - 1));
+                load_tile(min(tile + KW, n_tiles - 1));
                 f32x16_t sacc[2];
                 u32x4_t pop[4];
                 compute_s(sacc, std::true_type{}, no_hook);
@@ -1002,6 +1035,7 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
                     (u32x4_t*)o);
             }
         }
+        pad_rows();
         return;
     }
 
@@ -1041,6 +1075,7 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         if (g == 0)
             a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = m_run * a.scale + logf(l_tot);
     }
+    pad_rows();
 }
 
 // ------------------------------------------------------------------ f32 MFMA kernel
@@ -1093,9 +1128,13 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
         q_rope_off_ = m[3];
     }
     const int rows_total = q_len_ * a.group;
-    if (a.var_meta && r0 + BM > rows_total) {
-        write_padded_rows<float>(ka, b, kvh, max(r0, rows_total), min(r0 + BM, rows_pad), D);
-        if (r0 >= rows_total) return;
+    auto pad_rows = [&]() {
+        if (a.var_meta && r0 + BM > rows_total)
+            write_padded_rows<float>(ka, b, kvh, max(r0, rows_total), min(r0 + BM, rows_pad), D);
+    };
+    if (a.var_meta && r0 >= rows_total) {
+        pad_rows();
+        return;
     }
     const int row = r0 + wave * 32 + (lane & 31);
     const bool row_ok = row < rows_total;
@@ -1347,6 +1386,7 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
         if (g == 0)
             a.lse[(int64_t)b * a.lse_sb + (int64_t)hq * a.lse_sh + t] = m_run * a.scale + logf(l_tot);
     }
+    pad_rows();
 }
 
 // ------------------------------------------------------------------ f32, key groups
@@ -1378,10 +1418,14 @@ __global__ __launch_bounds__(64 * NW, DPAD == 128 ? 1 : 2) void prefill_f32_grou
         q_rope_off_ = m[3];
     }
     const int rows_total = q_len_ * a.group;
-    if (a.var_meta && r0 + 32 > rows_total) {
-        write_padded_rows<float>(ka, b, kvh, max(r0, rows_total),
-                                 min(r0 + 32, a.q_len * a.group), D);
-        if (r0 >= rows_total) return;
+    auto pad_rows = [&]() {
+        if (a.var_meta && r0 + 32 > rows_total)
+            write_padded_rows<float>(ka, b, kvh, max(r0, rows_total),
+                                     min(r0 + 32, a.q_len * a.group), D);
+    };
+    if (a.var_meta && r0 >= rows_total) {
+        pad_rows();
+        return;
     }
     const int row = r0 + c;
     const bool row_ok = row < rows_total;
@@ -1548,6 +1592,7 @@ __global__ __launch_bounds__(64 * NW, DPAD == 128 ? 1 : 2) void prefill_f32_grou
                         (int64_t)t_r * a.o_ss + ch * 4) = o;
         }
     }
+    pad_rows();
 }
 
 // ------------------------------------------------------------------ launcher
@@ -1657,7 +1702,8 @@ static void launch32(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s)
 //     the ping-pong one (B2 H16 S2048 D128, 512 blocks, 52.5 / 44.5; B4 H16 S2048, 1024 blocks,
 //     74.9 / 88.9; D64 B4 H16 S1024, 512 blocks, 22.4 / 19.8), or four at D 32 (B4 H16 S2048, 39.7
 //     / 33.9). A padded batch has blocks without work: one round (six sequences up to 300 x 500,
-//     480 blocks, 29.9 / 31.9).
+//     480 blocks, 29.9 / 31.9); paged: one round too (4 chunks of 500
+//   queries over 2000 cached tokens, Hq32 Hkv8 D64, 512 blocks, 59.1 / 71.8).
 //   Under six key tiles the assembly kernel stays: its fixed cost is the smaller one (S128 12.8
 //   against 11.9, S300 level). Paged pools that it reads stay with it (one 16-query chunk over
 //   2048 cached tokens 54.6 / 67.5 / 60.7): the key groups wait for each tile's page ids.
@@ -1689,7 +1735,7 @@ int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a) {
     if (tiles < (a64 ? 6 : 2)) return 0;
     const int64_t cus = device_cus(), rows = (int64_t)a.q_len * a.group;
     const int64_t units = (int64_t)a.batch * a.kv_heads;
-    const int64_t rounds = a64 || a.var_meta ? 1 : a.head_dim <= 32 ? 4 : 2;
+    const int64_t rounds = a64 || a.var_meta || paged ? 1 : a.head_dim <= 32 ? 4 : 2;
     if (units * ((rows + 63) / 64) <= cus) return 4;
     if (units * ((rows + 127) / 128) <= rounds * cus) return 2;
     return 0;
