@@ -369,8 +369,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
     // key blocks in ascending order: under a causal mask the early blocks see the most queries,
     // so the heaviest workgroups dispatch first
     const int bkv = blockIdx.x % nbk;
+    const int slot = blockIdx.x / nbk;
     int kb, part;
-    sp.coords(blockIdx.x / nbk, (S + kBwdKeys - 1) / kBwdKeys, G, a.causal, kb, part);
+    sp.coords(slot, (S + kBwdKeys - 1) / kBwdKeys, G, a.causal, kb, part);
     const int b = bkv / a.kv_heads, kvh = bkv - b * a.kv_heads;
     const int k0 = kb * kBwdKeys + wave * 32;
     const int64_t krow0 = (int64_t)bkv * S;
@@ -650,8 +651,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
     }
     // register r: key k0 + 8 (r / 4) + 4 g + r % 4, dim 32 m + c
     if (all_tiles > sp.chunk) {  // dK then dV, kBwdKeys rows of D each
-        const int nkb = (S + kBwdKeys - 1) / kBwdKeys;
-        float* const pp = sp.part + (((int64_t)bkv * nkb + kb) * sp.parts + part) * 2 * kBwdKeys * D;
+        float* const pp = sp.part + ((int64_t)bkv * sp.slots + slot) * 2 * kBwdKeys * D;
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
             const int d = 32 * m + c;
@@ -695,15 +695,20 @@ __device__ __forceinline__ void add_partials(const BackwardArgs& a, const Backwa
     const int n = (a.group * nqt + sp.chunk - 1) / sp.chunk;
     if (n <= 1) return;  // written by bwd_dkdv
     const int64_t step = (int64_t)2 * kBwdKeys * D;
-    const float* pp = sp.part + (int64_t)at * sp.parts * step + r0 * D;
+    const float* const base = sp.part + (int64_t)bkv * sp.slots * step + r0 * D;
+    const BackwardSplit::Walk first(sp, kb, nkb, a.group, a.causal);
     const int count = min(kAddRows, S - kb * kBwdKeys - r0) * D;  // (may be negative: no rows)
     const int64_t out = ((int64_t)bkv * S + kb * kBwdKeys + r0) * D;
     for (int e = threadIdx.x; e < count; e += blockDim.x) {
+        BackwardSplit::Walk at_chunk = first;
+        const float* pp = base + at_chunk.slot * step;
         float k = pp[e], v = pp[kBwdKeys * D + e];
 #pragma unroll 4
         for (int i = 1; i < n; ++i) {
-            k += pp[i * step + e];
-            v += pp[i * step + kBwdKeys * D + e];
+            at_chunk.next();
+            pp = base + at_chunk.slot * step;
+            k += pp[e];
+            v += pp[kBwdKeys * D + e];
         }
         B::store(a.dk, out + e, k * a.scale);
         B::store(a.dv, out + e, v);
@@ -1085,7 +1090,7 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
     if constexpr (std::is_same_v<T, float>) {
         // (no split: head dims above 64 only)
         if (sp.parts > 0) launch_backward_f32(a, sp, s);
-        else launch_dma<float, 128>(a, BackwardSplit{nullptr, 1, INT32_MAX, 0}, s);
+        else launch_dma<float, 128>(a, BackwardSplit{nullptr, 1, INT32_MAX, 0, 0}, s);
     } else {
         if (a.head_dim <= 32) launch_dma<T, 32>(a, sp, s);
         else if (a.head_dim <= 64) launch_dma<T, 64>(a, sp, s);
@@ -1106,12 +1111,13 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
 // eight tiles to a key block it stays. Where the HIP kernel runs anyway (another head dim, a
 // length off 128), one round against one workgroup per 128 keys: Hq8 Hkv2 S512 D64 66.5 / 24.8,
 // Hq6 Hkv1 S1500 D128 332.5 / 57.2, Hq32 Hkv8 S2000 335.5 / 152.7, B2 S3000 618.2 / 558.0.
-BackwardSplit backward_split(Dtype dt, const BackwardArgs& a) {
-    if (dt == Dtype::F32) return backward_f32_split(a);
+BackwardSplit backward_split(Dtype dt, const BackwardArgs& a, uint64_t limit) {
+    if (dt == Dtype::F32) return backward_f32_split(a, limit);
     const int64_t nkb = (a.seq + kBwdKeys - 1) / kBwdKeys, nbk = (int64_t)a.batch * a.kv_heads;
     const int64_t cus = device_cus();
     BackwardSplit sp{};
-    if (bwd_a64_eligible(dt, a) &&
+    const bool a64 = bwd_a64_eligible(dt, a);
+    if (a64 &&
         (a.a64 != kA64Auto || a.seq < 512 || a.group * nkb < 8 || nkb * nbk > cus / 2))
         return sp;
     const int64_t longest = a.group * nkb;  // tiles of the key block with the most
@@ -1121,6 +1127,8 @@ BackwardSplit backward_split(Dtype dt, const BackwardArgs& a) {
         BackwardSplit t{};  // (p = 0: the even share of a causal launch)
         t.chunk = (int)std::min(longest, p ? (longest + p - 1) / p : (tiles + cus - 1) / cus);
         t.parts = (int)((longest + t.chunk - 1) / t.chunk);
+        t.set_workspace((int)nkb, a.group, a.causal, nbk, 2 * kBwdKeys * a.head_dim);
+        if (t.bytes > limit) continue;  // (one chunk takes none)
         const double n = (double)(nbk * t.workgroups((int)nkb, a.group, a.causal));
         const double whole = t.parts == 1 ? n
                              : a.causal   ? (double)(nbk * std::min<int64_t>(nkb, t.chunk / a.group))
@@ -1133,12 +1141,10 @@ BackwardSplit backward_split(Dtype dt, const BackwardArgs& a) {
                                     t.chunk / (t.parts > 2 ? 2.0 : 8.0));
         if (best == 0.0 || est < best) {
             best = est;
-            sp.chunk = t.chunk;
+            sp = t;
         }
     }
-    sp.parts = (int)((longest + sp.chunk - 1) / sp.chunk);
-    sp.bytes = sp.parts > 1 ? (uint64_t)nbk * nkb * sp.parts * 2 * kBwdKeys * a.head_dim * 4 : 0;
-    return sp;
+    return a64 && sp.parts == 1 ? BackwardSplit{} : sp;
 }
 
 void launch_backward(Dtype dt, const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s,

@@ -104,8 +104,9 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     const int S = a.seq, D = a.head_dim, nq = (S + 31) / 32, nbk = a.batch * a.kv_heads;
     // early key blocks first: under a causal mask they see the most queries
     const int bkv = blockIdx.x % nbk;
+    const int slot = blockIdx.x / nbk;
     int kb, part;
-    sp.coords(blockIdx.x / nbk, nq, a.group, a.causal, kb, part);
+    sp.coords(slot, nq, a.group, a.causal, kb, part);
     const int qb0 = a.causal ? kb : 0, nqv = nq - qb0, items = a.group * nqv;
     const int first = part * sp.chunk, last = min(items, first + sp.chunk);
     const int b = bkv / a.kv_heads, kvh = bkv - b * a.kv_heads;
@@ -201,8 +202,7 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     }
     // one chunk: the gradients themselves; else this chunk's partials (dK, then dV)
     const bool whole = items <= sp.chunk;
-    const int nkb = (S + 31) / 32;
-    float* const pp = sp.part + (((int64_t)bkv * nkb + kb) * sp.parts + part) * 64 * D;
+    float* const pp = sp.part + ((int64_t)bkv * sp.slots + slot) * 64 * D;
     reduce_waves<DPAD, 4>(lds, dk, D, [&](int r, int d, float x) {
         if (!whole) pp[r * D + d] = x;
         else if (k0 + r < S) ((float*)a.dk)[(krow0 + k0 + r) * D + d] = x * a.scale;
@@ -221,22 +221,32 @@ __device__ __forceinline__ void add_partials(const BackwardArgs& a, const Backwa
     const int items = a.group * (nkb - (a.causal ? kb : 0));
     const int n = (items + sp.chunk - 1) / sp.chunk;
     if (n <= 1) return;  // written by bwd_f32_dkdv
-    const float* pp = sp.part + (int64_t)at * sp.parts * 64 * D + which * 32 * D;
+    const int64_t step = (int64_t)64 * D;
+    const float* const base = sp.part + (int64_t)bkv * sp.slots * step + which * 32 * D;
+    const BackwardSplit::Walk first(sp, kb, nkb, a.group, a.causal);
     const float scale = which ? 1.0f : a.scale;
     float* out = (float*)(which ? a.dv : a.dk) + ((int64_t)bkv * S + kb * 32) * D;
     const int count = min(32, S - kb * 32) * D;
     if (a.vec) {
         for (int e = threadIdx.x * 4; e < count; e += blockDim.x * 4) {
-            f32x4_t s = *(const f32x4_t*)(pp + e);
+            BackwardSplit::Walk at_chunk = first;
+            f32x4_t s = *(const f32x4_t*)(base + at_chunk.slot * step + e);
 #pragma unroll 8
-            for (int i = 1; i < n; ++i) s += *(const f32x4_t*)(pp + (int64_t)i * 64 * D + e);
+            for (int i = 1; i < n; ++i) {
+                at_chunk.next();
+                s += *(const f32x4_t*)(base + at_chunk.slot * step + e);
+            }
             *(f32x4_t*)(out + e) = s * scale;
         }
     } else {
         for (int e = threadIdx.x; e < count; e += blockDim.x) {
-            float s = pp[e];
+            BackwardSplit::Walk at_chunk = first;
+            float s = base[at_chunk.slot * step + e];
 #pragma unroll 8
-            for (int i = 1; i < n; ++i) s += pp[(int64_t)i * 64 * D + e];
+            for (int i = 1; i < n; ++i) {
+                at_chunk.next();
+                s += base[at_chunk.slot * step + e];
+            }
             out[e] = s * scale;
         }
     }
@@ -352,7 +362,7 @@ void launch_d(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
 // D 128, two below), so a launch is one round of about equal workgroups and the partials of a
 // small problem stay a few MB (at most one chunk more than the round has workgroups, twice for
 // the causal taper).
-BackwardSplit backward_f32_split(const BackwardArgs& a) {
+BackwardSplit backward_f32_split(const BackwardArgs& a, uint64_t limit) {
     const int64_t nq = (a.seq + 31) / 32, nbk = (int64_t)a.batch * a.kv_heads;
     const int64_t blocks = a.causal ? nq * (nq + 1) / 2 : nq * nq;
     const int64_t waves = (int64_t)device_cus() * 4 * (a.head_dim > 64 ? 1 : 2);
@@ -360,9 +370,12 @@ BackwardSplit backward_f32_split(const BackwardArgs& a) {
     BackwardSplit sp{};
     if (a.head_dim > 64 && nbk * ((a.seq + 127) / 128) >= device_cus() * (a.causal ? 2 : 1)) return sp;
     sp.chunk = (int)std::min<int64_t>(4 * per_wave, a.group * nq);
-    sp.parts = (int)((a.group * nq + sp.chunk - 1) / sp.chunk);
-    sp.bytes = sp.parts > 1 ? (uint64_t)nbk * nq * sp.parts * 64 * a.head_dim * 4 : 0;
-    return sp;
+    for (;;) {
+        sp.parts = (int)((a.group * nq + sp.chunk - 1) / sp.chunk);
+        sp.set_workspace((int)nq, a.group, a.causal, nbk, 64 * a.head_dim);
+        if (sp.bytes <= limit) return sp;
+        sp.chunk = (int)(a.group * nq);  // one chunk: no partials
+    }
 }
 
 void launch_backward_f32(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {

@@ -3159,11 +3159,19 @@ int fa_backward_grouped(fa_ctx* ctx, const void* q, const void* k, const void* v
     a.a64 = ctx->backward_kernel_policy == 0  ? fa::kA64Never
             : ctx->backward_kernel_policy > 0 ? fa::kA64Always
                                               : fa::kA64Auto;
-    fa::BackwardSplit sp = fa::backward_split((Dtype)dtype, a);
+    fa::BackwardSplit sp = fa::backward_split((Dtype)dtype, a, fa::kBackwardPartialBytes);
     if (sp.bytes) {
+        // (a power of two: the buffers that growing retires take less than the one in use)
+        size_t bytes = (size_t)1 << 20;
+        while (bytes < sp.bytes) bytes *= 2;
         void* part = nullptr;
-        if (int rc = grow(ctx, &ctx->ws_part, &ctx->ws_part_bytes, (size_t)sp.bytes, &part))
-            return rc;
+        if (grow(ctx, &ctx->ws_part, &ctx->ws_part_bytes, bytes, &part) != FA_OK) {
+            // no memory, or the stream is captured: the best split that the workspace of earlier
+            // calls holds, without one none
+            (void)hipGetLastError();
+            sp = fa::backward_split((Dtype)dtype, a, ctx->ws_part_bytes);
+            part = ctx->ws_part;
+        }
         sp.part = (float*)part;
     }
     bool a64 = false;

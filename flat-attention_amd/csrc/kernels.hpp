@@ -167,37 +167,80 @@ struct BackwardArgs {
 struct BackwardSplit {
     float* part;
     int parts, chunk;
+    int slots;  // partials of one (batch, kv head): its workgroups whose key block has several chunks
     uint64_t bytes;
 
-    // Key blocks (of nkb) that have a chunk `p`: G (nkb - kb) query blocks see key block kb under a
-    // causal mask.
+    // Key blocks (of nkb) that have a chunk `p` < parts: G (nkb - kb) query blocks see key block kb
+    // under a causal mask. (p * chunk < G * nkb)
     __host__ __device__ int blocks(int p, int nkb, int group, bool causal) const {
-        return causal ? nkb - (int)((int64_t)p * chunk / group) : nkb;
+        return causal ? nkb - (int)((uint32_t)p * (uint32_t)chunk / (uint32_t)group) : nkb;
+    }
+    // Key blocks with several chunks; they are the first ones.
+    __host__ __device__ int split_blocks(int nkb, int group, bool causal) const {
+        return parts > 1 ? blocks(1, nkb, group, causal) : 0;
     }
     // Workgroups of one (batch, kv head): last chunks first, so that whole chunks lead and the
     // short ones (causal: the late key blocks, which have only a chunk 0) come last. No workgroup
     // is without work: one would wait for a free CU like any other, and the dispatcher places them
     // in order, shader engine by shader engine, so short and long ones in turn left half the
     // engines idle (Hq32 Hkv8 B2 S3000 D128: 788 us for the backward, 618 unsplit).
+    // The workgroups of key blocks with several chunks come before the others, so a workgroup's
+    // index is the slot of its partials too.
     __host__ __device__ int workgroups(int nkb, int group, bool causal) const {
         int n = 0;
         for (int p = 0; p < parts; ++p) n += blocks(p, nkb, group, causal);
         return n;
     }
-    __device__ void coords(int idx, int nkb, int group, bool causal, int& kb, int& part) const {
+    // (Chunks are walked with two divisions in all: a lone wave takes longer over one per chunk than
+    // over a tile's loads.)
+    __host__ __device__ void coords(int idx, int nkb, int group, bool causal, int& kb, int& part) const {
+        const uint32_t g = (uint32_t)group, whole = chunk / g, odd = chunk - whole * g;
+        const uint32_t last = (uint32_t)(parts - 1) * (uint32_t)chunk;
+        uint32_t hidden = last / g, rest = last - hidden * g;  // blocks(part) = nkb - hidden
         for (part = parts - 1; part > 0; --part) {
-            const int n = blocks(part, nkb, group, causal);
+            const int n = causal ? nkb - (int)hidden : nkb;
             if (idx < n) break;
             idx -= n;
+            hidden -= whole + (rest < odd);
+            rest += (rest < odd ? g : 0) - odd;
         }
         kb = idx;
     }
+    // The slots of key block kb's chunks, chunk 0 first: next() goes on to the next one.
+    struct Walk {
+        int slot, nkb;
+        uint32_t g, whole, odd, hidden = 0, rest = 0;
+        bool causal;
+        __host__ __device__ Walk(const BackwardSplit& sp, int kb, int nkb_, int group, bool causal_)
+            : nkb(nkb_), g((uint32_t)group), whole((uint32_t)sp.chunk / g),
+              odd((uint32_t)sp.chunk - whole * g), causal(causal_) {
+            slot = sp.slots - (causal ? nkb - (int)whole : nkb) + kb;
+        }
+        __host__ __device__ void next() {
+            rest += odd;
+            hidden += whole + (rest >= g);
+            if (rest >= g) rest -= g;
+            slot -= causal ? nkb - (int)hidden : nkb;
+        }
+    };
+    // Sets slots and bytes; a partial is dK and dV of a key block, `floats` together.
+    void set_workspace(int nkb, int group, bool causal, uint64_t units, uint64_t floats) {
+        slots = parts > 1 ? workgroups(nkb, group, causal) - nkb + split_blocks(nkb, group, causal)
+                          : 0;
+        bytes = units * slots * floats * 4;
+    }
 };
-// The split of a backward under BackwardArgs::a64, `part` still to be set when bytes > 0. parts = 0:
-// the assembly dK/dV kernel (16-bit storage), the LDS-staged f32 kernels.
-BackwardSplit backward_split(Dtype dt, const BackwardArgs& a);
+// Most memory that the partials of a backward take. One round of workgroups on 256 CUs needs 32 MiB
+// at D 128 and up to 4096 tokens no split that pays more than 200; longer sequences would go on
+// taking more for a few per cent of a launch whose key blocks fill the chip anyway (causal MQA of 64
+// heads, 131071 tokens: 3.6 GiB).
+constexpr uint64_t kBackwardPartialBytes = (uint64_t)256 << 20;
+// The split of a backward under BackwardArgs::a64 whose partials take at most `limit` bytes, `part`
+// still to be set when bytes > 0. parts = 0: the assembly dK/dV kernel (16-bit storage), the
+// LDS-staged f32 kernels.
+BackwardSplit backward_split(Dtype dt, const BackwardArgs& a, uint64_t limit);
 // The f32 kernels without LDS staging, after bwd_delta; two launches.
-BackwardSplit backward_f32_split(const BackwardArgs& a);
+BackwardSplit backward_f32_split(const BackwardArgs& a, uint64_t limit);
 void launch_backward_f32(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s);
 // Three launches: delta, dK/dV (which also writes dS when `ds` is set), dQ. *a64_out (if set)
 // tells whether the assembly dK/dV kernel ran.

@@ -115,6 +115,52 @@ def test_captured_backward_replays_match_eager(hip):
         assert all(np.isfinite(x).all() for x in (res.dq, res.dk, res.dv))
 
 
+@pytest.mark.parametrize("dtype,warm,shape", [
+    # the larger call runs without partials (the assembly kernel; one chunk), the captured one splits
+    (fa.DTYPE_BF16, (2, 32, 32, 512, 128), (1, 8, 2, 512, 128)),
+    (fa.DTYPE_BF16, (2, 32, 32, 600, 64), (1, 8, 2, 500, 64)),
+    (fa.DTYPE_F32, (2, 32, 32, 600, 64), (1, 8, 2, 500, 64))])
+def test_captured_backward_needs_no_partials_workspace(dtype, warm, shape):
+    """A backward split over workgroups whose partials have no memory yet (it cannot be allocated
+    during a capture; the same when the device has none left) runs unsplit, as the workspaces of
+    an earlier, larger call allow, and agrees with the split one that an eager call runs."""
+    ctx = fa.HipContext(0)
+    try:
+        cfg = fa.FlatAttentionConfig(True)
+        pipe = fa.HipGroupedBackwardRecomputePipeline(ctx, dtype)
+        rnd = bf16_round if dtype == fa.DTYPE_BF16 else (lambda x: x)
+
+        def tensors(dims, seed):
+            sh = fa.GroupedAttentionShape(*dims)
+            B, hq, hkv, S, D = dims
+            q, k, v, do = (rnd(normal(n, seed + i)) for i, n in enumerate(
+                (B * hq * S * D, B * hkv * S * D, B * hkv * S * D, B * hq * S * D)))
+            fwd = fa.HipRotaryGroupedAttention(ctx, dtype).forward(q, k, v, sh, cfg, None)
+            o = fa.storage_to_f32(fwd.output, dtype)
+            packed = fa.pack_grouped_backward_recompute_inputs(
+                q, k, v, do, fa.FlatAttentionOutput(o, fwd.lse), sh, dtype, pipe.layout(sh))
+            return sh, fa.DeviceBuffer.from_array(ctx, packed)
+
+        big, fbig = tensors(warm, 61)
+        pipe.encode(fbig, pipe.create_gradient_buffer(big), big, cfg)
+        small, fsmall = tensors(shape, 71)
+        g_graph, g_eager = (pipe.create_gradient_buffer(small) for _ in range(2))
+        prep = pipe.prepare(fsmall, g_graph, small, cfg)
+        with ctx.capture() as cap:
+            pipe.encode_prepared(prep)
+        one = ctx.last_telemetry().workgroups[0]
+        for rep in range(3):
+            cap.graph.launch()
+            pipe.encode(fsmall, g_eager, small, cfg)
+            assert ctx.last_telemetry().workgroups[0] > one
+            got, want = pipe.download_gradients(g_graph, small), pipe.download_gradients(g_eager, small)
+            for a, e in zip((got.dq, got.dk, got.dv), (want.dq, want.dk, want.dv)):
+                bound = 1e-5 if dtype == fa.DTYPE_F32 else 2e-2
+                assert np.isfinite(a).all() and float(np.abs(a - e).max()) <= bound * float(np.abs(e).max())
+    finally:
+        ctx.close()
+
+
 def test_capture_refuses_allocation_upload_fill_and_wait(hip):
     fresh = fa.HipContext(0)
     try:
