@@ -1044,8 +1044,10 @@ void describe_prefill(const fa_ctx* ctx, const PrefillJob& j, const fa::PrefillA
         fb = "K pre-rotation pass needs head_dim % 8 == 0; K rotated on load";
     const char* dt = j.dtype == FA_DTYPE_BF16 ? "bf16" : j.dtype == FA_DTYPE_F16 ? "f16" : "f32";
     const bool a64 = fa::prefill_uses_a64(j.dt, j.paged, a);
-    const char* base =
-        j.dtype == FA_DTYPE_F32 ? "prefill_mfma_f32" : (a64 ? "prefill_a64" : "prefill_mfma16");
+    const bool groups32 = fa::prefill_uses_f32_groups(j.dt, j.paged, a);  // (32-key tiles)
+    const char* base = j.dtype == FA_DTYPE_F32 ? (groups32 ? "prefill_f32_groups" : "prefill_mfma_f32")
+                       : a64                   ? "prefill_a64"
+                                               : "prefill_mfma16";
     char name[64];
     if (prerot && a.k_lo && a64)
         snprintf(name, sizeof name, "rotate_rows + %s<%s> (split Q/K scores)", base, dt);
@@ -1059,8 +1061,8 @@ void describe_prefill(const fa_ctx* ctx, const PrefillJob& j, const fa::PrefillA
         snprintf(name, sizeof name, "%s<%s> (K rotated on load)", base, dt);
     else
         snprintf(name, sizeof name, "%s<%s>", base, dt);
-    fill_telemetry(*out, ctx, kid, name, rows, 64, grid, block, dispatches, 1, fb, allocs,
-                   alloc_bytes);
+    fill_telemetry(*out, ctx, kid, name, rows, groups32 ? 32 : 64, grid, block, dispatches, 1, fb,
+                   allocs, alloc_bytes);
 }
 
 // Enqueues the resolved prefill on the context's stream: the optional K pre-rotation pass, then
@@ -3186,6 +3188,14 @@ int fa_backward_grouped(fa_ctx* ctx, const void* q, const void* k, const void* v
                                   (unsigned)(sh->batch * sh->kv_heads),
                               1, 1};
     char name[64];
+    if (f32_split) {  // 32 x 32 blocks; only the partials of dK and dV are moved otherwise
+        snprintf(name, sizeof name, "bwd_delta + bwd_f32_dkdv + bwd_f32_dq<f32>");
+        record(ctx, FA_KERNEL_BACKWARD_RECOMPUTE, name, 32, 32, grid, 256, 3, 1,
+               vec || sp.parts == 1 ? nullptr
+                                    : "unaligned tensors or head_dim off the 16-byte chunk: "
+                                      "partial sums added one value at a time");
+        return ok();
+    }
     snprintf(name, sizeof name, "bwd_delta + %s + %s<%s>", a64 ? "bwd_dkdv_a64" : "bwd_dkdv",
              a.ds ? "bwd_dq_ds" : "bwd_dq", dtype_name(dtype));
     record(ctx, FA_KERNEL_BACKWARD_RECOMPUTE, name, 128, 64, grid, 256, 3, 1,

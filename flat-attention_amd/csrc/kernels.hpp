@@ -78,8 +78,9 @@ unsigned prefill_a64_workgroups(const PrefillArgs& a);
 // Key groups of the 16-bit launch of `a`: 2 or 4 where the row blocks alone would leave most of
 // the chip idle (prefill_mfma16's KW), 0 otherwise.
 int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a);
-// Whether launch_prefill runs the assembly kernel on `a`.
+// Whether launch_prefill runs the assembly kernel, or prefill_f32_groups, on `a`.
 bool prefill_uses_a64(Dtype dt, bool paged, const PrefillArgs& a);
+bool prefill_uses_f32_groups(Dtype dt, bool paged, const PrefillArgs& a);
 void launch_prefill(Dtype dt, bool paged, const PrefillArgs& a, hipStream_t s,
                     unsigned grid[3], unsigned* block);
 // The grid, workgroup size and query rows per workgroup launch_prefill uses for `a` (host only).

@@ -1759,8 +1759,8 @@ static bool f32_rows_ok(const PrefillArgs& a) {
 // causal, 256 blocks, 91.4 / 66.8; at 512 blocks H16 B2 S2048 D128 397.7 / 340.8, but Hq32 Hkv8
 // B2 S1000 D64 121.8 / 129.6; at 1024 blocks B4 H16 S2048 D128 628.8 / 691.2, where the tiles
 // that four waves share in LDS count for more.
-static bool prefill_f32_grouped(bool paged, const PrefillArgs& a) {
-    if (paged || !f32_rows_ok(a) || (uintptr_t)a.q % 16 || a.q_ss % 4 || a.q_sh % 4 || a.q_sb % 4 ||
+bool prefill_uses_f32_groups(Dtype dt, bool paged, const PrefillArgs& a) {
+    if (dt != Dtype::F32 || paged || !f32_rows_ok(a) || (uintptr_t)a.q % 16 || a.q_ss % 4 || a.q_sh % 4 || a.q_sb % 4 ||
         (uintptr_t)a.o % 16 || a.o_ss % 4 || a.o_sh % 4 || a.o_sb % 4)
         return false;
     const int64_t blocks = (int64_t)a.batch * a.kv_heads *
@@ -1786,7 +1786,7 @@ void prefill_geometry(Dtype dt, bool paged, const PrefillArgs& a, unsigned grid[
         *rows = 256;
         return;
     }
-    if (dt == Dtype::F32 && prefill_f32_grouped(paged, a)) {
+    if (prefill_uses_f32_groups(dt, paged, a)) {
         grid[0] = (unsigned)((int64_t)a.batch * a.kv_heads *
                              (((int64_t)a.q_len * a.group + 31) / 32));
         grid[1] = grid[2] = 1;
@@ -1824,7 +1824,7 @@ void launch_prefill(Dtype dt, bool paged, const PrefillArgs& a, hipStream_t s, u
         case Dtype::F16: launch16<f16_t>(ka, paged, dpad, g, s); break;
         default:
             if (paged) launch32<true>(ka, dpad, g, s);
-            else if (prefill_f32_grouped(paged, a)) launch32g(ka, dpad, g, s);
+            else if (prefill_uses_f32_groups(dt, paged, a)) launch32g(ka, dpad, g, s);
             // transfers (register staging uses 64-bit addresses)
             else if (f32_rows_ok(a)) launch32<false, true>(ka, dpad, g, s);
             else launch32<false>(ka, dpad, g, s);

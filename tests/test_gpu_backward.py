@@ -142,6 +142,14 @@ def test_f32_backward_splits_match_oracle(hip, dims, causal):
     fwd, want = _expected(q, k, v, do, shape, causal, None)
     pipe = fa.HipGroupedBackwardRecomputePipeline(hip, fa.DTYPE_F32)
     got = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
+    t = hip.last_telemetry()
+    staged = D > 64 and B * Hkv * ((S + 127) // 128) >= (512 if causal else 256)
+    if staged:
+        assert "bwd_dkdv + bwd_dq<f32>" in t.kernel_name
+        assert (t.query_rows, t.kv_rows) == (128, 64)
+    else:
+        assert "bwd_f32_dkdv + bwd_f32_dq<f32>" in t.kernel_name, t.kernel_name
+        assert (t.query_rows, t.kv_rows) == (32, 32)
     again = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
     for name, a, b_, e in zip(("dQ", "dK", "dV"), (got.dq, got.dk, got.dv),
                               (again.dq, again.dk, again.dv), want):
@@ -278,8 +286,9 @@ def test_16bit_partial_head_dims(hip, dtype, dims, causal):
 @pytest.mark.parametrize("dtype", [fa.DTYPE_BF16, fa.DTYPE_F32])
 def test_unaligned_tensors_take_the_staged_path(hip, dtype):
     """Tensors at 2-byte (16-bit) / 4-byte (f32) offsets: no 16-byte loads or buffer->LDS
-    transfers are possible, the kernels stage through registers (telemetry names the reason);
-    results equal the aligned call's bit for bit."""
+    transfers are possible, the 16-bit kernels stage through registers; the f32 ones, whose buffer
+    loads need 4-byte alignment only, add up partial sums one value at a time (telemetry names the
+    reason); results equal the aligned call's bit for bit."""
     B, Hq, Hkv, S, D = 1, 4, 2, 130, 64
     rnd = bf16_round if dtype == fa.DTYPE_BF16 else (lambda x: x)
     q, k, v, do = (rnd(normal(n, 61 + i)) for i, n in enumerate(
@@ -314,6 +323,7 @@ def test_unaligned_tensors_take_the_staged_path(hip, dtype):
     aligned, t0 = run(0)
     shifted, t1 = run(eb)
     assert t0.fallback_reason is None and t1.fallback_reason is not None
+    assert ("partial sums" in t1.fallback_reason) == (dtype == fa.DTYPE_F32)
     for a, b_ in zip(aligned, shifted):
         np.testing.assert_array_equal(a, b_)
     want = oracle.backward_grouped(q, k, v, do, o, fwd.lse, B, Hq, Hkv, S, D, True)

@@ -171,7 +171,10 @@ def test_f32_key_group_prefill_matches_oracle(hip, B, hq, hkv, S, D, rope, rows,
     shape = fa.GroupedAttentionShape(B, hq, hkv, S, D)
     rot = fa.RotaryEmbeddingConfig(1e4, 3) if rope and D % 8 == 0 else None
     o, l = _run_grouped(hip, q, k, v, shape, fa.FlatAttentionConfig(causal), rot, fa.DTYPE_F32)
-    assert hip.last_telemetry().query_rows == rows
+    t = hip.last_telemetry()
+    assert t.query_rows == rows
+    kernel, kv_rows = ("prefill_f32_groups", 32) if rows == 32 else ("prefill_mfma_f32", 64)
+    assert kernel in t.kernel_name and t.kv_rows == kv_rows, t.kernel_name
     eo, el = _oracle_grouped(q, k, v, shape, causal, rot)
     assert_close("O", o, eo, F32_ATOL, F32_RTOL)
     assert_close("LSE", l, el, F32_ATOL, F32_RTOL)
