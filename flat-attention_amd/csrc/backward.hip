@@ -1090,7 +1090,12 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
     if constexpr (std::is_same_v<T, float>) {
         // (no split: head dims above 64 only)
         if (sp.parts > 0) launch_backward_f32(a, sp, s);
-        else launch_dma<float, 128>(a, BackwardSplit{nullptr, 1, INT32_MAX, 0, 0}, s);
+        else {
+            BackwardSplit one{};
+            one.parts = 1;
+            one.chunk = INT32_MAX;
+            launch_dma<float, 128>(a, one, s);
+        }
     } else {
         if (a.head_dim <= 32) launch_dma<T, 32>(a, sp, s);
         else if (a.head_dim <= 64) launch_dma<T, 64>(a, sp, s);
@@ -1100,10 +1105,55 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
 
 }  // namespace
 
-// parts = 0: the assembly kernel. Else the number of chunks with the least estimated time, in tiles
-// (128 queries of one head) that a CU, which holds one workgroup, takes one after the other. A
-// workgroup costs about two tiles beside its own, one with partials up to five: its 256 D floats
-// are written and read again, and 256 of them keep the memory busy for 15 us, 3.5 tiles of 4.3 us.
+// Time, in tiles (128 queries of one head), of a split dK/dV launch: its workgroups in dispatch order,
+// each on the first of the CUs, which hold one workgroup, that is free. A workgroup costs two tiles
+// beside its own, one with partials four: 256 D floats are written and read again.
+static int64_t split_time(const BackwardSplit& sp, int nkb, const BackwardArgs& a, int64_t units,
+                          int64_t cus) {
+    constexpr int kSteps = 512;  // steps of time, of `unit` tiles
+    uint32_t free_at[kSteps] = {};
+    const int64_t longest = (int64_t)a.group * nkb;
+    const int64_t tiles = units * (a.causal ? longest * (nkb + 1) / 2 : longest * nkb);
+    const int64_t n = units * (nkb + sp.slots);  // (or a few more)
+    const int64_t unit = 1 + (tiles + 4 * n) / (cus * (kSteps / 4)) + (sp.chunk + 4) / (kSteps / 4);
+    free_at[0] = (uint32_t)cus;
+    int64_t now = 0, end = 0;
+    auto place = [&](int64_t count, int64_t time) {
+        const int64_t d = (time + unit - 1) / unit;
+        while (count > 0) {
+            while (free_at[now] == 0) ++now;
+            const int64_t k = std::min<int64_t>(count, free_at[now]);
+            const int64_t at = std::min<int64_t>(now + d, kSteps - 1);
+            if (at == now) return;  // (the last step: never reached under the unit above)
+            free_at[now] -= (uint32_t)k;
+            free_at[at] += (uint32_t)k;
+            end = std::max(end, at);
+            count -= k;
+        }
+    };
+    for (int p = sp.parts - 1; p >= 0; --p) {
+        const int64_t before = (int64_t)p * sp.chunk;
+        const int blocks = sp.blocks(p, nkb, a.group, a.causal);
+        // key blocks with a whole chunk p and something behind it, or before it: one time
+        int kb = !a.causal ? blocks : (int)std::max<int64_t>(0, nkb - (before + sp.chunk) / a.group);
+        kb = std::min(kb, blocks);
+        if (kb > 0)
+            place(units * kb, std::min<int64_t>(sp.chunk, longest - before) + (sp.parts > 1 ? 4 : 2));
+        for (; kb < blocks; ++kb) {  // (causal: the last blocks that have this chunk)
+            const int64_t all = (int64_t)a.group * (nkb - kb);
+            place(units, std::min<int64_t>(sp.chunk, all - before) + (all > sp.chunk ? 4 : 2));
+        }
+    }
+    return end * unit;
+}
+
+// parts = 0: the assembly kernel. Else the number of chunks with the least time: one, two, an even
+// share of the tiles for each CU, or a number next to one, two or three full rounds of workgroups.
+// Measured against 1 to 36 chunks at 25 shapes (Hq6 Hkv1 to B2 Hq32 Hkv8, S 512 to 4000, with and
+// without a mask) the choice took at most 1 % longer than the best of them; so did none of the
+// choices with three tiles for partials, and with five one 4 %. (us for the backward, bf16 causal D
+// 128, one chunk / chosen / twice as many: Hq16 Hkv4 S1000 166 / 51 / 61; Hq32 Hkv8 B2 S1000 177 /
+// 102 / 118; Hq16 Hkv4 S4000 623 / 286 / 320.)
 // The assembly kernel takes 3 us a tile against 4.3 but one workgroup per 128 keys: the split wins
 // while those are at most half the CUs and chains are long (bf16 causal D 128, us for the backward,
 // assembly / split: Hq8 Hkv2 S512, 8 workgroups, 62.5 / 33.2; Hq32 Hkv8 B2 S512, 64, 67.1 / 52.2;
@@ -1115,36 +1165,48 @@ BackwardSplit backward_split(Dtype dt, const BackwardArgs& a, uint64_t limit) {
     if (dt == Dtype::F32) return backward_f32_split(a, limit);
     const int64_t nkb = (a.seq + kBwdKeys - 1) / kBwdKeys, nbk = (int64_t)a.batch * a.kv_heads;
     const int64_t cus = device_cus();
-    BackwardSplit sp{};
     const bool a64 = bwd_a64_eligible(dt, a);
     if (a64 &&
         (a.a64 != kA64Auto || a.seq < 512 || a.group * nkb < 8 || nkb * nbk > cus / 2))
-        return sp;
+        return BackwardSplit{};
     const int64_t longest = a.group * nkb;  // tiles of the key block with the most
     const int64_t tiles = nbk * (a.causal ? longest * (nkb + 1) / 2 : longest * nkb);
-    double best = 0.0;
-    for (int64_t p = 0; p <= std::min<int64_t>(longest, 64); ++p) {
-        BackwardSplit t{};  // (p = 0: the even share of a causal launch)
-        t.chunk = (int)std::min(longest, p ? (longest + p - 1) / p : (tiles + cus - 1) / cus);
-        t.parts = (int)((longest + t.chunk - 1) / t.chunk);
-        t.set_workspace((int)nkb, a.group, a.causal, nbk, 2 * kBwdKeys * a.head_dim);
-        if (t.bytes > limit) continue;  // (one chunk takes none)
-        const double n = (double)(nbk * t.workgroups((int)nkb, a.group, a.causal));
-        const double whole = t.parts == 1 ? n
-                             : a.causal   ? (double)(nbk * std::min<int64_t>(nkb, t.chunk / a.group))
-                                          : 0.0;
-        const double cost = t.parts == 1 ? 2.0 : 2.0 + 3.0 * std::min(1.0, (n - whole) / cus);
-        double est = t.chunk + cost;                             // one round,
-        if (n > cus && !a.causal) est *= std::ceil(n / cus);     // rounds of equal chunks,
-        else if (n > cus)                                        // or the short ones level the end
-            est = std::max(est, (tiles + 2.0 * whole + cost * (n - whole)) / cus +
-                                    t.chunk / (t.parts > 2 ? 2.0 : 8.0));
-        if (best == 0.0 || est < best) {
-            best = est;
-            sp = t;
+    auto of_chunk = [&](int64_t chunk) {
+        BackwardSplit t{};
+        t.set_chunk(chunk, longest, (int)nkb, a.group, a.causal, nbk, 2 * kBwdKeys * a.head_dim);
+        return t;
+    };
+    BackwardSplit best = of_chunk(longest);
+    int64_t best_time = split_time(best, (int)nkb, a, nbk, cus);
+    auto consider = [&](const BackwardSplit& t) {
+        if (t.bytes > limit) return;
+        const int64_t time = split_time(t, (int)nkb, a, nbk, cus);
+        if (time < best_time) {
+            best_time = time;
+            best = t;
         }
+    };
+    auto rounds = [&](const BackwardSplit& t) {
+        const int n = (int)nkb + t.slots - t.split_blocks((int)nkb, a.group, a.causal);  // of a unit
+        return (nbk * n + cus - 1) / cus;
+    };
+    BackwardSplit last = best;
+    int64_t last_rounds = rounds(last);
+    for (int64_t p = 2; p <= std::min<int64_t>(longest, 64); ++p) {
+        const BackwardSplit t = of_chunk((longest + p - 1) / p);
+        if (t.chunk == last.chunk) continue;
+        const int64_t r = rounds(t);
+        if (r > 4) break;
+        if (r > last_rounds || p == 2) {
+            if (p > 2) consider(last);
+            consider(t);
+        }
+        last = t;
+        last_rounds = r;
     }
-    return a64 && sp.parts == 1 ? BackwardSplit{} : sp;
+    consider(last);
+    consider(of_chunk((tiles + cus - 1) / cus));
+    return a64 && best.parts == 1 ? BackwardSplit{} : best;
 }
 
 void launch_backward(Dtype dt, const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s,

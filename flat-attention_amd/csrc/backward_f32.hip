@@ -369,13 +369,11 @@ BackwardSplit backward_f32_split(const BackwardArgs& a, uint64_t limit) {
     const int64_t per_wave = std::max<int64_t>(1, (nbk * a.group * blocks + waves - 1) / waves);
     BackwardSplit sp{};
     if (a.head_dim > 64 && nbk * ((a.seq + 127) / 128) >= device_cus() * (a.causal ? 2 : 1)) return sp;
-    sp.chunk = (int)std::min<int64_t>(4 * per_wave, a.group * nq);
-    for (;;) {
-        sp.parts = (int)((a.group * nq + sp.chunk - 1) / sp.chunk);
-        sp.set_workspace((int)nq, a.group, a.causal, nbk, 64 * a.head_dim);
-        if (sp.bytes <= limit) return sp;
-        sp.chunk = (int)(a.group * nq);  // one chunk: no partials
-    }
+    const int64_t longest = a.group * nq;
+    sp.set_chunk(4 * per_wave, longest, (int)nq, a.group, a.causal, nbk, 64 * a.head_dim);
+    if (sp.bytes > limit)  // one chunk: no partials
+        sp.set_chunk(longest, longest, (int)nq, a.group, a.causal, nbk, 64 * a.head_dim);
+    return sp;
 }
 
 void launch_backward_f32(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {

@@ -169,6 +169,9 @@ struct BackwardSplit {
     float* part;
     int parts, chunk;
     int slots;  // partials of one (batch, kv head): its workgroups whose key block has several chunks
+    // chunk / group and the remainder, the same of the tiles before the last chunk: the kernels walk
+    // the chunks without a division, which takes a lone wave about a microsecond
+    int whole, odd, last_whole, last_odd;
     uint64_t bytes;
 
     // Key blocks (of nkb) that have a chunk `p` < parts: G (nkb - kb) query blocks see key block kb
@@ -189,43 +192,51 @@ struct BackwardSplit {
     // index is the slot of its partials too.
     __host__ __device__ int workgroups(int nkb, int group, bool causal) const {
         int n = 0;
-        for (int p = 0; p < parts; ++p) n += blocks(p, nkb, group, causal);
+        int hidden = 0, rest = 0;  // blocks(p) = nkb - hidden
+        for (int p = 0; p < parts; ++p) {
+            n += causal ? nkb - hidden : nkb;
+            rest += odd;
+            hidden += whole + (rest >= group);
+            if (rest >= group) rest -= group;
+        }
         return n;
     }
-    // (Chunks are walked with two divisions in all: a lone wave takes longer over one per chunk than
-    // over a tile's loads.)
     __host__ __device__ void coords(int idx, int nkb, int group, bool causal, int& kb, int& part) const {
-        const uint32_t g = (uint32_t)group, whole = chunk / g, odd = chunk - whole * g;
-        const uint32_t last = (uint32_t)(parts - 1) * (uint32_t)chunk;
-        uint32_t hidden = last / g, rest = last - hidden * g;  // blocks(part) = nkb - hidden
+        int hidden = last_whole, rest = last_odd;  // blocks(part) = nkb - hidden
         for (part = parts - 1; part > 0; --part) {
-            const int n = causal ? nkb - (int)hidden : nkb;
+            const int n = causal ? nkb - hidden : nkb;
             if (idx < n) break;
             idx -= n;
             hidden -= whole + (rest < odd);
-            rest += (rest < odd ? g : 0) - odd;
+            rest += (rest < odd ? group : 0) - odd;
         }
         kb = idx;
     }
     // The slots of key block kb's chunks, chunk 0 first: next() goes on to the next one.
     struct Walk {
-        int slot, nkb;
-        uint32_t g, whole, odd, hidden = 0, rest = 0;
+        int slot, nkb, group, whole, odd, hidden = 0, rest = 0;
         bool causal;
-        __host__ __device__ Walk(const BackwardSplit& sp, int kb, int nkb_, int group, bool causal_)
-            : nkb(nkb_), g((uint32_t)group), whole((uint32_t)sp.chunk / g),
-              odd((uint32_t)sp.chunk - whole * g), causal(causal_) {
-            slot = sp.slots - (causal ? nkb - (int)whole : nkb) + kb;
-        }
+        __host__ __device__ Walk(const BackwardSplit& sp, int kb, int nkb_, int group_, bool causal_)
+            : slot(sp.slots - (causal_ ? nkb_ - sp.whole : nkb_) + kb), nkb(nkb_), group(group_),
+              whole(sp.whole), odd(sp.odd), causal(causal_) {}
         __host__ __device__ void next() {
             rest += odd;
-            hidden += whole + (rest >= g);
-            if (rest >= g) rest -= g;
-            slot -= causal ? nkb - (int)hidden : nkb;
+            hidden += whole + (rest >= group);
+            if (rest >= group) rest -= group;
+            slot -= causal ? nkb - hidden : nkb;
         }
     };
-    // Sets slots and bytes; a partial is dK and dV of a key block, `floats` together.
-    void set_workspace(int nkb, int group, bool causal, uint64_t units, uint64_t floats) {
+    // Sets parts and what follows from chunk (of `longest` blocks that see the first key block); a
+    // partial is dK and dV of a key block, `floats` together.
+    void set_chunk(int64_t chunk_, int64_t longest, int nkb, int group, bool causal, uint64_t units,
+                   uint64_t floats) {
+        chunk = (int)(chunk_ < longest ? chunk_ : longest);
+        parts = (int)((longest + chunk - 1) / chunk);
+        whole = chunk / group;
+        odd = chunk % group;
+        const int64_t before = (int64_t)(parts - 1) * chunk;
+        last_whole = (int)(before / group);
+        last_odd = (int)(before % group);
         slots = parts > 1 ? workgroups(nkb, group, causal) - nkb + split_blocks(nkb, group, causal)
                           : 0;
         bytes = units * slots * floats * 4;

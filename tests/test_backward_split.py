@@ -2,6 +2,7 @@
 BackwardSplit in csrc/kernels.hpp): the partials' workspace stays under its limit, whatever the
 shape, and the index arithmetic of the kernels (chunk and slot of a workgroup, slots of a key block)
 agrees with plain loops. A small host program, built here, calls the library's own functions."""
+import heapq
 import os
 import shutil
 import subprocess
@@ -79,3 +80,39 @@ def test_short_sequences_keep_their_split(split):
     cases = [(fa.DTYPE_BF16, 1, 6, 1, 1500, 128, 1, LIMIT), (fa.DTYPE_BF16, 1, 32, 8, 2000, 128, 1, LIMIT),
              (fa.DTYPE_BF16, 1, 8, 2, 512, 64, 1, LIMIT), (fa.DTYPE_F32, 1, 8, 2, 512, 64, 1, LIMIT)]
     assert [r[:2] for r in split(cases)] == [(2, 36), (22, 3), (1, 16), (4, 16)]
+
+
+def _makespan(dims, causal, chunk, cus=256):
+    """Tiles of time of a dK/dV launch in chunks of `chunk` tiles: its workgroups in dispatch order,
+    each on the first CU that is free; two tiles for a workgroup, four for one with partials."""
+    b, hq, hkv, s, _ = dims
+    group, nkb = hq // hkv, -(-s // 128)
+    all_tiles = [group * (nkb - kb if causal else nkb) for kb in range(nkb)]
+    free = [0] * cus
+    for p in range(-(-group * nkb // chunk) - 1, -1, -1):
+        for t in all_tiles:
+            if t <= p * chunk:
+                break
+            cost = min(chunk, t - p * chunk) + (4 if t > chunk else 2)
+            for _ in range(b * hkv):
+                heapq.heapreplace(free, free[0] + cost)
+    return max(free)
+
+
+def test_split_has_the_least_time_of_all_splits(split):
+    """The chosen split's time is within 3 % (the candidates are few, time is counted in steps) of
+    the best of every number of chunks that gives up to four rounds of workgroups."""
+    rng = np.random.default_rng(8)
+    cases = []
+    while len(cases) < 40:
+        hq, hkv = [(8, 2), (16, 4), (32, 8), (8, 8), (12, 4), (6, 1)][int(rng.integers(6))]
+        cases.append((fa.DTYPE_BF16, int(rng.integers(1, 3)), hq, hkv,
+                      int(np.exp(rng.uniform(np.log(64), np.log(4096)))), 128,
+                      int(rng.integers(0, 2)), 1 << 40))
+    cases += [(fa.DTYPE_BF16, 2, 32, 8, 1000, 128, 1, LIMIT), (fa.DTYPE_BF16, 1, 16, 4, 4000, 128, 1, LIMIT)]
+    for case, (chunk, parts, slots, _, several) in zip(cases, split(cases)):
+        dims, causal = case[1:6], case[6]
+        longest = dims[1] // dims[2] * -(-dims[3] // 128)
+        best = min(_makespan(dims, causal, -(-longest // p)) for p in range(1, min(longest, 40) + 1)
+                   if p < 3 or dims[0] * dims[2] * p * -(-dims[3] // 128) < 8 * 256)
+        assert _makespan(dims, causal, chunk) <= 1.03 * best + 1, case
