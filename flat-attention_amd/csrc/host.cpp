@@ -1974,14 +1974,35 @@ uint64_t max_split_tokens(uint64_t page_size) {
     return std::max<uint64_t>(16, t);
 }
 
-// Tokens per segment: an equal share of `total` for each of G resident workgroups, in whole 16-key
-// steps. Shares of one step are doubled once there are more than 256 of them: by then a head's
-// partials cost the combine more than a second step costs a wave (one sequence of 8192 bf16
-// tokens, Hq16 Hkv4 D64: 13.1 us at 16 tokens, 10.6 at 32; four of 40..600 tokens, Hq32 Hkv8
-// D128: 11.7 at 16, 16.8 at 32).
-uint64_t segment_tokens(uint64_t total, uint64_t G) {
-    const uint64_t L = std::max<uint64_t>(16, ((total + G - 1) / G + 15) / 16 * 16);
-    return L == 16 && total > 256 * 16 ? 32 : L;
+// Tokens per segment, and whether a unit's first segment begins a workgroup's share (`apart`). The
+// share is an equal part of all keys for each of G resident workgroups, in whole 16-key steps; every
+// context counts `units` times. Laid end to end, a workgroup may take the end of one unit and the
+// begin of the next, and its second prologue costs more than a step: units are kept apart where the
+// workgroups suffice for that, with a share at most a step longer (us, end to end / apart, D 128: four
+// sequences of 1200 tokens, f16 Hq32 Hkv8 18.7 / 14.2, f32 28.7 / 21.9).
+// Shares of one step are doubled where a head has more than 128 of them, or there are 512 in all: then
+// the combine, or so many workgroups at once, cost more than the second step (16 / 32 tokens: 8192 f16
+// tokens, Hq16 Hkv4 D64, 13.7 / 11.1; f32 D128, two of 3000 22.1 / 18.1, sixteen of 500 24.5 / 19.2;
+// with fewer f16 Hq8 Hkv8 D128 1024 tokens 11.5 / 12.4, four of 600 12.0 / 12.9).
+struct SegmentShare {
+    uint64_t tokens;
+    bool apart;
+};
+SegmentShare segment_share(const std::vector<int32_t>& ctx_lens, uint64_t units, uint64_t G) {
+    uint64_t steps = 0, most = 0;
+    for (int32_t c : ctx_lens) {
+        const uint64_t n = ((uint64_t)c + 15) / 16;
+        steps += n * units;
+        most = std::max(most, n);
+    }
+    uint64_t share = std::max<uint64_t>(1, (steps + G - 1) / G);
+    if (share == 1 && (most > 128 || steps >= 512)) share = 2;
+    for (uint64_t s = share; s <= share + 1; ++s) {
+        uint64_t n = 0;
+        for (int32_t c : ctx_lens) n += units * (((uint64_t)c + 16 * s - 1) / (16 * s));
+        if (n <= G) return {16 * s, true};
+    }
+    return {16 * share, false};
 }
 
 // Work list of a decode plan. A unit is (kv head, chunk of <= 16 query heads); the key space
@@ -2014,9 +2035,7 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
     std::vector<int32_t> unit_part(p->n_seqs * units + 1, 0);
     uint64_t longest = 0;
     if (p->grouped > 0) {
-        uint64_t total = 0;
-        for (int32_t c : p->ctx_lens) total += ((uint64_t)c + 15) / 16 * 16;
-        const uint64_t L = segment_tokens(total, G);
+        const auto [L, apart] = segment_share(p->ctx_lens, 1, G);
         uint64_t pos = 0;
         int32_t slot = 0;
         for (uint64_t s = 0; s < p->n_seqs; ++s) {
@@ -2030,7 +2049,7 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
                 longest = std::max(longest, e - t);
                 t = e;
             }
-            pos += cpad;
+            pos += apart ? (cpad + L - 1) / L * L : cpad;
             const int32_t nseg = (int32_t)(segs.size() - first);
             for (uint64_t u = 0; u < units; ++u)
                 unit_part[s * units + u] = nseg > 1 ? slot + (int32_t)u * nseg : slot;
@@ -2048,10 +2067,8 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
             return fail(FA_ERR_DISPATCH_LIMIT, "paged decode requires %llu segments",
                         (unsigned long long)segs.size());
     } else {
-    uint64_t total = 0;
-    for (int32_t c : p->ctx_lens) total += ((uint64_t)c + 15) / 16 * 16 * units;
     if (p->split_req == 0) {
-        const uint64_t L = segment_tokens(total, G);
+        const auto [L, apart] = segment_share(p->ctx_lens, units, G);
         uint64_t pos = 0;
         for (uint64_t s = 0; s < p->n_seqs; ++s) {
             const uint64_t c = (uint64_t)p->ctx_lens[s];
@@ -2066,7 +2083,7 @@ int compute_work(fa_decode_plan* p, std::vector<int32_t>* all_out) {
                     longest = std::max(longest, e - t);
                     t = e;
                 }
-                pos += cpad;
+                pos += apart ? (cpad + L - 1) / L * L : cpad;
             }
         }
     } else {

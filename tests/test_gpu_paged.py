@@ -172,6 +172,35 @@ def test_split_count_invariance(hip):
             assert_close(f"LSE split {split}", l, ref[1], 1e-4, 1e-5)
 
 
+@pytest.mark.parametrize("dtype,hq,hkv,D,ctx_lens,tokens", [
+    # f32: one-wave workgroups, every kv head a unit of its own
+    (fa.DTYPE_F32, 32, 8, 128, [600], 16),        # 4864 keys in all, but 38 steps a head
+    (fa.DTYPE_F32, 8, 8, 64, [100] * 8, 16),
+    (fa.DTYPE_F32, 16, 4, 128, [2000, 2000], 32),  # 1000 steps in all; an odd 125 to a unit
+    (fa.DTYPE_F32, 16, 4, 64, [3000], 32),         # 188 steps
+    (fa.DTYPE_F32, 8, 2, 64, [2048], 16),          # 128 steps
+    # f16: head-grouped workgroups, one segment list for all kv heads
+    (fa.DTYPE_F16, 16, 4, 64, [1200] * 4, 16),
+    (fa.DTYPE_F16, 16, 4, 64, [8192], 32),
+    (fa.DTYPE_F16, 16, 4, 64, [3000, 2999], 32),
+    (fa.DTYPE_F16, 6, 1, 128, [5000, 100], 32),    # 313 steps and 7
+    (fa.DTYPE_BF16, 4, 2, 64, [33], 16),
+])
+def test_segments_end_with_their_unit(hip, dtype, hq, hkv, D, ctx_lens, tokens):
+    """No workgroup takes parts of two units where there are enough of them, and segments of one
+    16-key step double by the partials of a head or the steps of the call; and the result."""
+    rnd = {fa.DTYPE_F32: lambda x: x, fa.DTYPE_BF16: bf16_round, fa.DTYPE_F16: f16_round}[dtype]
+    ps = 16
+    bt, kp, vp, total = _make_pool(np.random.default_rng(3), ctx_lens, ps, hkv, D, rnd)
+    q = rnd(normal(len(ctx_lens) * hq * D, 4))
+    o, l, plan = _decode(hip, bt, ctx_lens, kp, vp, total, ps, hq, hkv, D, q, dtype)
+    assert plan.info()["work_items"] == hkv * sum(-(-c // tokens) for c in ctx_lens)
+    eo, el = oracle.paged_decode(q, kp, vp, total, ps, bt, ctx_lens, hq, hkv, D, True, 1e4)
+    atol, rtol = (F32_ATOL, F32_RTOL) if dtype == fa.DTYPE_F32 else (H16_ATOL, 0.0)
+    assert_close("O", o, eo, atol, rtol)
+    assert_close("LSE", l, el, atol, rtol)
+
+
 @pytest.mark.parametrize("D,dtype", [(32, fa.DTYPE_F32), (64, fa.DTYPE_BF16), (80, fa.DTYPE_F32),
                                      (128, fa.DTYPE_F32), (128, fa.DTYPE_F16)])
 @pytest.mark.parametrize("most", [2, 8, 9, 33, 130])
