@@ -1753,19 +1753,34 @@ static bool f32_rows_ok(const PrefillArgs& a) {
            (uint64_t)a.kv_len * (uint64_t)a.k_ss * 4u <= INT32_MAX;
 }
 
-// f32 launches that take prefill_f32_groups: those whose 128-row blocks do not fill the places of
-// prefill_mfma_f32, two to a CU (times in us per call, that kernel / this one): H2 S128 D64 causal
-// 19.4 / 7.4, B4 H2 S655 D128 105.0 / 35.2, H8 S2048 D64 causal 161.6 / 49.2, B4 H16 S512 D128
-// causal, 256 blocks, 91.4 / 66.8; at 512 blocks H16 B2 S2048 D128 397.7 / 340.8, but Hq32 Hkv8
-// B2 S1000 D64 121.8 / 129.6; at 1024 blocks B4 H16 S2048 D128 628.8 / 691.2, where the tiles
-// that four waves share in LDS count for more.
+// f32 launches that take prefill_f32_groups: where 128-row blocks leave prefill_mfma_f32 idle, which
+// runs one block per CU in one time, up to two in 1.75, and whose tiles, which four waves share in LDS,
+// count for more once it is full (times in us per call, that kernel / this one):
+//   head_dim <= 32: fewer blocks than two per CU (H32 B2 S300 20.2 / 16.6, S500 28.9 / 27.0, B4 S200,
+//     256 blocks, 16.4 / 16.9; B4 S500, 512 blocks, 47.9 / 48.9);
+//   where the 32-row workgroups, two to a CU, are one round (no mask, D64 H32 B2 S200, 448 of them,
+//     27.4 / 19.0, S300, 640, 35.5 / 38.8; B4 S200, 896, 28.2 / 34.6; D80 42.6 / 55.5), or at D128
+//     one and a half (B2 S300 61.0 / 55.9; B4 S200 49.4 / 57.0), except that with as many blocks of
+//     few rows the two are level;
+//   more of them under a causal mask: by the share of the keys that the rows see, as blocks of unequal length leave that kernel
+//     idle and this one not: up to 0.8 of one block per CU, 0.6 of two (D128 H32 B2 S500, 256 blocks of
+//     which 0.63 counts, 89.9 / 66.7; B4 S200, 256 of 0.82, 44.6 / 44.6, D80 39.1 / 41.9; S300, 384 of
+//     0.71, 77.9 / 67.4; S500, 512 of 0.63, 123.4 / 132.7; B2 H16 S2048, 512 of 0.53, 398 / 341).
 bool prefill_uses_f32_groups(Dtype dt, bool paged, const PrefillArgs& a) {
-    if (dt != Dtype::F32 || paged || !f32_rows_ok(a) || (uintptr_t)a.q % 16 || a.q_ss % 4 || a.q_sh % 4 || a.q_sb % 4 ||
-        (uintptr_t)a.o % 16 || a.o_ss % 4 || a.o_sh % 4 || a.o_sb % 4)
+    if (dt != Dtype::F32 || paged || !f32_rows_ok(a) || (uintptr_t)a.q % 16 || a.q_ss % 4 ||
+        a.q_sh % 4 || a.q_sb % 4 || (uintptr_t)a.o % 16 || a.o_ss % 4 || a.o_sh % 4 || a.o_sb % 4)
         return false;
-    const int64_t blocks = (int64_t)a.batch * a.kv_heads *
-                           (((int64_t)a.q_len * a.group + 127) / 128);
-    return blocks < 2 * (int64_t)device_cus() + (a.head_dim > 64 ? 1 : 0);
+    const int64_t cus = device_cus(), units = (int64_t)a.batch * a.kv_heads;
+    const int64_t rows = (int64_t)a.q_len * a.group, blocks = units * ((rows + 127) / 128);
+    if (a.head_dim <= 32) return blocks < 2 * cus;
+    if (units * ((rows + 31) / 32) <= (a.head_dim == 128 ? 3 : 2) * cus)
+        return blocks < 2 * cus + (a.head_dim > 64 ? 1 : 0);
+    if (!a.causal) return false;
+    // positions of the first row, and of the one past the last (a padded batch: of its longest)
+    const int64_t first = a.var_meta ? std::max(0, a.kv_len - a.q_len) : a.causal_offset;
+    const int64_t last = first + a.q_len;
+    const double seen = std::min(1.0, (double)(first + last + 128) / (2.0 * (double)last));
+    return blocks <= 2 * cus && (double)blocks * seen <= (blocks <= cus ? 0.8 : 1.2) * (double)cus;
 }
 
 void prefill_geometry(Dtype dt, bool paged, const PrefillArgs& a, unsigned grid[3],

@@ -180,6 +180,36 @@ def test_f32_key_group_prefill_matches_oracle(hip, B, hq, hkv, S, D, rope, rows,
     assert_close("LSE", l, el, F32_ATOL, F32_RTOL)
 
 
+@pytest.mark.parametrize("B,H,S,D,causal,rows", [
+    (1, 32, 500, 64, False, 32),    # 512 workgroups of 32 rows: one round
+    (2, 32, 300, 64, False, 128),   # 640: more than one, and 192 blocks of 128 rows
+    (2, 32, 300, 64, True, 32),     # causal: of which 0.71 counts
+    (2, 32, 300, 128, False, 32),   # one and a half rounds at D 128
+    (4, 32, 200, 80, False, 128),
+    (4, 32, 200, 80, True, 128),    # 256 blocks of which 0.82 counts
+    (4, 32, 300, 96, True, 32),     # 384 of which 0.71 counts
+    (6, 32, 257, 64, False, 128),   # 576 blocks: the LDS kernel, three of them and five key tiles a head
+    (6, 32, 257, 64, True, 128),
+    (6, 32, 257, 80, True, 128),
+    (6, 32, 257, 128, False, 128),
+    (6, 32, 257, 128, True, 128),
+    (4, 32, 300, 32, False, 32),
+    (6, 32, 257, 32, True, 128),
+])
+def test_f32_prefill_kernel_by_filled_chip(hip, B, H, S, D, causal, rows):
+    """Which f32 kernel a launch takes as its row blocks fill the chip, and both kernels over several
+    row blocks and key tiles that end part-way (the first and the last heads against the oracle)."""
+    q, k, v = (normal(B * H * S * D, 770 + S + i) for i in range(3))
+    shape = fa.GroupedAttentionShape(B, H, H, S, D)
+    o, l = _run_grouped(hip, q, k, v, shape, fa.FlatAttentionConfig(causal), None, fa.DTYPE_F32)
+    assert hip.last_telemetry().query_rows == rows
+    for u in (0, B * H - 2):
+        eo, el = _oracle_grouped(q, k, v, shape, causal, None, units=(u, u + 2))
+        at = slice(u * S, (u + 2) * S)
+        assert_close("O", o.reshape(-1, D)[at], eo.reshape(-1, D)[at], F32_ATOL, F32_RTOL)
+        assert_close("LSE", l[at], el[at], F32_ATOL, F32_RTOL)
+
+
 @pytest.mark.parametrize("dtype,rnd", [(fa.DTYPE_BF16, bf16_round), (fa.DTYPE_F16, f16_round)])
 @pytest.mark.parametrize("B,hq,hkv,S,D,rope,groups", [
     (1, 8, 2, 65, 64, True, 4),      # two key tiles: groups 2 and 3 have none; K rotated on load
