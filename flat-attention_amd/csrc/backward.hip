@@ -369,9 +369,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
     // key blocks in ascending order: under a causal mask the early blocks see the most queries,
     // so the heaviest workgroups dispatch first
     const int bkv = blockIdx.x % nbk;
-    const int slot = blockIdx.x / nbk;
     int kb, part;
-    sp.coords(slot, (S + kBwdKeys - 1) / kBwdKeys, G, a.causal, kb, part);
+    sp.coords(blockIdx.x / nbk, (S + kBwdKeys - 1) / kBwdKeys, G, a.causal, kb, part);
     const int b = bkv / a.kv_heads, kvh = bkv - b * a.kv_heads;
     const int k0 = kb * kBwdKeys + wave * 32;
     const int64_t krow0 = (int64_t)bkv * S;
@@ -651,7 +650,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
     }
     // register r: key k0 + 8 (r / 4) + 4 g + r % 4, dim 32 m + c
     if (all_tiles > sp.chunk) {  // dK then dV, kBwdKeys rows of D each
-        float* const pp = sp.part + ((int64_t)bkv * sp.slots + slot) * 2 * kBwdKeys * D;
+        float* const pp = sp.part + (int64_t)blockIdx.x * 2 * kBwdKeys * D;
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
             const int d = 32 * m + c;
@@ -694,8 +693,8 @@ __device__ __forceinline__ void add_partials(const BackwardArgs& a, const Backwa
     const int nqt = nkb - (a.causal ? kb : 0);
     const int n = (a.group * nqt + sp.chunk - 1) / sp.chunk;
     if (n <= 1) return;  // written by bwd_dkdv
-    const int64_t step = (int64_t)2 * kBwdKeys * D;
-    const float* const base = sp.part + (int64_t)bkv * sp.slots * step + r0 * D;
+    const int64_t step = (int64_t)2 * kBwdKeys * D * a.batch * a.kv_heads;
+    const float* const base = sp.part + (int64_t)bkv * 2 * kBwdKeys * D + r0 * D;
     const BackwardSplit::Walk first(sp, kb, nkb, a.group, a.causal);
     const int count = min(kAddRows, S - kb * kBwdKeys - r0) * D;  // (may be negative: no rows)
     const int64_t out = ((int64_t)bkv * S + kb * kBwdKeys + r0) * D;
@@ -1088,14 +1087,16 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
     hipLaunchKernelGGL((bwd_delta<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, s, a,
                        rows);
     if constexpr (std::is_same_v<T, float>) {
-        // (no split: head dims above 64 only)
-        if (sp.parts > 0) launch_backward_f32(a, sp, s);
-        else {
-            BackwardSplit one{};
-            one.parts = 1;
-            one.chunk = INT32_MAX;
-            launch_dma<float, 128>(a, one, s);
+        if (sp.parts > 0) {
+            launch_backward_f32(a, sp, s);
+            return;
         }
+        BackwardSplit one{};
+        one.parts = 1;
+        one.chunk = INT32_MAX;
+        if (a.head_dim <= 32) launch_dma<T, 32>(a, one, s);
+        else if (a.head_dim <= 64) launch_dma<T, 64>(a, one, s);
+        else launch_dma<T, 128>(a, one, s);
     } else {
         if (a.head_dim <= 32) launch_dma<T, 32>(a, sp, s);
         else if (a.head_dim <= 64) launch_dma<T, 64>(a, sp, s);
@@ -1105,18 +1106,16 @@ void launch_dims(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s, 
 
 }  // namespace
 
-// Time, in tiles (128 queries of one head), of a split dK/dV launch: its workgroups in dispatch order,
-// each on the first of the CUs, which hold one workgroup, that is free. A workgroup costs two tiles
-// beside its own, one with partials four: 256 D floats are written and read again.
-static int64_t split_time(const BackwardSplit& sp, int nkb, const BackwardArgs& a, int64_t units,
-                          int64_t cus) {
+int64_t backward_time(const BackwardSplit& sp, int nkb, const BackwardArgs& a, int64_t places,
+                      int whole, int split) {
     constexpr int kSteps = 512;  // steps of time, of `unit` tiles
     uint32_t free_at[kSteps] = {};
-    const int64_t longest = (int64_t)a.group * nkb;
+    const int64_t longest = (int64_t)a.group * nkb, units = (int64_t)a.batch * a.kv_heads;
     const int64_t tiles = units * (a.causal ? longest * (nkb + 1) / 2 : longest * nkb);
-    const int64_t n = units * (nkb + sp.slots);  // (or a few more)
-    const int64_t unit = 1 + (tiles + 4 * n) / (cus * (kSteps / 4)) + (sp.chunk + 4) / (kSteps / 4);
-    free_at[0] = (uint32_t)cus;
+    const int64_t n = units * (nkb + sp.slots);  // (or a few less)
+    if (n > 16 * places) return (tiles + (sp.parts > 1 ? split : whole) * n + places - 1) / places;
+    const int64_t unit = 1 + (tiles + split * n) / (places * (kSteps / 4)) + (sp.chunk + split) / (kSteps / 4);
+    free_at[0] = (uint32_t)places;
     int64_t now = 0, end = 0;
     auto place = [&](int64_t count, int64_t time) {
         const int64_t d = (time + unit - 1) / unit;
@@ -1138,18 +1137,19 @@ static int64_t split_time(const BackwardSplit& sp, int nkb, const BackwardArgs& 
         int kb = !a.causal ? blocks : (int)std::max<int64_t>(0, nkb - (before + sp.chunk) / a.group);
         kb = std::min(kb, blocks);
         if (kb > 0)
-            place(units * kb, std::min<int64_t>(sp.chunk, longest - before) + (sp.parts > 1 ? 4 : 2));
+            place(units * kb, std::min<int64_t>(sp.chunk, longest - before) + (sp.parts > 1 ? split : whole));
         for (; kb < blocks; ++kb) {  // (causal: the last blocks that have this chunk)
             const int64_t all = (int64_t)a.group * (nkb - kb);
-            place(units, std::min<int64_t>(sp.chunk, all - before) + (all > sp.chunk ? 4 : 2));
+            place(units, std::min<int64_t>(sp.chunk, all - before) + (all > sp.chunk ? split : whole));
         }
     }
     return end * unit;
 }
 
-// parts = 0: the assembly kernel. Else the number of chunks with the least time: one, two, an even
-// share of the tiles for each CU, or a number next to one, two or three full rounds of workgroups.
-// Measured against 1 to 36 chunks at 25 shapes (Hq6 Hkv1 to B2 Hq32 Hkv8, S 512 to 4000, with and
+// parts = 0: the assembly kernel. Else the number of chunks with the least time (one workgroup to a
+// CU; one costs two tiles of 128 queries of a head beside its own, one with partials four, as 256 D
+// floats are written and read again): one, two, an even share of the tiles for each CU, or a number
+// next to one, two or three full rounds of workgroups. Measured against 1 to 36 chunks at 25 shapes (Hq6 Hkv1 to B2 Hq32 Hkv8, S 512 to 4000, with and
 // without a mask) the choice took at most 1 % longer than the best of them; so did none of the
 // choices with three tiles for partials, and with five one 4 %. (us for the backward, bf16 causal D
 // 128, one chunk / chosen / twice as many: Hq16 Hkv4 S1000 166 / 51 / 61; Hq32 Hkv8 B2 S1000 177 /
@@ -1177,10 +1177,10 @@ BackwardSplit backward_split(Dtype dt, const BackwardArgs& a, uint64_t limit) {
         return t;
     };
     BackwardSplit best = of_chunk(longest);
-    int64_t best_time = split_time(best, (int)nkb, a, nbk, cus);
+    int64_t best_time = backward_time(best, (int)nkb, a, cus, 2, 4);
     auto consider = [&](const BackwardSplit& t) {
         if (t.bytes > limit) return;
-        const int64_t time = split_time(t, (int)nkb, a, nbk, cus);
+        const int64_t time = backward_time(t, (int)nkb, a, cus, 2, 4);
         if (time < best_time) {
             best_time = time;
             best = t;

@@ -104,9 +104,8 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     const int S = a.seq, D = a.head_dim, nq = (S + 31) / 32, nbk = a.batch * a.kv_heads;
     // early key blocks first: under a causal mask they see the most queries
     const int bkv = blockIdx.x % nbk;
-    const int slot = blockIdx.x / nbk;
     int kb, part;
-    sp.coords(slot, nq, a.group, a.causal, kb, part);
+    sp.coords(blockIdx.x / nbk, nq, a.group, a.causal, kb, part);
     const int qb0 = a.causal ? kb : 0, nqv = nq - qb0, items = a.group * nqv;
     const int first = part * sp.chunk, last = min(items, first + sp.chunk);
     const int b = bkv / a.kv_heads, kvh = bkv - b * a.kv_heads;
@@ -202,7 +201,7 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     }
     // one chunk: the gradients themselves; else this chunk's partials (dK, then dV)
     const bool whole = items <= sp.chunk;
-    float* const pp = sp.part + ((int64_t)bkv * sp.slots + slot) * 64 * D;
+    float* const pp = sp.part + (int64_t)blockIdx.x * 64 * D;
     reduce_waves<DPAD, 4>(lds, dk, D, [&](int r, int d, float x) {
         if (!whole) pp[r * D + d] = x;
         else if (k0 + r < S) ((float*)a.dk)[(krow0 + k0 + r) * D + d] = x * a.scale;
@@ -221,8 +220,8 @@ __device__ __forceinline__ void add_partials(const BackwardArgs& a, const Backwa
     const int items = a.group * (nkb - (a.causal ? kb : 0));
     const int n = (items + sp.chunk - 1) / sp.chunk;
     if (n <= 1) return;  // written by bwd_f32_dkdv
-    const int64_t step = (int64_t)64 * D;
-    const float* const base = sp.part + (int64_t)bkv * sp.slots * step + which * 32 * D;
+    const int64_t step = (int64_t)64 * D * a.batch * a.kv_heads;
+    const float* const base = sp.part + (int64_t)bkv * 64 * D + which * 32 * D;
     const BackwardSplit::Walk first(sp, kb, nkb, a.group, a.causal);
     const float scale = which ? 1.0f : a.scale;
     float* out = (float*)(which ? a.dv : a.dk) + ((int64_t)bkv * S + kb * 32) * D;
@@ -353,11 +352,36 @@ void launch_d(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
 
 }  // namespace
 
-// No split (parts = 0): head dims above 64 where the staged kernels' 128-key workgroups fill the
-// chip, in two rounds under a causal mask (heads H, B1 S2048 D128, those kernels / these, us: H16
-// 962 / 1164, H16 causal 948 / 656, H32 causal 1061 / 1297; Hq32 Hkv8 causal, 128 workgroups, 2529
-// / 1218). At D 64 and below these win throughout (B4 H16 S2048 D64 causal, 1024 workgroups, 1132 /
-// 1095; B2 H8 S1024 D32 causal 158 / 69).
+// Whether the LDS-staged kernels (backward.hip: one workgroup per 128 keys, four waves share the
+// tiles) are the faster ones: where those workgroups fill the chip. `filled` is the part of the CUs'
+// time that they keep busy, one to a CU; over 400 shapes the ratio of the two follows it (us for the
+// backward, staged / these):
+//   D 128: 0.62 (H32 B2 S500 causal) 276 / 253, 0.75 (B4 S200 causal) 145 / 155, 1 (B4 S384 causal)
+//     267 / 326, (B4 S200) 148 / 214; Hq32 Hkv8 S2048 causal, 0.27, 2529 / 1218;
+//   64 < D < 128, where these load and multiply the padding too: D 96, 0.50 (B2 S384 causal) 208 / 197,
+//     0.62 (B2 S500 causal) 266 / 316, 1 (B4 S200) 139 / 261;
+//   D <= 64, where a CU holds two of them: with that chip filled too (D 64, H32 B4 S500 292 / 318, B8
+//     S384 causal 254 / 276, B8 S500 576 / 650; not B4 S384 causal 129 / 118, B6 S384 251 / 221), or up
+//     to 256 keys without a mask, a few tiles to a workgroup, once (B4 S200 85.5 / 94.9), and at D 32
+//     and 64 not with long sequences (B4 S1000 1059 / 1085, B4 H16 S2048 causal 1132 / 1095; D 40 B4
+//     S1000 1034 / 1138).
+static bool staged_f32(const BackwardArgs& a) {
+    const int64_t nkb = (a.seq + 127) / 128, n = (int64_t)a.batch * a.kv_heads * nkb;
+    const int64_t cus = device_cus();
+    if (n < cus / 2) return false;
+    const int64_t longest = a.group * nkb, units = (int64_t)a.batch * a.kv_heads;
+    const double tiles = (double)units * (a.causal ? 0.5 * longest * (nkb + 1) : longest * nkb);
+    BackwardSplit one{};
+    one.set_chunk(longest, longest, (int)nkb, a.group, a.causal, units, 0);
+    auto filled = [&](int64_t places) {
+        return tiles / (double)(places * backward_time(one, (int)nkb, a, places, 0, 0));
+    };
+    if (a.head_dim > 64) return filled(cus) >= (a.head_dim == 128 ? 0.7 : 0.55);
+    const bool full = a.head_dim == 64 || a.head_dim == 32;
+    return (a.seq < 1500 || !full) && filled(cus) >= 0.9 &&
+           (filled(2 * cus) >= (full ? 0.7 : 0.6) || (!a.causal && a.seq <= 256));
+}
+
 // Blocks a wave takes: the total over the waves that the chip holds at once (one per SIMD at
 // D 128, two below), so a launch is one round of about equal workgroups and the partials of a
 // small problem stay a few MB (at most one chunk more than the round has workgroups, twice for
@@ -368,7 +392,7 @@ BackwardSplit backward_f32_split(const BackwardArgs& a, uint64_t limit) {
     const int64_t waves = (int64_t)device_cus() * 4 * (a.head_dim > 64 ? 1 : 2);
     const int64_t per_wave = std::max<int64_t>(1, (nbk * a.group * blocks + waves - 1) / waves);
     BackwardSplit sp{};
-    if (a.head_dim > 64 && nbk * ((a.seq + 127) / 128) >= device_cus() * (a.causal ? 2 : 1)) return sp;
+    if (staged_f32(a)) return sp;
     const int64_t longest = a.group * nq;
     sp.set_chunk(4 * per_wave, longest, (int)nq, a.group, a.causal, nbk, 64 * a.head_dim);
     if (sp.bytes > limit)  // one chunk: no partials

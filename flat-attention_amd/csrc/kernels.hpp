@@ -189,7 +189,7 @@ struct BackwardSplit {
     // in order, shader engine by shader engine, so short and long ones in turn left half the
     // engines idle (Hq32 Hkv8 B2 S3000 D128: 788 us for the backward, 618 unsplit).
     // The workgroups of key blocks with several chunks come before the others, so a workgroup's
-    // index is the slot of its partials too.
+    // index is the slot of its partials too (the (batch, kv head) units of an index side by side).
     __host__ __device__ int workgroups(int nkb, int group, bool causal) const {
         int n = 0;
         int hidden = 0, rest = 0;  // blocks(p) = nkb - hidden
@@ -251,6 +251,10 @@ constexpr uint64_t kBackwardPartialBytes = (uint64_t)256 << 20;
 // still to be set when bytes > 0. parts = 0: the assembly dK/dV kernel (16-bit storage), the
 // LDS-staged f32 kernels.
 BackwardSplit backward_split(Dtype dt, const BackwardArgs& a, uint64_t limit);
+// Time of a dK/dV launch in tiles: its workgroups in dispatch order, each in the first of `places` that
+// is free; a workgroup costs `whole` tiles beside its own, one with partials `split`.
+int64_t backward_time(const BackwardSplit& sp, int nkb, const BackwardArgs& a, int64_t places,
+                      int whole, int split);
 // The f32 kernels without LDS staging, after bwd_delta; two launches.
 BackwardSplit backward_f32_split(const BackwardArgs& a, uint64_t limit);
 void launch_backward_f32(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s);

@@ -128,8 +128,8 @@ def test_f32_tile_edges(hip, dims, causal):
     (1, 8, 8, 129, 100),   # MHA
     (1, 4, 1, 200, 128),
     (1, 2, 2, 1056, 32),   # 33 blocks of one wave's chunk
-    (8, 32, 32, 40, 128),  # 256 key blocks: the LDS-staged kernels without a mask
-    (16, 32, 32, 33, 96),  # 512: and with one
+    (8, 32, 32, 40, 128),  # 256 key blocks of 128: the LDS-staged kernels
+    (16, 32, 32, 33, 96),
 ])
 @pytest.mark.parametrize("causal", [True, False])
 def test_f32_backward_splits_match_oracle(hip, dims, causal):
@@ -143,8 +143,7 @@ def test_f32_backward_splits_match_oracle(hip, dims, causal):
     pipe = fa.HipGroupedBackwardRecomputePipeline(hip, fa.DTYPE_F32)
     got = pipe.backward(q, k, v, do, fwd, shape, fa.FlatAttentionConfig(causal))
     t = hip.last_telemetry()
-    staged = D > 64 and B * Hkv * ((S + 127) // 128) >= (512 if causal else 256)
-    if staged:
+    if B >= 8:
         assert "bwd_dkdv + bwd_dq<f32>" in t.kernel_name
         assert (t.query_rows, t.kv_rows) == (128, 64)
     else:
@@ -155,6 +154,42 @@ def test_f32_backward_splits_match_oracle(hip, dims, causal):
                               (again.dq, again.dk, again.dv), want):
         assert_close(name, a, e, 2e-5 * max(1.0, float(np.abs(e).max())), 1e-4)
         np.testing.assert_array_equal(a, b_, err_msg=name)
+
+
+@pytest.mark.parametrize("dims,staged", [
+    ((6, 32, 32, 257, 128), (True, True)),   # three key blocks, the last of one row; five query tiles
+    ((6, 64, 32, 257, 96), (True, True)),
+    ((6, 32, 32, 257, 99), (True, True)),    # rows off the 16-byte chunk: staged through registers
+    ((2, 32, 32, 300, 128), (True, False)),  # 192 workgroups; under a mask they are busy half the time
+    ((8, 32, 32, 300, 64), (True, True)),
+    ((8, 32, 32, 300, 33), (True, True)),
+    ((4, 32, 32, 200, 40), (True, False)),   # 256: once round
+    ((4, 32, 32, 300, 32), (False, False)),  # 384: the second of two rounds half filled
+])
+@pytest.mark.parametrize("causal", [False, True])
+def test_f32_backward_of_filled_chip_matches_oracle(hip, dims, staged, causal):
+    """Which f32 backward a call takes, and the LDS-staged kernels over several key blocks and query
+    tiles with remainders (first and last batch element against the oracle); bitwise repeatable."""
+    B, Hq, Hkv, S, D = dims
+    shape, cfg = fa.GroupedAttentionShape(*dims), fa.FlatAttentionConfig(causal)
+    q, k, v, do = (normal(n, 231 + i).reshape(B, -1) for i, n in enumerate(
+        (B * Hq * S * D, B * Hkv * S * D, B * Hkv * S * D, B * Hq * S * D)))
+    fwd = fa.HipRotaryGroupedAttention(hip, fa.DTYPE_F32).forward(
+        q.ravel(), k.ravel(), v.ravel(), shape, cfg, None)
+    pipe = fa.HipGroupedBackwardRecomputePipeline(hip, fa.DTYPE_F32)
+    got, again = (pipe.backward(q.ravel(), k.ravel(), v.ravel(), do.ravel(), fwd, shape, cfg)
+                  for _ in range(2))
+    assert ("bwd_f32" not in hip.last_telemetry().kernel_name) == staged[causal]
+    for name, a, b_ in zip(("dQ", "dK", "dV"), (got.dq, got.dk, got.dv),
+                           (again.dq, again.dk, again.dv)):
+        np.testing.assert_array_equal(a, b_, err_msg=name)
+    o, lse = fwd.output.reshape(B, -1), fwd.lse.reshape(B, -1)
+    for b in (0, B - 1):
+        want = oracle.backward_grouped(q[b], k[b], v[b], do[b], o[b], lse[b], 1, Hq, Hkv, S, D,
+                                       causal, threads=8)
+        for name, a, e in zip(("dQ", "dK", "dV"), (got.dq, got.dk, got.dv), want):
+            assert_close(f"{name}[{b}]", a.reshape(B, -1)[b], e,
+                         2e-5 * max(1.0, float(np.abs(e).max())), 1e-4)
 
 
 @pytest.mark.parametrize("dtype", [fa.DTYPE_BF16, fa.DTYPE_F16])
