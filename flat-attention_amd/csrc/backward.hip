@@ -681,7 +681,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
 
 // ------------------------------------------------------------------ partial dK, dV
 // dK and dV of kAddRows keys of one (batch * kv head, 128 keys): the partials in chunk order. The dQ
-// launches carry these workgroups after their own.
+// launches carry these workgroups after their own, for the key blocks that have several chunks; the
+// early ones, which under a mask have the most, come first.
 constexpr int kAddRows = 16;
 template <typename T>
 __device__ __forceinline__ void add_partials(const BackwardArgs& a, const BackwardSplit& sp,
@@ -689,10 +690,9 @@ __device__ __forceinline__ void add_partials(const BackwardArgs& a, const Backwa
     using B = Blk<T>;
     const int S = a.seq, D = a.head_dim, nkb = (S + kBwdKeys - 1) / kBwdKeys;
     const int r0 = block % (kBwdKeys / kAddRows) * kAddRows, at = block / (kBwdKeys / kAddRows);
-    const int bkv = at / nkb, kb = at - bkv * nkb;
+    const int kb = at / (a.batch * a.kv_heads), bkv = at - kb * (a.batch * a.kv_heads);
     const int nqt = nkb - (a.causal ? kb : 0);
     const int n = (a.group * nqt + sp.chunk - 1) / sp.chunk;
-    if (n <= 1) return;  // written by bwd_dkdv
     const int64_t step = (int64_t)2 * kBwdKeys * D * a.batch * a.kv_heads;
     const float* const base = sp.part + (int64_t)bkv * 2 * kBwdKeys * D + r0 * D;
     const BackwardSplit::Walk first(sp, kb, nkb, a.group, a.causal);
@@ -1046,8 +1046,8 @@ void launch_typed(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s)
     const int nkb = (S + kBwdKeys - 1) / kBwdKeys, nqb = (S + kBwdQueries - 1) / kBwdQueries;
     const unsigned n_kv =
         (unsigned)sp.workgroups(nkb, a.group, a.causal) * a.batch * a.kv_heads;
-    const unsigned n_add =
-        sp.parts > 1 ? (unsigned)nkb * a.batch * a.kv_heads * (kBwdKeys / kAddRows) : 0;
+    const unsigned n_add = (unsigned)sp.split_blocks(nkb, a.group, a.causal) * a.batch *
+                           a.kv_heads * (kBwdKeys / kAddRows);
     if constexpr (DMA && Blk<T>::ES == 2) {
         if (a.ds) {
             hipLaunchKernelGGL((bwd_dkdv<T, DPAD, true, true>), dim3(n_kv), dim3(256), 0, s, a, sp);

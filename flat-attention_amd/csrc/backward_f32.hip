@@ -212,14 +212,15 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     });
 }
 
-// dK (which = 0) or dV of one (batch * kv head, 32 keys): the partials in chunk order.
+// dK (which = 0) or dV of one (batch * kv head, 32 keys) with several chunks: the partials in chunk
+// order.
 __device__ __forceinline__ void add_partials(const BackwardArgs& a, const BackwardSplit& sp,
                                              int block) {
     const int S = a.seq, D = a.head_dim, nkb = (S + 31) / 32;
-    const int which = block & 1, at = block >> 1, bkv = at / nkb, kb = at - bkv * nkb;
+    const int split = sp.split_blocks(nkb, a.group, a.causal);
+    const int which = block & 1, at = block >> 1, bkv = at / split, kb = at - bkv * split;
     const int items = a.group * (nkb - (a.causal ? kb : 0));
     const int n = (items + sp.chunk - 1) / sp.chunk;
-    if (n <= 1) return;  // written by bwd_f32_dkdv
     const int64_t step = (int64_t)64 * D * a.batch * a.kv_heads;
     const float* const base = sp.part + (int64_t)bkv * 64 * D + which * 32 * D;
     const BackwardSplit::Walk first(sp, kb, nkb, a.group, a.causal);
@@ -339,7 +340,7 @@ void launch_v(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
                        dim3((unsigned)(sp.workgroups(nb, a.group, a.causal) * nbk)), dim3(256), 0,
                        s, a, sp);
     const int n_dq = nb * a.batch * a.q_heads;
-    const int n_add = sp.parts > 1 ? 2 * nb * nbk : 0;
+    const int n_add = 2 * sp.split_blocks(nb, a.group, a.causal) * nbk;
     hipLaunchKernelGGL((bwd_f32_dq<DPAD, NW, FULL>), dim3((unsigned)(n_dq + n_add)), dim3(64 * NW), 0, s,
                        a, sp, n_dq);
 }

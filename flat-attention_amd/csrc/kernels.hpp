@@ -176,12 +176,12 @@ struct BackwardSplit {
 
     // Key blocks (of nkb) that have a chunk `p` < parts: G (nkb - kb) query blocks see key block kb
     // under a causal mask. (p * chunk < G * nkb)
-    __host__ __device__ int blocks(int p, int nkb, int group, bool causal) const {
+    int blocks(int p, int nkb, int group, bool causal) const {
         return causal ? nkb - (int)((uint32_t)p * (uint32_t)chunk / (uint32_t)group) : nkb;
     }
     // Key blocks with several chunks; they are the first ones.
     __host__ __device__ int split_blocks(int nkb, int group, bool causal) const {
-        return parts > 1 ? blocks(1, nkb, group, causal) : 0;
+        return parts > 1 ? (causal ? nkb - whole : nkb) : 0;
     }
     // Workgroups of one (batch, kv head): last chunks first, so that whole chunks lead and the
     // short ones (causal: the late key blocks, which have only a chunk 0) come last. No workgroup
