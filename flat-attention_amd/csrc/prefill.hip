@@ -445,37 +445,51 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         }
     };
 
+    // (K rotated between the HBM load and the LDS store: the (cos, sin) loads of up to four passes
+    // run together. Behind a branch each, for rows past kv_len, every pass waited for its own: with
+    // eight passes, D 128 in four key groups, 11.2 us at 66 keys, ROTNOW now. Rows past kv_len and
+    // dims past head_dim are zeros, rotated by some other row's angles.)
     auto store_k = [&](int tile) {
+        constexpr int PB = ROPEK ? (KPASS < 4 ? KPASS : 4) : KPASS;
+        const int cs0 = FULLD ? k_dc * 4 : min(k_dc * 8, D - 8) >> 1;
 #pragma unroll
-        for (int p = 0; p < KPASS; ++p) {
-            const int kl = p * KRPP + k_r;
-            u32x4_t val = kreg[p];
-            if (ROPEK && tile * BN + kl < kv_len_ && (FULLD || k_dc * 8 < D)) {
-                // K rotated between the HBM load and the LDS store (cos/sin from the table)
-                const float2* csp = a.rope_table +
-                                    (int64_t)(a.kv_rope_offset + tile * BN + kl) * half + k_dc * 4;
-                const f32x4_t c0 = *(const f32x4_t*)csp;
-                const f32x4_t c1 = *(const f32x4_t*)(csp + 2);
-                float x[8], cs[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
+        for (int p0 = 0; p0 < KPASS; p0 += PB) {
+            f32x4_t c0v[PB], c1v[PB];
+            if constexpr (ROPEK) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    x[2 * j] = H::lo(val[j]);
-                    x[2 * j + 1] = H::hi(val[j]);
+                for (int p = 0; p < PB; ++p) {
+                    const int row = min(tile * BN + (p0 + p) * KRPP + k_r, kv_len_ - 1);
+                    const float2* csp = a.rope_table + (int64_t)(a.kv_rope_offset + row) * half + cs0;
+                    c0v[p] = *(const f32x4_t*)csp;
+                    c1v[p] = *(const f32x4_t*)(csp + 2);
                 }
-                rope4(x, cs);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) val[j] = H::pack(x[2 * j], x[2 * j + 1]);
-                if constexpr (SPLIT) {
-                    u32x4_t lo;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        lo[j] = H::pack(x[2 * j] - H::lo(val[j]), x[2 * j + 1] - H::hi(val[j]));
-                    *(u32x4_t*)(smem + st_w + KLO + kl * KROWB + k_dc * 16) = lo;
-                }
-            } else if constexpr (SPLIT) {
-                *(u32x4_t*)(smem + st_w + KLO + kl * KROWB + k_dc * 16) = u32x4_t{0u, 0u, 0u, 0u};
             }
-            *(u32x4_t*)(smem + st_w + kl * KROWB + k_dc * 16) = val;
+#pragma unroll
+            for (int p = 0; p < PB; ++p) {
+                const int kl = (p0 + p) * KRPP + k_r;
+                u32x4_t val = kreg[p0 + p];
+                if constexpr (ROPEK) {
+                    const f32x4_t c0 = c0v[p], c1 = c1v[p];
+                    float x[8], cs[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        x[2 * j] = H::lo(val[j]);
+                        x[2 * j + 1] = H::hi(val[j]);
+                    }
+                    rope4(x, cs);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) val[j] = H::pack(x[2 * j], x[2 * j + 1]);
+                    if constexpr (SPLIT) {
+                        u32x4_t lo;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            lo[j] = H::pack(x[2 * j] - H::lo(val[j]), x[2 * j + 1] - H::hi(val[j]));
+                        *(u32x4_t*)(smem + st_w + KLO + kl * KROWB + k_dc * 16) = lo;
+                    }
+                }
+                *(u32x4_t*)(smem + st_w + kl * KROWB + k_dc * 16) = val;
+            }
+            if constexpr (PB < KPASS) __builtin_amdgcn_sched_barrier(0);
         }
     };
     auto store_v = [&]() {
