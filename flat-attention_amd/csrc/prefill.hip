@@ -447,7 +447,7 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
 
     // (K rotated between the HBM load and the LDS store: the (cos, sin) loads of up to four passes
     // run together. Behind a branch each, for rows past kv_len, every pass waited for its own: with
-    // eight passes, D 128 in four key groups, 11.2 us at 66 keys, ROTNOW now. Rows past kv_len and
+    // eight passes (D 96, four key groups) 13.5 us at 66 keys, 10.3 now. Rows past kv_len and
     // dims past head_dim are zeros, rotated by some other row's angles.)
     auto store_k = [&](int tile) {
         constexpr int PB = ROPEK ? (KPASS < 4 ? KPASS : 4) : KPASS;
@@ -1705,22 +1705,6 @@ static void launch32(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s)
     }
 }
 
-// Which launches take key groups (times in us per call, bf16, the whole call; other loop / two
-// groups / four groups; one workgroup of them fills a CU's LDS at D 128):
-//   four, while 64-row blocks do not outnumber the CUs:
-//     causal RoPE Hq8 Hkv2 S1024 D64 24.3 / 17.5 / 14.6, D128 28.2 (assembly) / 23.3 / 20.8;
-//     Hq32 Hkv8 S512 D128, 256 blocks, 19.6 / 17.4 / 16.0; S1024, 512 blocks, 28.8 / 24.5 / 29.9;
-//     H16 S2048 D128, 512 blocks, 48.3 / 32.6 / 34.2;
-//   two, while 128-row blocks do not outnumber the CUs (the assembly loop: H32/8 S1024, 256
-//     blocks, 28.8 / 24.5; twice that 31.8 / 35.7), or two rounds of them where the other loop is
-//     the ping-pong one (B2 H16 S2048 D128, 512 blocks, 52.5 / 44.5; B4 H16 S2048, 1024 blocks,
-//     74.9 / 88.9; D64 B4 H16 S1024, 512 blocks, 22.4 / 19.8), or four at D 32 (B4 H16 S2048, 39.7
-//     / 33.9). A padded batch has blocks without work: one round (six sequences up to 300 x 500,
-//     480 blocks, 29.9 / 31.9); paged: one round too (4 chunks of 500
-//   queries over 2000 cached tokens, Hq32 Hkv8 D64, 512 blocks, 59.1 / 71.8).
-//   Under six key tiles the assembly kernel stays: its fixed cost is the smaller one (S128 12.8
-//   against 11.9, S300 level). Paged pools that it reads stay with it (one 16-query chunk over
-//   2048 cached tokens 54.6 / 67.5 / 60.7): the key groups wait for each tile's page ids.
 static void launch32g(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s) {
     const bool full = ka.a.head_dim == dpad;
     switch (dpad) {
@@ -1739,6 +1723,32 @@ static void launch32g(const PrefillKArgs& ka, int dpad, dim3 grid, hipStream_t s
     }
 }
 
+// Which 16-bit launches take key groups (times in us per call, bf16, the whole call; other loop / two
+// groups / four groups; one workgroup of them fills a CU's LDS at D 128):
+//   four, while 64-row blocks do not outnumber the CUs:
+//     causal RoPE Hq8 Hkv2 S1024 D64 24.3 / 17.5 / 14.6, D128 28.2 (assembly) / 23.3 / 20.8;
+//     Hq32 Hkv8 S512 D128, 256 blocks, 19.6 / 17.4 / 16.0; S1024, 512 blocks, 28.8 / 24.5 / 29.9;
+//     H16 S2048 D128, 512 blocks, 48.3 / 32.6 / 34.2;
+//   but two for two tiles of one row block (16 queries over 100 cached tokens, Hq8 Hkv2 D64 7.7 / 7.4
+//     / 8.2, D96 10.5 / 10.2 / 11.6) and for contiguous rows of over 64 dims (no RoPE, Hq8 Hkv2 D128,
+//     66 keys 8.8 / 7.7 / 8.5, causal 128 dims three tiles too, 130 keys 10.1 / 8.4 / 8.7, no mask
+//     11.8 / 9.5 / 9.1);
+//   two, while 128-row blocks do not outnumber the CUs (the assembly loop: H32/8 S1024, 256
+//     blocks, 28.8 / 24.5; twice that 31.8 / 35.7);
+//   where the other loop is the ping-pong one, two rounds of them under a causal mask from eleven tiles
+//     on, as its blocks of unequal length leave the chip idle (B4 H16 S1000 D64, 512 blocks, 22.6 /
+//     20.2, B2 H16 S2048 D128 53.0 / 46.1, B2 Hq32 Hkv8 S700 D128, 352, 22.0 / 19.7; but S400 with
+//     H32 B4 D64, 512, 13.1 / 15.3, and without a mask S1000 24.2 / 28.6, S300 D128, 384, 15.8 / 20.7);
+//     at D 32 three rounds (B6 H32 S512, 768 blocks, 17.3 / 15.8, causal 13.6 / 13.0), causal from 16
+//     tiles on four (B4 H16 S2048, 1024, 40.4 / 34.1; no mask 56.3 / 58.3; B8 H32 S512 13.9 / 15.9).
+//     A padded batch has blocks without work: one round (six sequences up to 300 x 500, 480 blocks,
+//     29.9 / 31.9); paged: one round too (4 chunks of 500 queries over 2000 cached tokens, Hq32 Hkv8
+//     D64, 512 blocks, 59.1 / 71.8).
+//   Under six key tiles the assembly kernel stays: its fixed cost is the smaller one (S128 12.8
+//   against 11.9, S300 level). Paged pools that it reads stay with it: over few keys it is the faster
+//   one (64 queries after 512 cached tokens, Hq32 Hkv8, 18.7 / 21.4 / 20.6; 8 x 21 after 488 16.6 / 19.0
+//   / 17.6), over many four groups would be (64 after 2048 45.2 / 52.5 / 43.3, 256 after 2048 48.6 /
+//   55.8 / 44.1, 128 after 8000 149.7 / 175.1 / 132.4), a line that is not drawn here.
 int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a) {
     if (dt == Dtype::F32 || a.split_qk || a.k_lo || (paged && a.page_size % 16)) return 0;
     const bool a64 = prefill_a64_eligible(dt, paged, a);
@@ -1748,11 +1758,16 @@ int prefill_key_groups(Dtype dt, bool paged, const PrefillArgs& a) {
     const int64_t tiles = (keys + 63) / 64;
     if (tiles < (a64 ? 6 : 2)) return 0;
     const int64_t cus = device_cus(), rows = (int64_t)a.q_len * a.group;
-    const int64_t units = (int64_t)a.batch * a.kv_heads;
-    const int64_t rounds = a64 || a.var_meta || paged ? 1 : a.head_dim <= 32 ? 4 : 2;
-    if (units * ((rows + 63) / 64) <= cus) return 4;
-    if (units * ((rows + 127) / 128) <= rounds * cus) return 2;
-    return 0;
+    const int64_t units = (int64_t)a.batch * a.kv_heads, blocks = units * ((rows + 127) / 128);
+    if (units * ((rows + 63) / 64) <= cus) {
+        if (tiles == 2 && rows <= 64) return 2;
+        if (!paged && a.head_dim > 64 && tiles <= (a.head_dim == 128 && a.causal ? 3 : 2)) return 2;
+        return 4;
+    }
+    if (blocks <= cus) return 2;
+    if (a64 || a.var_meta || paged) return 0;
+    if (a.head_dim <= 32) return blocks <= (a.causal && tiles >= 16 ? 4 : 3) * cus ? 2 : 0;
+    return a.causal && tiles >= 11 && blocks <= 2 * cus ? 2 : 0;
 }
 
 bool prefill_uses_a64(Dtype dt, bool paged, const PrefillArgs& a) {

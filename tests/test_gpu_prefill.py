@@ -68,9 +68,9 @@ def test_mha_f32_shapes(hip, D, S, causal):
 @pytest.mark.parametrize("S", [1, 7, 64, 65, 130, 300])
 @pytest.mark.parametrize("causal", [False, True])
 def test_mha_16bit_shapes(hip, D, S, causal):
-    """The 16-bit kernel (256-row ping-pong workgroups) at edge shapes: a single key, partial
-    key tiles, head dims below the padded width, and query blocks whose rows run out part-way
-    through either wave group."""
+    """The 16-bit kernel at edge shapes of few rows (one key tile: 256-row ping-pong workgroups, more:
+    key groups): a single key, partial key tiles, head dims below the padded width, and query blocks
+    whose rows run out part-way."""
     B, H = 2, 3
     q, k, v = (bf16_round(normal(B * H * S * D, 300 + s + D + S)) for s in range(3))
     shape = fa.GroupedAttentionShape(B, H, H, S, D)
@@ -240,6 +240,64 @@ def test_key_group_prefill_matches_oracle(hip, dtype, rnd, B, hq, hkv, S, D, rop
     assert_close("O", o[:n * D], eo[:n * D], H16_ATOL, 0.0)
     assert_close("LSE", l[:n], el[:n], H16_ATOL, 0.0)
     assert np.isfinite(o).all() and np.isfinite(l).all()
+
+
+@pytest.mark.parametrize("B,H,S,D,rows", [
+    (8, 64, 130, 64, (256, 256)),   # the ping-pong loop: blocks that end in either wave group, several
+    (8, 64, 300, 80, (256, 256)),   # key tiles with remainders, head dims below the padded width
+    (9, 64, 65, 96, (256, 256)),
+    (9, 64, 300, 32, (256, 256)),
+    (8, 64, 300, 128, (256, 256)),
+    (4, 32, 300, 64, (256, 256)),   # 384 blocks of 128 rows, five tiles
+    (2, 32, 705, 64, (256, 128)),   # twelve tiles: key groups where blocks are of unequal length
+    (8, 32, 200, 32, (128, 128)),   # 32 dims: two rounds of them
+    (8, 32, 500, 32, (256, 256)),   # not four, of eight tiles
+    (1, 8, 66, 128, (128, 128)),    # two tiles: two groups
+    (1, 8, 130, 128, (64, 128)),    # three
+])
+@pytest.mark.parametrize("dtype,rnd", [(fa.DTYPE_BF16, bf16_round), (fa.DTYPE_F16, f16_round)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_16bit_prefill_kernel_by_filled_chip(hip, dtype, rnd, B, H, S, D, rows, causal):
+    """Which loop of the 16-bit kernel a launch takes as its row blocks fill the chip, and its result
+    (the first and the last heads against the oracle)."""
+    q, k, v = (rnd(normal(B * H * S * D, 790 + S + i)) for i in range(3))
+    shape = fa.GroupedAttentionShape(B, H, H, S, D)
+    o, l = _run_grouped(hip, q, k, v, shape, fa.FlatAttentionConfig(causal), None, dtype)
+    assert hip.last_telemetry().query_rows == rows[causal]
+    for u in (0, B * H - 2):
+        eo, el = _oracle_grouped(q, k, v, shape, causal, None, units=(u, u + 2))
+        at = slice(u * S, (u + 2) * S)
+        assert_close("O", o.reshape(-1, D)[at], eo.reshape(-1, D)[at], H16_ATOL, 0.0)
+        assert_close("LSE", l[at], el[at], H16_ATOL, 0.0)
+
+
+@pytest.mark.parametrize("B,hq,hkv,S,D,rows", [
+    (1, 8, 2, 66, 64, 64), (1, 8, 2, 66, 96, 128), (1, 8, 2, 500, 128, 64),  # four and two key groups
+    (1, 32, 8, 901, 80, 128), (9, 64, 64, 130, 64, 128), (8, 64, 64, 300, 40, 128)])  # and none
+def test_rotation_on_load_in_every_loop_is_bit_identical(hip, B, hq, hkv, S, D, rows):
+    """K rotated while a tile is staged against K rotated by the pre-pass, in each loop that stages
+    tiles through registers: rows past kv_len, dims past the head dim."""
+    shape = fa.GroupedAttentionShape(B, hq, hkv, S, D)
+    rot, cfg = fa.RotaryEmbeddingConfig(1e4, 7), fa.FlatAttentionConfig(True)
+    q, k, v = (bf16_round(normal(n, 830 + i)) for i, n in enumerate(
+        (B * hq * S * D, B * hkv * S * D, B * hkv * S * D)))
+    got = []
+    hip.set_prefill_kernel(0)
+    try:
+        for policy in (0, 1):
+            hip.set_prefill_policy(policy)
+            got.append(_run_grouped(hip, q, k, v, shape, cfg, rot, fa.DTYPE_BF16))
+            if policy == 0:
+                assert hip.last_telemetry().query_rows == rows
+    finally:
+        hip.set_prefill_policy(-1)
+        hip.set_prefill_kernel(-1)
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    u = B * hq - 2
+    eo, _ = _oracle_grouped(q, k, v, shape, True, rot, units=(u, u + 2))
+    at = slice(u * S, (u + 2) * S)
+    assert_close("O", got[0][0].reshape(-1, D)[at], eo.reshape(-1, D)[at], H16_ATOL, 0.0)
 
 
 @pytest.mark.parametrize("kind", ["rising", "falling", "far_apart"])
