@@ -1326,6 +1326,7 @@ __global__ __launch_bounds__(256, DMA ? 2 : 1) void prefill_mfma_f32(PrefillKArg
             }
         }
 
+        if constexpr (DMA) wait_mfma(sacc[KB - 1]);
         const int tile_end = (tile + 1) * BN;
         if (tile_end > kv_len_ || (a.causal && tile_end - 1 > cpos_min)) {
             const int lim = a.causal ? min(kv_len_ - 1, cpos) : kv_len_ - 1;
