@@ -249,7 +249,7 @@ __device__ __forceinline__ void decode_item(const DecodeKArgs& ka, int s, int kv
             }
             load_k(kbuf[s], key0 + 16 * NS);
             if (live) {
-                if constexpr (F32) wait_mfma(sc);
+                if constexpr (F32 && NS == 2) wait_mfma(sc);
                 if (key0 + 16 > k1) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
