@@ -83,8 +83,9 @@ __device__ __forceinline__ void store8(void* dst, const float* x) {
 }
 
 // Waves per SIMD of decode_splitk. f32 rows of 128 dims: two waves with two steps of K/V in flight
-// each (8 sequences of 100..2000 tokens, Hq16 Hkv4: 29.1 us; 36.7 with one wave and three steps).
-// At 64 dims one wave (8192 tokens, Hq16 Hkv4: 14.6 against 15.1 us; four such sequences 23.4 / 26.1).
+// each (8 sequences of 100..2000 tokens, Hq16 Hkv4: 15.8 us a launch; 23.1 with one wave and three
+// steps; one sequence of 8192: 18.6 / 26.4). At 64 dims one wave (8192 tokens, Hq16 Hkv4: 14.6
+// against 15.1 us; four such sequences 23.4 / 26.1).
 template <typename T, int DPAD, int GT>
 constexpr int splitk_waves() {
     return std::is_same<T, float>::value && DPAD == 128 && GT <= 4 ? 2 : 1;
@@ -99,7 +100,11 @@ __device__ __forceinline__ void decode_item(const DecodeKArgs& ka, int s, int kv
     constexpr bool F32 = std::is_same<T, float>::value;
     constexpr int EB = DecodeIO<T>::kBytes;
     const DecodeArgs& a = ka.a;
-    const int lane = threadIdx.x;
+    int lane = threadIdx.x;
+    // (opaque: what depends on the lane alone would be kept over all segments of a wave, with 256
+    // registers up to 23 of them in scratch memory, whose loads then wait behind the K/V stream: 8
+    // sequences of 100..2000 tokens, Hq16 Hkv4 18.7 us a launch, so 15.8)
+    if constexpr (splitk_waves<T, DPAD, GT>() == 2) asm volatile("" : "+v"(lane));
     const int n = lane & 15, g4 = lane >> 4;
     const int D = a.head_dim, half = D >> 1;
     const int hl0 = hc * 16;                 // first head of this chunk within the group
