@@ -133,6 +133,9 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     // Loads run ahead of the products that need them, in the order the fences fix: the next block's
     // rows under this block's dV/dK products (D 128: one wave per SIMD has the registers, and
     // nothing else hides their latency), the columns of block m + 1 under the products of m.
+    // (D 128 takes all 512 registers and twelve more, 16-byte pieces of K and V that are read again
+    // from scratch memory once a block, of 16384 clocks; the lane offsets are opaque in the loop, or
+    // ten to fifteen of them would be kept there too.)
     constexpr bool AHEAD = DPAD == 128;
     struct At {
         Tile q, o, ld;
@@ -151,21 +154,25 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
     };
     Frag32 qr[MB], dr[MB];
     auto load_rows = [&](const At& t) {
+        int row = c;
+        if (AHEAD) asm volatile("" : "+v"(row));
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
-            qr[m] = row_frag<FULL>(t.q, 32 * m, D, g, c);
-            dr[m] = row_frag<FULL>(t.o, 32 * m, D, g, c);
+            qr[m] = row_frag<FULL>(t.q, 32 * m, D, g, row);
+            dr[m] = row_frag<FULL>(t.o, 32 * m, D, g, row);
         }
     };
     if (AHEAD && first + wave < last) load_rows(tiles(first + wave));
     for (int it = first + wave; it < last; it += 4) {
         const At t = tiles(it);
+        int cc = c, gg = g;
+        if (AHEAD) asm volatile("" : "+v"(cc), "+v"(gg));
         if (!AHEAD) load_rows(t);
         u32x4_t ld[8];  // (LSE log2 e, delta) of rows kidx(g, 2 i), kidx(g, 2 i + 1)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             ld[i] = __builtin_amdgcn_raw_buffer_load_b128(
-                t.ld, (8 * (i >> 1) + 4 * g + 2 * (i & 1)) * 8, 0, 0);
+                t.ld, (8 * (i >> 1) + 4 * gg + 2 * (i & 1)) * 8, 0, 0);
         f32x16_t s = (f32x16_t)0.0f, dp = (f32x16_t)0.0f;
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
@@ -173,7 +180,7 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
             dp = mma32(dr[m], vf[m], dp);
         }
         __builtin_amdgcn_sched_barrier(0);
-        Frag32 oc = col_frag(t.o, c, D, g), qc = col_frag(t.q, c, D, g);
+        Frag32 oc = col_frag(t.o, cc, D, gg), qc = col_frag(t.q, cc, D, gg);
         __builtin_amdgcn_sched_barrier(0);
         // Rows past the sequence: dO = 0 and delta = 0, so they add nothing.
         Frag32 pf, df;
@@ -181,7 +188,7 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
         for (int i = 0; i < 16; ++i) {
             const u32x4_t l = ld[i >> 1];
             float p = fast_exp2(fmaf(s[i], c2, -__uint_as_float(l[2 * (i & 1)])));
-            if (a.causal && t.qb == kb && c > kidx32(g, i)) p = 0.0f;
+            if (a.causal && t.qb == kb && cc > kidx32(gg, i)) p = 0.0f;
             pf.v[i] = p;
             df.v[i] = p * (dp[i] - __uint_as_float(l[2 * (i & 1) + 1]));
         }
@@ -191,8 +198,8 @@ __global__ __launch_bounds__(256, DPAD == 128 ? 1 : 2) void bwd_f32_dkdv(Backwar
             const Frag32 om = oc, qm = qc;
             __builtin_amdgcn_sched_barrier(0);
             if (m + 1 < MB) {
-                oc = col_frag(t.o, 32 * (m + 1) + c, D, g);
-                qc = col_frag(t.q, 32 * (m + 1) + c, D, g);
+                oc = col_frag(t.o, 32 * (m + 1) + cc, D, gg);
+                qc = col_frag(t.q, 32 * (m + 1) + cc, D, gg);
             }
             __builtin_amdgcn_sched_barrier(0);
             dv[m] = mma32(pf, om, dv[m]);

@@ -15,7 +15,7 @@ import pytest
 LIB = pathlib.Path(__file__).resolve().parents[1] / "flat-attention_amd/flat_attention_amd/libflat_hip.so"
 LLVM = pathlib.Path("/opt/rocm/llvm/bin")
 ALLOWED = {"decode_splitkIfLi32ELi16E": 8, "decode_splitkIfLi64ELi16E": 8, "decode_splitkIfLi128ELi16E": 8,
-           "decode_splitkIfLi128ELi4E": 2, "bwd_f32_dkdvILi128E": 27}
+           "decode_splitkIfLi128ELi4E": 2, "bwd_f32_dkdvILi128E": 12}
 
 
 @pytest.mark.skipif(not LIB.exists() or not (LLVM / "llvm-readelf").exists(),
