@@ -161,15 +161,11 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
-// Wait for the result of an f32 MFMA of 8 (16x16) or 16 (32x32) passes: the hardware holds no vector
-// instruction back for it. Written out where a branch comes between the product and its first
-// reader: the compiler counts the instructions between them along one way only, and where the other
-// is shorter the reader gets results that lack the last products. The reader needs the wait anyway
-// (4 clocks each state: 40 and 72).
+// Wait for the result of an f32 16x16 MFMA: the hardware holds no vector instruction back for it.
+// Written out where a branch comes between the product and its first reader: the compiler counts the
+// instructions between them along one way only, and where the other is shorter the reader gets
+// results that lack the last product. The reader needs the wait anyway (10 states of 4 clocks).
 __device__ __forceinline__ void wait_mfma(f32x4_t& v) { asm volatile("s_nop 9" : "+v"(v)); }
-__device__ __forceinline__ void wait_mfma(f32x16_t& v) {
-    asm volatile("s_nop 15\n\ts_nop 1" : "+v"(v));
-}
 // Buffer resource words: base, stride 0, num_records bytes, the same flags as
 // __builtin_amdgcn_make_buffer_rsrc is given elsewhere (0x00020000).
 __device__ __forceinline__ i32x4_t make_rsrc_words(const void* base, int nrec) {
