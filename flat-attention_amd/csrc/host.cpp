@@ -584,7 +584,9 @@ int fa_ctx_create(int device, fa_ctx** out) {
             slot.copied = nullptr;
             break;  // (the last slot's event is there only if all are)
         }
-    if (hipHostMalloc((void**)&ctx->na_host, kNoAllocMetaBytes, hipHostMallocDefault) !=
+    // (coherent by name: a kernel reads the parts while the host writes others, and a part is used
+    // again after an event alone, whatever HIP_HOST_COHERENT makes of the default)
+    if (hipHostMalloc((void**)&ctx->na_host, kNoAllocMetaBytes, hipHostMallocCoherent) !=
         hipSuccess)
         ctx->na_host = nullptr;
     *out = ctx;
