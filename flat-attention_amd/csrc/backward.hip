@@ -517,11 +517,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
             using H = typename B::H;
             constexpr int NS = 4 * MB;  // MFMAs of S+dP, and of dV+dK, per sub-block
             constexpr int R = 2, RV = 2;
-            const uint8_t* tile0 = smem + st;
+            const uint8_t* stage = smem + st;
             // A operand of MFMA i of S / dP: chain i & 1 (Q for S, dO for dP), dims
             // 32 (i >> 2) + 16 ((i >> 1) & 1) + 8 g ..
             auto aread = [&](int sb, int i) {
-                return ops.rread(tile0 + (i & 1 ? T_DO : 0) + sb * 32 * RB, i >> 2, (i >> 1) & 1);
+                return ops.rread(stage + (i & 1 ? T_DO : 0) + sb * 32 * RB, i >> 2, (i >> 1) & 1);
             };
             auto sdp = [&](int sb, f32x16_t& sa, f32x16_t& da) {
                 u32x4_t ring[R];
@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv(BackwardArgs a, BackwardSplit
             // B operand of MFMA i of dV / dK: chain i & 1 (dO^T for dV, Q^T for dK), column
             // block i >> 2, rows 16 ((i >> 1) & 1) + 8 g .. (two transposing reads)
             auto bread = [&](int sb, int i) {
-                return ops.tread(tile0 + (i & 1 ? 0 : T_DO) + sb * 32 * RB, i >> 2, (i >> 1) & 1);
+                return ops.tread(stage + (i & 1 ? 0 : T_DO) + sb * 32 * RB, i >> 2, (i >> 1) & 1);
             };
             auto dvdk = [&](int sb, const F& pf, const F& df) {
                 u32x4_t ring[RV];

@@ -894,7 +894,8 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
         // that ended step i-1), computes its tile, then waits for its own transfers and meets the
         // other waves: one barrier per step, a group without a tile in the last step included.
         const int gbase = kg * NST * STAGE;
-        const int n_steps = KW > 1 ? (n_tiles + KW - 1) / KW : n_tiles;
+        static_assert(KW > 1, "one group takes the ping-pong loop");
+        const int n_steps = (n_tiles + KW - 1) / KW;
         if (kg < n_tiles) dma_tile(kg, gbase);
         wait_dma();
         __syncthreads();
@@ -903,7 +904,7 @@ __global__ __launch_bounds__(64 * NW, SPLIT ? 1 : 2) void prefill_mfma16(Prefill
             st_r = gbase + (i & 1) * STAGE;
             st_k = st_v = st_r;
             if (tile + KW < n_tiles) dma_tile(tile + KW, gbase + STAGE - (i & 1) * STAGE);
-            if (KW == 1 || tile < n_tiles) {
+            if (tile < n_tiles) {
                 f32x16_t sacc[2];
                 u32x4_t pop[4];
                 compute_s(sacc, std::true_type{}, no_hook);
