@@ -504,8 +504,8 @@ def _paged_prefill(hip, bt, ps, total, n_seqs, hq, hkv, D, cached, ql, theta, ra
 @pytest.mark.parametrize("D,causal", [(128, True), (64, True), (128, False)])
 def test_paged_prefill_modes_match_oracle_and_gather_bit_exactly(hip, dtype, ps, D, causal):
     """Chunked prefill over the paged cache in every addressing mode: 16-bit with page size a
-    multiple of 16 (one page per 16-key group, 8-wave ping-pong kernel), 16-bit with any page
-    size (4-wave kernel), and f32. A query
+    multiple of 16 (one page per 16-key group: 8 waves in key groups, at D 128 and 16-row pages the
+    assembly kernel), 16-bit with any page size (4-wave kernel), and f32. A query
     chunk of 50 rows after 37 cached tokens, so key tiles and pages end mid-way. The same
     data under the identity block table and a shuffled one must give bitwise identical O/LSE."""
     rnd = {fa.DTYPE_BF16: bf16_round, fa.DTYPE_F16: f16_round, fa.DTYPE_F32: lambda x: x}[dtype]
@@ -526,7 +526,7 @@ def test_paged_prefill_modes_match_oracle_and_gather_bit_exactly(hip, dtype, ps,
     t = hip.last_telemetry()
     if dtype != fa.DTYPE_F32 and ps == 16 and D == 128:  # the paged assembly kernel
         assert "prefill_a64" in t.kernel_name and t.workgroup_size == 256, t.kernel_name
-    elif dtype != fa.DTYPE_F32:  # page % 16 == 0: 8-wave ping-pong kernel; else the 4-wave one
+    elif dtype != fa.DTYPE_F32:  # page % 16 == 0: 8 waves; else 4
         assert t.workgroup_size == (512 if ps % 16 == 0 else 256)
     pools = []
     o2, l2 = _paged_prefill(hip, shuf, ps, total, n_seqs, hq, hkv, D, cached, ql, theta, raw_k,
@@ -551,11 +551,15 @@ def test_paged_prefill_modes_match_oracle_and_gather_bit_exactly(hip, dtype, ps,
 
 
 @pytest.mark.parametrize("ps,D,cached,ql,groups", [(16, 64, 3, 70, 4), (32, 64, 300, 50, 4),
-                                                   (32, 128, 90, 33, 4), (48, 64, 200, 700, 2)])
+                                                   (32, 128, 90, 33, 4), (48, 64, 200, 700, 2),
+                                                   # past the 64 table entries held at a time
+                                                   (16, 64, 1993, 77, 4), (16, 64, 1201, 700, 2),
+                                                   (16, 64, 100, 1100, 1)])
 def test_paged_prefill_key_groups_match_oracle_and_gather_bit_exactly(hip, ps, D, cached, ql,
                                                                       groups):
-    """The key-group prefill over a paged cache: pages of one and several 16-key groups, key
-    tiles and pages that end part-way; identity and shuffled tables bitwise identical."""
+    """The key-group prefill over a paged cache (and, as one group, the ping-pong loop): pages of one
+    and several 16-key groups, key tiles and pages that end part-way, more pages than a wave holds
+    table entries; identity and shuffled tables bitwise identical."""
     dtype, n_seqs, hq, hkv, theta = fa.DTYPE_BF16, 2, 16, 8, 1e4
     kv_len = cached + ql
     pages_per = -(-kv_len // ps)
