@@ -195,7 +195,10 @@ def test_f32_backward_of_filled_chip_matches_oracle(hip, dims, staged, causal):
 @pytest.mark.parametrize("dtype", [fa.DTYPE_BF16, fa.DTYPE_F16])
 @pytest.mark.parametrize("dims,causal", [((1, 8, 2, 256, 128), True),
                                          ((2, 4, 4, 130, 64), False),
-                                         ((1, 4, 1, 77, 32), True)])
+                                         ((1, 4, 1, 77, 32), True),
+                                         # whole key blocks on a filled chip, the last of one row
+                                         ((6, 32, 32, 257, 64), True),
+                                         ((6, 32, 32, 257, 80), False)])
 def test_16bit_storage(hip, dtype, dims, causal):
     rnd = bf16_round if dtype == fa.DTYPE_BF16 else f16_round
     shape = fa.GroupedAttentionShape(*dims)
