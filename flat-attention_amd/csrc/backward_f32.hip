@@ -370,9 +370,11 @@ void launch_d(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
 //     0.62 (B2 S500 causal) 266 / 316, 1 (B4 S200) 139 / 261;
 //   D <= 64, where a CU holds two of them: with that chip filled too (D 64, H32 B4 S500 292 / 318, B8
 //     S384 causal 254 / 276, B8 S500 576 / 650; not B4 S384 causal 129 / 118, B6 S384 251 / 221), or up
-//     to 256 keys without a mask, a few tiles to a workgroup, once (B4 S200 85.5 / 94.9), and at D 32
-//     and 64 not with long sequences (B4 S1000 1059 / 1085, B4 H16 S2048 causal 1132 / 1095; D 40 B4
-//     S1000 1034 / 1138).
+//     to 256 keys without a mask, a few tiles to a workgroup, once (B4 S200 85.5 / 94.9). Between 33 and
+//     63 dims, where these load half the padding, a little earlier (D 40: B4 S500 causal 202 / 215, but
+//     D 24 113 / 102), to 512 keys (B2 S500 152 / 161) and with one key block (B8 S100 causal 52 / 60;
+//     not at 0.75, B12 S60 53 / 46, although B6 S100 51 / 56). At D 32 and 64 not with long sequences
+//     (B4 S1000 1059 / 1085, B4 H16 S2048 causal 1132 / 1095; D 40 B4 S1000 1034 / 1138).
 static bool staged_f32(const BackwardArgs& a) {
     const int64_t nkb = (a.seq + 127) / 128, n = (int64_t)a.batch * a.kv_heads * nkb;
     const int64_t cus = device_cus();
@@ -385,9 +387,10 @@ static bool staged_f32(const BackwardArgs& a) {
         return tiles / (double)(places * backward_time(one, (int)nkb, a, places, 0, 0));
     };
     if (a.head_dim > 64) return filled(cus) >= (a.head_dim == 128 ? 0.7 : 0.55);
-    const bool full = a.head_dim == 64 || a.head_dim == 32;
+    const bool full = a.head_dim == 64 || a.head_dim == 32, padded = a.head_dim > 32 && !full;
     return (a.seq < 1500 || !full) && filled(cus) >= 0.9 &&
-           (filled(2 * cus) >= (full ? 0.7 : 0.6) || (!a.causal && a.seq <= 256));
+           (filled(2 * cus) >= (padded ? 0.6 : 0.7) || (padded && a.seq <= 128) ||
+            (!a.causal && a.seq <= (padded ? 512 : 256)));
 }
 
 // Blocks a wave takes: the total over the waves that the chip holds at once (one per SIMD at
