@@ -1792,12 +1792,16 @@ static bool f32_rows_ok(const PrefillArgs& a) {
 // count for more once it is full (times in us per call, that kernel / this one):
 //   head_dim <= 32: fewer blocks than two per CU (H32 B2 S300 20.2 / 16.6, S500 28.9 / 27.0, B4 S200,
 //     256 blocks, 16.4 / 16.9; B4 S500, 512 blocks, 47.9 / 48.9);
-//   where the 32-row workgroups, two to a CU, are one round (no mask, D64 H32 B2 S200, 448 of them,
-//     27.4 / 19.0, S300, 640, 35.5 / 38.8; B4 S200, 896, 28.2 / 34.6; D80 42.6 / 55.5), or at D128
-//     one and a half (B2 S300 61.0 / 55.9; B4 S200 49.4 / 57.0), except that with as many blocks of
-//     few rows the two are level;
-//   more of them under a causal mask: by the share of the keys that the rows see, as blocks of unequal length leave that kernel
-//     idle and this one not: up to 0.8 of one block per CU, 0.6 of two (D128 H32 B2 S500, 256 blocks of
+//   where the 32-row workgroups are at most two per CU (no mask, D64 H32 B2 S200, 448 of them, 27.4 /
+//     19.0, S300, 640, 35.5 / 38.8; B4 S200, 896, 28.2 / 34.6; D80 42.6 / 55.5), at D128 three (B2 S300
+//     61.0 / 55.9; B4 S200 49.4 / 57.0), and at any head dim over more than 384 keys, as these take the
+//     keys in turns of 256 and the blocks of the other kernel leave CUs without any (D64 H16 S1100, 560
+//     of them, 99 / 77, H8 S2500, 632, 209 / 142, H32 S700, 704, 65.8 / 61.6; D96 H16 S1500 212 / 194);
+//     except that with as many blocks of few rows the two are level;
+//   at D64 without a mask, four per CU over 1536 keys or more (H16 S2048, 1024 of them, 175 / 159, H8
+//     S4096 337 / 283; S1024, 1024, 93.5 / 96.2; D48 S2048 172 / 180);
+//   more of them under a causal mask: by the share of the keys that the rows see, as blocks of unequal
+//     length leave that kernel idle and this one not: up to 0.8 of one block per CU, 0.6 of two (D128 H32 B2 S500, 256 blocks of
 //     which 0.63 counts, 89.9 / 66.7; B4 S200, 256 of 0.82, 44.6 / 44.6, D80 39.1 / 41.9; S300, 384 of
 //     0.71, 77.9 / 67.4; S500, 512 of 0.63, 123.4 / 132.7; B2 H16 S2048, 512 of 0.53, 398 / 341).
 bool prefill_uses_f32_groups(Dtype dt, bool paged, const PrefillArgs& a) {
@@ -1807,9 +1811,9 @@ bool prefill_uses_f32_groups(Dtype dt, bool paged, const PrefillArgs& a) {
     const int64_t cus = device_cus(), units = (int64_t)a.batch * a.kv_heads;
     const int64_t rows = (int64_t)a.q_len * a.group, blocks = units * ((rows + 127) / 128);
     if (a.head_dim <= 32) return blocks < 2 * cus;
-    if (units * ((rows + 31) / 32) <= (a.head_dim == 128 ? 3 : 2) * cus)
+    if (units * ((rows + 31) / 32) <= (a.head_dim == 128 || a.kv_len > 384 ? 3 : 2) * cus)
         return blocks < 2 * cus + (a.head_dim > 64 ? 1 : 0);
-    if (!a.causal) return false;
+    if (!a.causal) return a.head_dim == 64 && blocks <= cus && a.kv_len >= 1536;
     // positions of the first row, and of the one past the last (a padded batch: of its longest)
     const int64_t first = a.var_meta ? std::max(0, a.kv_len - a.q_len) : a.causal_offset;
     const int64_t last = first + a.q_len;

@@ -185,6 +185,10 @@ def test_f32_key_group_prefill_matches_oracle(hip, B, hq, hkv, S, D, rope, rows,
     (2, 32, 300, 64, False, 128),   # 640: more than one, and 192 blocks of 128 rows
     (2, 32, 300, 64, True, 32),     # causal: of which 0.71 counts
     (2, 32, 300, 128, False, 32),   # one and a half rounds at D 128
+    (1, 16, 1100, 64, False, 32),   # 560 over more than 384 keys: the blocks are 144
+    (3, 16, 385, 80, False, 32),    # 624
+    (1, 16, 2048, 64, False, 32),   # 1024 over many keys
+    (1, 32, 900, 64, False, 128),   # 928 over fewer
     (4, 32, 200, 80, False, 128),
     (4, 32, 200, 80, True, 128),    # 256 blocks of which 0.82 counts
     (4, 32, 300, 96, True, 32),     # 384 of which 0.71 counts
