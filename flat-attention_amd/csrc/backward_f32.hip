@@ -365,7 +365,9 @@ void launch_d(const BackwardArgs& a, const BackwardSplit& sp, hipStream_t s) {
 // time that they keep busy, one to a CU; over 400 shapes the ratio of the two follows it (us for the
 // backward, staged / these):
 //   D 128: 0.62 (H32 B2 S500 causal) 276 / 253, 0.75 (B4 S200 causal) 145 / 155, 1 (B4 S384 causal)
-//     267 / 326, (B4 S200) 148 / 214; Hq32 Hkv8 S2048 causal, 0.27, 2529 / 1218;
+//     267 / 326, (B4 S200) 148 / 214; Hq32 Hkv8 S2048 causal, 0.27, 2529 / 1218; over long sequences,
+//     whose chunks come out even, from 0.78 (B2 H8 S1500, 0.75, 707 / 661, H4 S6000, 0.73, 2722 /
+//     2431; H24 S2048 causal, 0.80, 957 / 987);
 //   64 < D < 128, where these load and multiply the padding too: D 96, 0.50 (B2 S384 causal) 208 / 197,
 //     0.62 (B2 S500 causal) 266 / 316, 1 (B4 S200) 139 / 261;
 //   D <= 64, where a CU holds two of them: with that chip filled too (D 64, H32 B4 S500 292 / 318, B8
@@ -386,7 +388,7 @@ static bool staged_f32(const BackwardArgs& a) {
     auto filled = [&](int64_t places) {
         return tiles / (double)(places * backward_time(one, (int)nkb, a, places, 0, 0));
     };
-    if (a.head_dim > 64) return filled(cus) >= (a.head_dim == 128 ? 0.7 : 0.55);
+    if (a.head_dim > 64) return filled(cus) >= (a.head_dim < 128 ? 0.55 : a.seq < 1024 ? 0.7 : 0.78);
     const bool full = a.head_dim == 64 || a.head_dim == 32, padded = a.head_dim > 32 && !full;
     return (a.seq < 1500 || !full) && filled(cus) >= 0.9 &&
            (filled(2 * cus) >= (padded ? 0.6 : 0.7) || (padded && a.seq <= 128) ||

@@ -165,6 +165,7 @@ def test_f32_backward_splits_match_oracle(hip, dims, causal):
     ((8, 32, 32, 300, 33), (True, True)),
     ((4, 32, 32, 200, 40), (True, False)),   # 256: once round
     ((4, 32, 32, 300, 32), (False, False)),  # 384: the second of two rounds half filled
+    ((7, 3, 3, 1025, 128), (False, False)),  # 189 workgroups of a long sequence
     ((8, 32, 32, 100, 40), (True, True)),    # one key block each
     ((2, 32, 32, 500, 48), (True, False)),
     ((4, 32, 32, 500, 24), (True, False)),
