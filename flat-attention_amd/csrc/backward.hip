@@ -1149,11 +1149,10 @@ int64_t backward_time(const BackwardSplit& sp, int nkb, const BackwardArgs& a, i
 // parts = 0: the assembly kernel. Else the number of chunks with the least time (one workgroup to a
 // CU; one costs two tiles of 128 queries of a head beside its own, one with partials four, as 256 D
 // floats are written and read again): one, two, an even share of the tiles for each CU, or a number
-// next to one, two or three full rounds of workgroups. Measured against 1 to 36 chunks at 25 shapes (Hq6 Hkv1 to B2 Hq32 Hkv8, S 512 to 4000, with and
-// without a mask) the choice took at most 1 % longer than the best of them; so did none of the
-// choices with three tiles for partials, and with five one 4 %. (us for the backward, bf16 causal D
-// 128, one chunk / chosen / twice as many: Hq16 Hkv4 S1000 166 / 51 / 61; Hq32 Hkv8 B2 S1000 177 /
-// 102 / 118; Hq16 Hkv4 S4000 623 / 286 / 320.)
+// next to one, two or three full rounds of workgroups. Measured against 1 to 36 chunks at 25 shapes
+// (Hq6 Hkv1 to B2 Hq32 Hkv8, S 512 to 4000, with and without a mask) the choice took at most 1 % longer
+// than the best of them; with three tiles for partials too, with five one shape took 4 %. (us for the backward, bf16 causal D 128, one chunk / chosen / twice as many: Hq16 Hkv4 S1000
+// 166 / 51 / 61; Hq32 Hkv8 B2 S1000 177 / 102 / 118; Hq16 Hkv4 S4000 623 / 286 / 320.)
 // The assembly kernel takes 3 us a tile against 4.3 but one workgroup per 128 keys: the split wins
 // while those are at most half the CUs and chains are long (bf16 causal D 128, us for the backward,
 // assembly / split: Hq8 Hkv2 S512, 8 workgroups, 62.5 / 33.2; Hq32 Hkv8 B2 S512, 64, 67.1 / 52.2;
